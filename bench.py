@@ -122,7 +122,7 @@ def group_times(stages: dict) -> dict:
 # kernel-name prefixes of each stage group's launches (the k-space stage also
 # launches the small k_x = 0 column kernel, counted with it)
 GROUP_KERNELS = {"deposit_chain": ("k_bucket_count", "k_scan_local", "k_scan_partials", "k_scan_add", "k_scatter",
-                                   "k_deposit_tiles"),
+                                   "k_deposit"),
                  "r2c": ("k_fft_x_fwd", "k_fft_y_fwd"), "kspace": ("k_fft_z_green",),
                  "c2r": ("k_fft_y_inv", "k_fft_x_inv"), "interp": ("k_interp",)}
 

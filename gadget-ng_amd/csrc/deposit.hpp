@@ -20,7 +20,7 @@
 //   3. k_scatter       particles to bucket order as 24-byte cell records
 //      (PartRec: per axis the cell index and a 43-bit in-cell fraction, plus
 //      the FP32 mass), and the sum of the fixed-point masses.
-//   4. k_deposit_tiles one workgroup per tile owns its T^3 cells outright.  It
+//   4. k_deposit       one workgroup per tile owns its T^3 cells outright.  It
 //      reads its own particles and, from the 7 lower neighbour tiles, only the
 //      classes that reach into it, and adds each of the 8 CIC targets exactly
 //      once over all tiles (target offset a lands in tile t + (a & class)).
@@ -56,8 +56,7 @@ struct TileMap {
   // workgroup finds its 72 bucket offsets after one table load
   const unsigned* src;
   // per tile rank, kRangeWords words of the flattened layout of its 14
-  // bucket ranges, filled by k_tile_ranges for each solve (null: the deposit
-  // works it out from the offsets itself)
+  // bucket ranges, filled by k_tile_ranges for each solve
   unsigned* ranges;
 };
 
@@ -83,10 +82,6 @@ __device__ __forceinline__ void zero_body(uint4* __restrict__ p, long long n16) 
     p[i] = z;
 }
 
-__global__ __launch_bounds__(256) void k_zero(uint4* __restrict__ p, long long n16) {
-  zero_body(p, n16);
-}
-
 // The bucket counts cleared and, by the first workgroup, the solve's scalars
 // reset: the two clears before a sort in one launch.
 __global__ __launch_bounds__(256) void k_sort_reset(uint4* __restrict__ p, long long n16, SolveScalars* sc) {
@@ -94,8 +89,9 @@ __global__ __launch_bounds__(256) void k_sort_reset(uint4* __restrict__ p, long 
   zero_body(p, n16);
 }
 
-__global__ __launch_bounds__(256) void k_zero_box(const BoxArgs* __restrict__ bx, long long n16) {
+__global__ __launch_bounds__(256) void k_sort_reset_box(const BoxArgs* __restrict__ bx, long long n16) {
   const BoxArgs& b = bx[blockIdx.z];
+  if (blockIdx.x == 0) reset_scalars_body(b.sc);
   zero_body(reinterpret_cast<uint4*>(b.count), n16);
 }
 
@@ -220,7 +216,7 @@ __global__ __launch_bounds__(256) void k_bucket_count_box(const BoxArgs* __restr
 }
 
 // Exclusive scan of `count` (nb entries) into `offset` (nb + 1 entries),
-// in the three phases of scan.hpp.
+// in the two launches of scan.hpp (the second adds each workgroup's prefix).
 __global__ __launch_bounds__(256) void k_scan_local(const unsigned* __restrict__ count, unsigned* __restrict__ offset,
                                                     unsigned* __restrict__ partial, long long nb) {
   scan_local_body(count, offset, partial, nb);
@@ -231,30 +227,15 @@ __global__ __launch_bounds__(256) void k_scan_local_box(const BoxArgs* __restric
   scan_local_body(b.count, b.offset, b.partial, nb);
 }
 
-__global__ __launch_bounds__(256) void k_scan_partials(unsigned* __restrict__ partial, int nblocks,
-                                                       unsigned* __restrict__ offset, long long nb) {
-  scan_partials_body(partial, nblocks, offset, nb);
-}
-
-__global__ __launch_bounds__(256) void k_scan_partials_box(const BoxArgs* __restrict__ bx, int nblocks, long long nb) {
-  const BoxArgs& b = bx[blockIdx.z];
-  scan_partials_body(b.partial, nblocks, b.offset, nb);
-}
-
-__global__ __launch_bounds__(256) void k_scan_add(unsigned* __restrict__ offset, const unsigned* __restrict__ partial,
-                                                  long long nb) {
-  scan_add_body(offset, partial, nb);
-}
-
 __global__ __launch_bounds__(256) void k_scan_add_prefix(unsigned* __restrict__ offset,
                                                          const unsigned* __restrict__ partial, int nblocks,
                                                          long long nb) {
   scan_add_prefix_body(offset, partial, nblocks, nb);
 }
 
-__global__ __launch_bounds__(256) void k_scan_add_box(const BoxArgs* __restrict__ bx, long long nb) {
+__global__ __launch_bounds__(256) void k_scan_add_prefix_box(const BoxArgs* __restrict__ bx, int nblocks, long long nb) {
   const BoxArgs& b = bx[blockIdx.z];
-  scan_add_body(b.offset, b.partial, nb);
+  scan_add_prefix_body(b.offset, b.partial, nblocks, nb);
 }
 
 // Particle i to its bucket slot as a cell record, and the sum of the
@@ -335,29 +316,6 @@ __global__ __launch_bounds__(256) void k_scatter_box(const BoxArgs* __restrict__
                              nullptr, b.sc);
 }
 
-// LDS fixed-point add with wavefront aggregation: the lanes whose cell equals
-// the first valid lane's cell sum their contributions in registers and one
-// lane adds the total; the others add directly.  In a dense cluster most of a
-// wavefront hits one cell, so this turns 64 serialised atomics into one; with
-// scattered cells the ballot finds a single match and the reduction is skipped.
-// Integer sums keep the result independent of the grouping.
-__device__ __forceinline__ void lds_add_aggregated(unsigned long long* acc, int cell, long long q, bool valid) {
-  const unsigned long long vmask = __ballot(valid);
-  if (vmask == 0ull) return;
-  const int lane = threadIdx.x & 63;
-  const int leader = __ffsll((long long)vmask) - 1;
-  const int lcell = __shfl(cell, leader);
-  const bool mine = valid && cell == lcell;
-  const unsigned long long mm = __ballot(mine);
-  if (__popcll(mm) > 1) {
-    long long v = mine ? q : 0ll;
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    if (lane == leader) atomicAdd(acc + lcell, (unsigned long long)v);
-    valid = valid && !mine;
-  }
-  if (valid) atomicAdd(acc + cell, (unsigned long long)q);
-}
-
 // The 14 bucket ranges a tile reads: (d, first class, end class).  d is the
 // neighbour offset (bit 0 x, bit 1 y, bit 2 z: the source tile is u - d) and
 // the classes are those containing every bit of d, merged where adjacent.
@@ -372,47 +330,60 @@ constexpr unsigned long long kRangeD = pack_range_d();
 __constant__ unsigned char kRangeLo[14] = {0, 1, 3, 5, 7, 2, 6, 3, 7, 4, 5, 7, 6, 7};
 __constant__ unsigned char kRangeHi[14] = {8, 2, 4, 6, 8, 4, 8, 4, 8, 8, 6, 8, 8, 8};
 
-// Heavy tiles over several workgroups.  Workgroup r of the deposit handles
-// tile rank r.  A tile whose 14 ranges hold more than kSliceItems particles
-// gets S = ceil(items / kSliceItems) slices (at most kMaxSlices): its own
-// workgroup takes slice 0, and S - 1 extra workgroups past the ntiles
-// primary ones take the others, each depositing an equal share of the
-// ranges into its own LDS tile.  The slices add their int64 tiles into a
-// scratch tile with global atomics (integer sums: the result does not depend
-// on the order or on how a tile is split) and the last slice to finish
-// converts the scratch tile and clears it for the next solve.  Clustered
-// inputs otherwise leave a few Plummer-core tiles running hundreds of rounds
-// on one workgroup each.
-constexpr unsigned kSliceItems = 32768;
+// Heavy tiles over several workgroups.  A tile whose 14 ranges hold more than
+// `items` particles gets S = ceil(count / items) slices (at most kMaxSlices):
+// S workgroups of their own, in front of those of the ordinary tiles so that
+// the longest work starts first, each depositing an equal share of the ranges
+// into its own LDS tile.  The slices add their int64 tiles into a scratch
+// tile with global atomics (integer sums: the result does not depend on the
+// order or on how a tile is split) and the last slice to finish converts the
+// scratch tile and clears it for the next solve.  Clustered inputs otherwise
+// leave a few Plummer-core tiles running hundreds of rounds on one workgroup
+// each while the chip idles.
 constexpr unsigned kMaxSlices = 1024;
 constexpr unsigned kNoSlice = 0xffffffffu;
 
 struct DepositSplit {
-  const unsigned* slices;        // slices of each tile rank (null: no splitting)
-  const unsigned* slot;          // scratch tile of each split tile rank
-  const unsigned* extra;         // extra workgroup e -> rank | slice << 20, or kNoSlice
-  const SolveScalars* sc;        // split_budget: extra workgroups reserved this solve
-  unsigned ntiles, slots;
-  unsigned long long* scratch;   // slots x T^3 partial tiles, zero between solves
-  unsigned* done;                // slots finished-slice counters, zero between solves
+  unsigned* extra;   // slice workgroup e -> rank | slice << 20, or kNoSlice
+  unsigned slots;    // slice workgroups launched (0: no splitting)
+  unsigned items;    // particles per slice
+  unsigned long long* scratch;   // slots / 2 x T^3 partial tiles, zero between solves
+  unsigned* done;                // slots / 2 finished-slice counters, zero between solves
 };
+
+// Slice workgroups (and half as many scratch tiles) for n particles: a tile
+// is split only above `items`, so S <= 2 count / items, and 2 n / items
+// covers every split tile unless most particles also feed neighbour tiles;
+// then the budget runs out and the remaining heavy tiles run unsplit.
+inline unsigned deposit_slots(long long n, unsigned items) { return (unsigned)((2 * n / items + 16) & ~7LL); }
 
 // The flattened range layout of every tile rank r, written after the scatter
 // so that a deposit workgroup reads its whole prologue with scalar loads:
 // ranges[kRangeWords r + k] is, for k < 13, the end of range k when the 14
 // ranges are laid end to end; word 13 is their total, word 14 the slot delta
 // of range 0 (sorted slot = flattened index + delta) and word 15 + k the
-// change of that delta from range k to k + 1.  Thread 0 also sums the
-// scatter's fixed-point mass slots into sc->qtot.
+// change of that delta from range k to k + 1.  Word 28 is the tile's slice
+// count (1: not split) and word 29 its scratch tile: a tile above sp.items
+// particles reserves S slice workgroups from the budget sp.slots with one
+// atomic and writes their table entries; S >= 2, so reservation / 2 names a
+// scratch tile that no other tile has.  A tile that finds the budget spent
+// marks its reservation unused and runs unsplit.  The first wavefront also
+// sums the scatter's fixed-point mass slots into the integer part of the mean
+// mass per cell (sc->qmean) and keeps the fixed-point exponent (sc->shift).
 constexpr int kRangeWords = 32;
-__global__ __launch_bounds__(256) void k_tile_ranges(const unsigned* __restrict__ offset, const TileMap tm,
-                                                     SolveScalars* sc) {
+__device__ __forceinline__ void tile_ranges_body(const unsigned* __restrict__ offset, const TileMap& tm,
+                                                 SolveScalars* sc, long long ntot, const DepositSplit& sp) {
   const unsigned ntiles = (unsigned)tm.nt * tm.nt * tm.nt;
   const unsigned r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r == 0) {
-    unsigned long long q = 0;
-    for (int k = 0; k < kQSlots; ++k) q += sc->qsum[k * kQStride];
-    sc->qtot = q;
+  if (blockIdx.x == 0 && threadIdx.x < 64) {
+    static_assert(kQSlots == 64, "one mass slot per lane");
+    unsigned long long q = sc->qsum[threadIdx.x * kQStride];
+    for (int off = 32; off > 0; off >>= 1) q += __shfl_xor(q, off);
+    if (threadIdx.x == 0) {
+      const long long nm = (long long)tm.T * tm.nt;
+      sc->qmean = (long long)(q / (unsigned long long)(nm * nm * nm));
+      sc->shift = fixed_shift(sc, ntot);
+    }
   }
   if (r >= ntiles) return;
   unsigned w[kRangeWords];
@@ -431,25 +402,53 @@ __global__ __launch_bounds__(256) void k_tile_ranges(const unsigned* __restrict_
     prev = delta;
   }
   w[13] = pre;
-#pragma unroll
-  for (int k = 28; k < kRangeWords; ++k) w[k] = 0u;
+  unsigned S = 1u, slot = 0u;
+  if (sp.slots != 0u && pre > sp.items) {
+    S = (pre + sp.items - 1u) / sp.items;
+    if (S > kMaxSlices) S = kMaxSlices;
+    const unsigned base = atomicAdd(&sc->split_budget, S);
+    if (base + S > sp.slots) {
+      for (unsigned e = base; e < sp.slots; ++e) sp.extra[e] = kNoSlice;
+      S = 1u;
+    } else {
+      slot = base / 2u;
+      for (unsigned k = 0; k < S; ++k) sp.extra[base + k] = r | (k << 20);
+    }
+  }
+  w[28] = S;
+  w[29] = slot;
+  w[30] = w[31] = 0u;
   uint4* dst = reinterpret_cast<uint4*>(tm.ranges + (size_t)r * kRangeWords);
 #pragma unroll
   for (int k = 0; k < kRangeWords / 4; ++k) dst[k] = make_uint4(w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]);
+}
+
+__global__ __launch_bounds__(256) void k_tile_ranges(const unsigned* __restrict__ offset, const TileMap tm,
+                                                     SolveScalars* sc, long long ntot, const DepositSplit sp) {
+  tile_ranges_body(offset, tm, sc, ntot, sp);
+}
+
+__global__ __launch_bounds__(256) void k_tile_ranges_box(const BoxArgs* __restrict__ bx, const TileMap tm) {
+  const BoxArgs& b = bx[blockIdx.z];
+  TileMap t = tm;
+  t.ranges = b.ranges;
+  tile_ranges_body(b.offset, t, b.sc, b.n, DepositSplit{});
 }
 
 // The 8 CIC targets of one cell record of source range r (d = the range's
 // neighbour offset) into the LDS tile acc of T^3 int64 accumulators: FP64
 // weights (the 43-bit fractions convert exactly, 1 - f is exact, and the
 // products round far below the fixed-point unit) times m 2^s (scale), as
-// 64-bit fixed point.  Every lane of the wavefront calls it (live marks the
-// lanes with a record), so the ballots see whole waves.
+// 64-bit fixed point; live marks the lanes with a record.  Every lane adds
+// directly, also where a clump puts much of a wavefront into one cell: lanes
+// on one LDS word take turns, but summing them with shuffles first costs as
+// many LDS turns (deposit of 512^3 particles, 30 % in Plummer spheres of 0.4
+// cells, on 1024^3: 3.42 ms with a shuffle reduction of the most common cell,
+// 2.78 ms without; 2^22 particles in one cell: 0.32 ms either way).
 template <int T>
 __device__ __forceinline__ void deposit_record(unsigned long long* acc, const PartRec& p, int r, bool live,
                                                double scale) {
-  const int lane = threadIdx.x & 63;
   const int d = (int)((kRangeD >> (3 * r)) & 7ull);
-  const int dx = d & 1, dy = (d >> 1) & 1, dz = (d >> 2) & 1;
   const double fx = rec_frac(p, 0), fy = rec_frac(p, 1), fz = rec_frac(p, 2);
   const double ms = (double)rec_mass(p) * scale;
   const double wx[2] = {1.0 - fx, fx}, wy[2] = {1.0 - fy, fy};
@@ -457,14 +456,7 @@ __device__ __forceinline__ void deposit_record(unsigned long long* acc, const Pa
   // local base index in the particle's own tile; its class follows from it
   const int lx0 = rec_cell(p, 0) % T, ly0 = rec_cell(p, 1) % T, lz0 = rec_cell(p, 2) % T;
   const int cx = lx0 == T - 1, cy = ly0 == T - 1, cz = lz0 == T - 1;
-  // Crowded wavefront: some lane shares its base cell (and source range)
-  // with the lane before it, as in dense clumps, where the sorted order puts
-  // a cell's particles next to each other.  Only then do the targets go
-  // through the wave-level aggregation; otherwise each lane adds directly.
-  // Integer sums are exact, so both paths give the same totals.
-  const int key = (((lz0 * T + ly0) * T + lx0) << 3) | d;
-  const int prev_key = __shfl_up(key, 1);
-  const bool crowded = __ballot(live && lane != 0 && prev_key == key) != 0ull;
+  const int dx = d & 1, dy = (d >> 1) & 1, dz = (d >> 2) & 1;
 #pragma unroll
   for (int a = 0; a < 2; ++a) {
     const int lz = dz ? 0 : lz0 + a;
@@ -475,274 +467,270 @@ __device__ __forceinline__ void deposit_record(unsigned long long* acc, const Pa
       for (int c = 0; c < 2; ++c) {
         const int lx = dx ? 0 : lx0 + c;
         const bool valid = live && (a & cz) == dz && (b & cy) == dy && (c & cx) == dx;
-        const long long qv = valid ? rint_small(wx[c] * (wy[b] * wz[a])) : 0ll;
-        if (crowded)
-          lds_add_aggregated(acc, valid ? (lz * T + ly) * T + lx : 0, qv, valid);
-        else if (valid)
-          atomicAdd(acc + (lz * T + ly) * T + lx, (unsigned long long)qv);
+        if (valid) atomicAdd(acc + (lz * T + ly) * T + lx, (unsigned long long)rint_small(wx[c] * (wy[b] * wz[a])));
       }
     }
   }
 }
 
-// Particles the 14 ranges of the tile of rank r hold, from the bucket offsets.
-__device__ __forceinline__ unsigned tile_items(const unsigned* __restrict__ offset, const TileMap& tm, unsigned r) {
-  unsigned w = 0;
-#pragma unroll
-  for (int k = 0; k < 14; ++k) {
-    const int d = (int)((kRangeD >> (3 * k)) & 7ull);
-    const unsigned b = tm.src[(size_t)r * 8 + d];
-    w += offset[b + kRangeHi[k]] - offset[b + kRangeLo[k]];
-  }
-  return w;
-}
-
-// Slices per tile rank.  A split tile reserves its S - 1 extra workgroups
-// from a budget of `slots` and writes their table entries; the first of them
-// also names its scratch tile.  A tile that finds the budget spent marks its
-// reservation unused and runs unsplit, so no more than ntiles + slots
-// workgroups are ever needed.
-__global__ __launch_bounds__(256) void k_deposit_plan(const unsigned* __restrict__ offset, const TileMap tm,
-                                                      unsigned* __restrict__ slices, unsigned* __restrict__ slot,
-                                                      unsigned* __restrict__ extra, SolveScalars* sc,
-                                                      unsigned slots) {
-  const unsigned ntiles = (unsigned)tm.nt * tm.nt * tm.nt;
-  const unsigned r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= ntiles) return;
-  const unsigned w = tile_items(offset, tm, r);
-  unsigned S = w > kSliceItems ? (w + kSliceItems - 1) / kSliceItems : 1u;
-  if (S > kMaxSlices) S = kMaxSlices;
-  if (S > 1) {
-    const unsigned base = atomicAdd(&sc->split_budget, S - 1u);
-    if (base + S - 1u > slots) {
-      for (unsigned e = base; e < slots; ++e) extra[e] = kNoSlice;
-      S = 1;
-    } else {
-      slot[r] = base;
-      for (unsigned k = 1; k < S; ++k) extra[base + k - 1u] = r | (k << 20);
-    }
-  }
-  slices[r] = S;
-}
-// One workgroup per tile; T is the tile side (T^3 int64 accumulators in LDS).
-// Cell (x, y, z) of the shifted mass mesh is rho[z*rho_plane + y*nm + x];
-// keep (when not null) receives the unshifted mass per cell, unpadded.
-// The 72 bucket offsets of the 8 source tiles are fetched in parallel, the 14
-// ranges are laid end to end, and all their particles are processed in one
-// flat loop, so the only serial latency is one offset load.  Eight wavefronts
-// per workgroup: the LDS accumulators cap a CU at four tiles, and eight waves
-// each keep twice as many particle loads and atomics in flight as four.
-constexpr int kDepositThreads = 512;
-
-//
-// TABLE: the range layout and the mass total come from k_tile_ranges (scalar
-// loads, no LDS prologue); otherwise the workgroup computes them.
-template <int T, int NT = kDepositThreads, bool SPLIT = false, bool TABLE = false>
-__device__ __forceinline__ void deposit_tiles_body(const PartRec* __restrict__ sorted,
-                                                       const unsigned* __restrict__ offset, const CellMap cm,
-                                                       const TileMap tm, const SolveScalars* sc, long long ntot,
-                                                       float* __restrict__ rho, long long rho_plane,
-                                                       float* __restrict__ keep,
-                                                       const DepositSplit sp = DepositSplit{}) {
-  constexpr int T3 = T * T * T;
-  __shared__ unsigned long long acc[T3];
-  // Prologue scratch inside the accumulator tile, which is cleared only after
-  // it has been read: the bucket offsets of the 8 source tiles (72 words),
-  // the range prefix sums (15) and slot deltas (14), and the mass total.
-  // With no other LDS the 16^3 tile takes exactly 32 KB, so five workgroups
-  // share a CU's 160 KB instead of four.
-  static_assert(T3 * 2 >= 106, "the prologue scratch must fit in the tile");
-  unsigned* const toff = reinterpret_cast<unsigned*>(acc);  // [8][9]
-  unsigned* const rpre = toff + 72;                         // [15]
-  unsigned* const rdelta = toff + 88;                       // [14]
-  unsigned long long* const qtotp = acc + 52;               // words 104-105
-  const int tid = threadIdx.x;
-  const int nt = tm.nt;
-  // this workgroup's tile rank and slice (k of S): the primary workgroups
-  // [0, ntiles) take slice 0 of their rank, extra workgroups the others
-  unsigned rank_r = blockIdx.x, k_slice = 0, n_slice = 1, my_slot = 0;
-  if constexpr (SPLIT) {
-    if (blockIdx.x >= sp.ntiles) {
-      const unsigned e = blockIdx.x - sp.ntiles;
-      if (e >= sp.slots || e >= sp.sc->split_budget) return;  // uniform: no slice for this workgroup
-      const unsigned v = sp.extra[e];
-      if (v == kNoSlice) return;
-      rank_r = v & 0xfffffu;
-      k_slice = v >> 20;
-    }
-    n_slice = sp.slices[rank_r];
-    if (n_slice > 1) my_slot = sp.slot[rank_r];
-  }
-  // the tile itself is needed only for the output rows; its load and the
-  // source-bucket load below depend on the rank alone
-  const int tile = (int)tm.order[rank_r];
-  const int ux = tile % nt, uy = (tile / nt) % nt, uz = tile / (nt * nt);
-  // range ends and slot deltas, uniform over the workgroup, in scalar
-  // registers
-  unsigned rend[13], dstep[13], dbase, all;
-  unsigned long long qtot;
-  if constexpr (TABLE) {
-    const unsigned* __restrict__ w = tm.ranges + (size_t)rank_r * kRangeWords;
+// Record of flattened item q of the tile whose range row is w (uniform, so
+// its words come from the scalar cache), for q < limit: the sorted slot is q
+// plus the delta of its range, summed as masked steps over the range ends at
+// or below q (range ends never decrease; written as arithmetic so that it
+// stays in registers).  Range 0, the tile's own bucket, holds most of its
+// particles: a wavefront whose 64 items all lie in it (the items of a
+// wavefront are consecutive, lane 0's first) skips the per-lane search.
+__device__ __forceinline__ PartRec fetch_record(const PartRec* __restrict__ sorted, const unsigned* __restrict__ w,
+                                                unsigned q, unsigned limit, int& r, bool& live) {
+  const unsigned qw = __builtin_amdgcn_readfirstlane(q);
+  unsigned dl = w[14];
+  r = 0;
+  if (qw + 63u >= w[0]) {
 #pragma unroll
     for (int k = 0; k < 13; ++k) {
-      rend[k] = w[k];
-      dstep[k] = w[15 + k];
+      const bool ge = q >= w[k];
+      r += ge ? 1 : 0;
+      dl += w[15 + k] & (0u - (unsigned)ge);
     }
-    all = w[13];
-    dbase = w[14];
-    qtot = sc->qtot;
+  }
+  live = q < limit;
+  PartRec v;
+  if (live) {
+    v = sorted[q + dl];
   } else {
-  if (tid < 72) {
-    const int d = tid / 9, j = tid % 9;
-    toff[d * 9 + j] = offset[tm.src[(size_t)rank_r * 8 + d] + j];
+    v.a[0] = v.a[1] = v.a[2] = 0ull;
   }
-  // the fixed-point mass total, reduced by the third wavefront while the
-  // offsets load (one slot per lane; NT >= 256)
-  static_assert(NT >= 192 && kQSlots == 64, "one qsum slot per lane of the third wavefront");
-  if (tid >= 128 && tid < 192) {
-    unsigned long long v = sc->qsum[(tid - 128) * kQStride];
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off);
-    if (tid == 128) *qtotp = v;
-  }
-  __syncthreads();
-  if (tid < 64) {
-    unsigned len = 0, beg = 0;
-    if (tid < 14) {
-      const int d = (int)((kRangeD >> (3 * tid)) & 7ull);
-      beg = toff[d * 9 + kRangeLo[tid]];
-      len = toff[d * 9 + kRangeHi[tid]] - beg;
-    }
-    unsigned incl = len;
-    for (int off = 1; off < 16; off <<= 1) {
-      const unsigned t = __shfl_up(incl, off);
-      if (tid >= off) incl += t;
-    }
-    if (tid < 14) {
-      rpre[tid + 1] = incl;
-      // slot of particle q of range tid in the sorted array: q + rdelta
-      rdelta[tid] = beg - (incl - len);
-    }
-    if (tid == 0) rpre[0] = 0;
-  }
-  __syncthreads();
-  // then the scratch is free for the accumulators
-#pragma unroll
-  for (int k = 0; k < 13; ++k) rend[k] = __builtin_amdgcn_readfirstlane(rpre[k + 1]);
-  dbase = __builtin_amdgcn_readfirstlane(rdelta[0]);
-#pragma unroll
-  for (int k = 0; k < 13; ++k) dstep[k] = __builtin_amdgcn_readfirstlane(rdelta[k + 1] - rdelta[k]);
-  all = __builtin_amdgcn_readfirstlane(rpre[14]);
-  qtot = *qtotp;
-  __syncthreads();
-  }
-  const int s = fixed_shift(sc, ntot);
-  // this slice's share [q0, total) of the tile's flattened ranges
-  unsigned q0 = 0, total = all;
-  if constexpr (SPLIT) {
-    const unsigned share = (all + n_slice - 1u) / n_slice;
-    q0 = min(all, k_slice * share);
-    total = min(all, q0 + share);
-  }
-  // every lane of a wavefront runs the same number of iterations (lanes past
-  // the end carry no particle), so the aggregation ballots see whole waves
+  return v;
+}
+
+// Rounds of records in flight at once: a tile of the uniform headline holds
+// about 2.5 rounds at 256 threads, so all of its loads share one memory
+// latency.  Slot j holds the record of round it + j; the round loops are
+// unrolled by kPrefetch so every slot index is static.
+constexpr int kPrefetch = 3;
+
+// Workgroup index b of n to item index so that each XCD (workgroups are dealt
+// to the eight round robin) works on one contiguous eighth of the items.
+__device__ __forceinline__ unsigned xcd_item(unsigned b, unsigned n) {
+  const unsigned per = (n + 7u) / 8u;
+  return (b & 7u) * per + (b >> 3);
+}
+constexpr unsigned xcd_grid(unsigned n) { return (n + 7u) / 8u * 8u; }
+
+// One slice of a heavy tile (sp): its share of the flattened ranges into the
+// LDS tile, the LDS tile into the scratch tile, and the last slice of the
+// tile converts.
+template <int T, int NT>
+__device__ __forceinline__ void deposit_slice(unsigned long long* acc, const PartRec* __restrict__ sorted,
+                                              const CellMap& cm, const TileMap& tm, const SolveScalars* sc,
+                                              float* __restrict__ rho, long long rho_plane, float* __restrict__ keep,
+                                              const DepositSplit& sp) {
+  constexpr int T3 = T * T * T;
+  const int tid = threadIdx.x, nt = tm.nt;
+  const unsigned e = blockIdx.x;
+  if (e >= sc->split_budget) return;  // uniform: no slice for this workgroup
+  const unsigned v = sp.extra[e];
+  if (v == kNoSlice) return;
+  const unsigned rank = v & 0xfffffu;
+  const unsigned* __restrict__ w = tm.ranges + (size_t)rank * kRangeWords;
+  const unsigned all = w[13], S = w[28], slot = w[29];
+  const unsigned share = (all + S - 1u) / S;
+  const unsigned q0 = min(all, (v >> 20) * share), total = min(all, q0 + share);
   const unsigned rounds = (total - q0 + NT - 1u) / NT;
-  // Range r of flattened item q (the number of range ends at or below it, 13
-  // past the end) and its record: the sorted slot is q + the delta of its
-  // range, summed as masked steps over the range starts at or below q (range
-  // ends never decrease; written as arithmetic so that it stays in
-  // registers).  Range 0, the tile's own bucket, holds most of its particles:
-  // a wavefront whose 64 items all lie in it (the items of a wavefront are
-  // consecutive, lane 0's first) skips the per-lane search.
-  auto fetch = [&](unsigned q, int& r) {
-    const unsigned qw = __builtin_amdgcn_readfirstlane(q);
-    unsigned dl = dbase;
-    r = 0;
-    if (qw + 63u >= rend[0]) {
-#pragma unroll
-      for (int k = 0; k < 13; ++k) {
-        const bool ge = q >= rend[k];
-        r += ge ? 1 : 0;
-        dl += dstep[k] & (0u - (unsigned)ge);
-      }
-    }
-    PartRec v;
-    if (q < total) {
-      v = sorted[q + dl];
-    } else {
-      v.a[0] = v.a[1] = v.a[2] = 0ull;
-    }
-    return v;
-  };
-  // m 2^s of a record: the FP32 mass scaled exactly
-  const double scale = ldexp(1.0, s);
-  auto deposit_one = [&](const PartRec& p, int r, bool live) { deposit_record<T>(acc, p, r, live, scale); };
-  // kPrefetch rounds of records are in flight at once: a tile of the uniform
-  // headline holds about 2.5 rounds at 256 threads, so all of its loads
-  // share one memory latency.  Slot j holds the record of round it + j; the
-  // round loop is unrolled by kPrefetch so every slot index is static.
-  constexpr int kPrefetch = 3;
-  const unsigned qbase = q0 + (unsigned)tid;
+  const double scale = ldexp(1.0, sc->shift), unit = ldexp(1.0, -sc->shift);
   PartRec buf[kPrefetch];
   int rbuf[kPrefetch];
+  bool lbuf[kPrefetch];
 #pragma unroll
   for (int j = 0; j < kPrefetch; ++j) {
-    const unsigned qj = qbase + (unsigned)j * NT;
-    buf[j] = fetch(qj, rbuf[j]);
+    rbuf[j] = 0;
+    lbuf[j] = false;
+    if ((unsigned)j < rounds) buf[j] = fetch_record(sorted, w, q0 + j * NT + tid, total, rbuf[j], lbuf[j]);
   }
-  // the accumulators are cleared while the first records load
   for (int c = tid; c < T3; c += NT) acc[c] = 0ull;
   __syncthreads();
   for (unsigned it = 0; it < rounds; it += kPrefetch) {
 #pragma unroll
     for (int j = 0; j < kPrefetch; ++j) {
-      if (it + j < rounds) {  // uniform over the workgroup
-        const unsigned qc = qbase + (it + j) * NT;
+      const unsigned g = it + (unsigned)j;
+      if (g < rounds) {  // uniform over the workgroup
         const PartRec p = buf[j];
         const int r = rbuf[j];
-        if (it + j + kPrefetch < rounds) {
-          const unsigned qn = qc + (unsigned)kPrefetch * NT;
-          buf[j] = fetch(qn, rbuf[j]);
-        }
-        deposit_one(p, r, qc < total);
+        const bool live = lbuf[j];
+        if (g + kPrefetch < rounds)
+          buf[j] = fetch_record(sorted, w, q0 + (g + kPrefetch) * NT + tid, total, rbuf[j], lbuf[j]);
+        deposit_record<T>(acc, p, r, live, scale);
       }
     }
   }
   __syncthreads();
-  unsigned long long* part = nullptr;
-  if (SPLIT && n_slice > 1) {
-    // add this slice's partial tile into the scratch tile; the last slice
-    // to finish converts the sum and clears the scratch tile
-    part = sp.scratch + (size_t)my_slot * T3;
-    for (int c = tid; c < T3; c += NT) {
-      const unsigned long long v = acc[c];
-      if (v) atomicAdd(part + c, v);
-    }
-    __threadfence();
-    __syncthreads();
-    // the accumulators have been read: their first word holds the flag
-    unsigned* const last = reinterpret_cast<unsigned*>(acc);
-    if (tid == 0) *last = atomicAdd(sp.done + my_slot, 1u) == n_slice - 1u;
-    __syncthreads();
-    if (!*last) return;
-    __threadfence();
+  unsigned long long* part = sp.scratch + (size_t)slot * T3;
+  for (int c = tid; c < T3; c += NT) {
+    const unsigned long long x = acc[c];
+    if (x) atomicAdd(part + c, x);
   }
-  const double unit = ldexp(1.0, -s);
-  // the integer part of the mean fixed-point mass per cell
-  const long long qmean = (long long)(qtot / (unsigned long long)((long long)cm.nm * cm.nm * cm.nm));
+  __threadfence();
+  __syncthreads();
+  // the accumulators have been read: their first word holds the flag
+  unsigned* const last = reinterpret_cast<unsigned*>(acc);
+  if (tid == 0) *last = atomicAdd(sp.done + slot, 1u) == S - 1u;
+  __syncthreads();
+  if (!*last) return;
+  __threadfence();
+  const int tile = (int)tm.order[rank];
+  const int ux = tile % nt, uy = (tile / nt) % nt, uz = tile / (nt * nt);
+  const long long qmean = sc->qmean;
   for (int c = tid; c < T3; c += NT) {
     const int lx = c % T, ly = (c / T) % T, lz = c / (T * T);
     const size_t row = (size_t)(uy * T + ly) * cm.nm + (ux * T + lx);
-    long long v;
-    if (SPLIT && part) {
-      v = (long long)__hip_atomic_load(part + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      part[c] = 0ull;
-    } else {
-      v = (long long)acc[c];
-    }
-    rho[(size_t)(uz * T + lz) * rho_plane + row] = (float)((double)(v - qmean) * unit);
-    if (keep) keep[(size_t)(uz * T + lz) * cm.nm * cm.nm + row] = (float)((double)v * unit);
+    const long long x = (long long)__hip_atomic_load(part + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    part[c] = 0ull;
+    rho[(size_t)(uz * T + lz) * rho_plane + row] = (float)((double)(x - qmean) * unit);
+    if (keep) keep[(size_t)(uz * T + lz) * cm.nm * cm.nm + row] = (float)((double)x * unit);
   }
-  if (SPLIT && part && tid == 0) sp.done[my_slot] = 0u;
+  if (tid == 0) sp.done[slot] = 0u;
+}
+
+// One workgroup per group of TILES tiles (1 or 2, neighbours along the
+// Hilbert curve); T is the tile side (T^3 int64 accumulators in LDS).  Cell
+// (x, y, z) of the shifted mass mesh is rho[z*rho_plane + y*nm + x]; keep
+// (when not null) receives the unshifted mass per cell, unpadded.  The first
+// sp.slots workgroups of the grid are the slices of the heavy tiles, which
+// the others skip.
+// With two tiles, their rounds of records form one sequence, so the prefetch
+// ring runs across the tile boundary: the second tile's records load while
+// the first tile is converted and written.
+template <int T, int NT, int TILES>
+__device__ __forceinline__ void deposit_body(const PartRec* __restrict__ sorted, const CellMap& cm, const TileMap& tm,
+                                             const SolveScalars* sc, float* __restrict__ rho, long long rho_plane,
+                                             float* __restrict__ keep, const DepositSplit& sp) {
+  constexpr int T3 = T * T * T;
+  __shared__ unsigned long long acc[T3];
+  const int tid = threadIdx.x;
+  const int nt = tm.nt;
+  if (blockIdx.x < sp.slots) {
+    deposit_slice<T, NT>(acc, sorted, cm, tm, sc, rho, rho_plane, keep, sp);
+    return;
+  }
+  const unsigned ntiles = (unsigned)(nt * nt * nt), groups = (ntiles + TILES - 1u) / TILES;
+  const unsigned grp = xcd_item(blockIdx.x - sp.slots, groups);
+  if (grp >= groups) return;  // uniform: padding of the last eighth
+  const unsigned ra = TILES * grp, rb = ra + 1u;
+  const bool has_b = TILES == 2 && rb < ntiles;  // uniform: the last workgroup may hold one tile
+  const unsigned* __restrict__ wa = tm.ranges + (size_t)ra * kRangeWords;
+  const unsigned* __restrict__ wb = tm.ranges + (size_t)(has_b ? rb : ra) * kRangeWords;
+  const bool own_a = wa[28] == 1u, own_b = has_b && wb[28] == 1u;  // not left to slices
+  const unsigned tot_a = own_a ? wa[13] : 0u, tot_b = own_b ? wb[13] : 0u;
+  const unsigned rounds_a = (tot_a + NT - 1u) / NT, rounds = rounds_a + (tot_b + NT - 1u) / NT;
+  const int tile_a = (int)tm.order[ra], tile_b = has_b ? (int)tm.order[rb] : 0;
+  const double scale = ldexp(1.0, sc->shift), unit = ldexp(1.0, -sc->shift);
+  const long long qmean = sc->qmean;
+  // record of concatenated round g: tile a below rounds_a, then tile b
+  auto fetch = [&](unsigned g, int& r, bool& live) {
+    if (TILES == 1) return fetch_record(sorted, wa, g * NT + (unsigned)tid, tot_a, r, live);
+    const bool in_b = g >= rounds_a;  // uniform
+    return fetch_record(sorted, in_b ? wb : wa, (in_b ? g - rounds_a : g) * NT + (unsigned)tid, in_b ? tot_b : tot_a,
+                        r, live);
+  };
+  // the accumulated tile as FP32 mass per cell minus the mean (and, with
+  // keep, unshifted); clears the accumulators behind itself for a next tile
+  auto write_tile = [&](int tile, bool clear) {
+    const int ux = tile % nt, uy = (tile / nt) % nt, uz = tile / (nt * nt);
+    for (int c = tid; c < T3; c += NT) {
+      const int lx = c % T, ly = (c / T) % T, lz = c / (T * T);
+      const size_t row = (size_t)(uy * T + ly) * cm.nm + (ux * T + lx);
+      const long long v = (long long)acc[c];
+      if (clear) acc[c] = 0ull;
+      rho[(size_t)(uz * T + lz) * rho_plane + row] = (float)((double)(v - qmean) * unit);
+      if (keep) keep[(size_t)(uz * T + lz) * cm.nm * cm.nm + row] = (float)((double)v * unit);
+    }
+  };
+  PartRec buf[kPrefetch];
+  int rbuf[kPrefetch];
+  bool lbuf[kPrefetch];
+#pragma unroll
+  for (int j = 0; j < kPrefetch; ++j) {
+    rbuf[j] = 0;
+    lbuf[j] = false;
+    if ((unsigned)j < rounds) buf[j] = fetch((unsigned)j, rbuf[j], lbuf[j]);
+  }
+  // the accumulators are cleared while the first records load
+  for (int c = tid; c < T3; c += NT) acc[c] = 0ull;
+  __syncthreads();
+  if (TILES == 2 && rounds_a == 0u && own_a) {  // an empty tile a: zeros
+    write_tile(tile_a, false);
+    __syncthreads();
+  }
+  for (unsigned it = 0; it < rounds; it += kPrefetch) {
+#pragma unroll
+    for (int j = 0; j < kPrefetch; ++j) {
+      const unsigned g = it + (unsigned)j;
+      if (g < rounds) {  // uniform over the workgroup
+        if (TILES == 2 && g == rounds_a && g != 0u) {
+          // tile a is complete: write it and start tile b from zero
+          __syncthreads();
+          write_tile(tile_a, true);
+          __syncthreads();
+        }
+        const PartRec p = buf[j];
+        const int r = rbuf[j];
+        const bool live = lbuf[j];
+        if (g + kPrefetch < rounds) buf[j] = fetch(g + kPrefetch, rbuf[j], lbuf[j]);
+        deposit_record<T>(acc, p, r, live, scale);
+      }
+    }
+  }
+  __syncthreads();
+  if (TILES == 1) {
+    if (own_a) write_tile(tile_a, false);
+    return;
+  }
+  if (rounds == rounds_a && rounds_a != 0u) {
+    // tile b had no records (or is not this workgroup's): tile a is still in acc
+    write_tile(tile_a, true);
+    __syncthreads();
+  }
+  if (own_b) write_tile(tile_b, false);
+}
+
+// At most 96 VGPRs, so five 256-thread workgroups (the LDS limit of a 16^3
+// tile) fit a CU.
+template <int T, int NT, int TILES>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void k_deposit(
+    const PartRec* __restrict__ sorted, const CellMap cm, const TileMap tm, const SolveScalars* sc,
+    float* __restrict__ rho, long long rho_plane, float* __restrict__ keep, const DepositSplit sp) {
+  deposit_body<T, NT, TILES>(sorted, cm, tm, sc, rho, rho_plane, keep, sp);
+}
+
+template <int T, int NT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void k_deposit_box(
+    const BoxArgs* __restrict__ bx, const TileMap tm) {
+  const BoxArgs& b = bx[blockIdx.z];
+  TileMap t = tm;
+  t.ranges = b.ranges;
+  deposit_body<T, NT, 1>(b.sorted, b.cm, t, b.sc, reinterpret_cast<float*>(b.P), 2 * mesh_plane(b.cm.nm),
+                         nullptr, DepositSplit{});
+}
+
+// LDS fixed-point add with wavefront aggregation: the lanes whose cell equals
+// the first valid lane's cell sum their contributions in registers and one
+// lane adds the total; the others add directly.
+// Integer sums keep the result independent of the grouping.
+__device__ __forceinline__ void lds_add_aggregated(unsigned long long* acc, int cell, long long q, bool valid) {
+  const unsigned long long vmask = __ballot(valid);
+  if (vmask == 0ull) return;
+  const int lane = threadIdx.x & 63;
+  const int leader = __ffsll((long long)vmask) - 1;
+  const int lcell = __shfl(cell, leader);
+  const bool mine = valid && cell == lcell;
+  const unsigned long long mm = __ballot(mine);
+  if (__popcll(mm) > 1) {
+    long long v = mine ? q : 0ll;
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    if (lane == leader) atomicAdd(acc + lcell, (unsigned long long)v);
+    valid = valid && !mine;
+  }
+  if (valid) atomicAdd(acc + cell, (unsigned long long)q);
 }
 
 // Particle moments per cell from the sorted cell records of the last sort,
@@ -807,145 +795,6 @@ __global__ __launch_bounds__(kCellMomThreads) void k_cell_moments(const PartRec*
       for (int k = 0; k < kCellMoments; ++k) mom[cell * kCellMoments + k] = (double)(long long)acc[k][c] * unit;
     }
   }
-}
-
-// At most 96 VGPRs, so five 256-thread workgroups (the LDS limit of a 16^3
-// tile) fit a CU.
-template <int T, int NT = kDepositThreads, bool SPLIT = false>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void k_deposit_tiles(const PartRec* __restrict__ sorted,
-                                                       const unsigned* __restrict__ offset, const CellMap cm,
-                                                       const TileMap tm, const SolveScalars* sc, long long ntot,
-                                                       float* __restrict__ rho, long long rho_plane,
-                                                       float* __restrict__ keep, const DepositSplit sp) {
-  deposit_tiles_body<T, NT, SPLIT, true>(sorted, offset, cm, tm, sc, ntot, rho, rho_plane, keep, sp);
-}
-
-// Two tiles per workgroup: ranks 2w and 2w + 1, neighbours along the
-// Hilbert curve, from the range table.  Their rounds of records form one
-// sequence, so the prefetch ring runs across the tile boundary: the second
-// tile's records load while the first tile is converted and written.  The
-// accumulator tile, the per-record work and the result are those of
-// k_deposit_tiles (integer sums: bit for bit the same density).
-template <int T, int NT>
-__device__ __forceinline__ void deposit_pair_body(const PartRec* __restrict__ sorted, const CellMap cm,
-                                                  const TileMap tm, const SolveScalars* sc, long long ntot,
-                                                  float* __restrict__ rho, long long rho_plane,
-                                                  float* __restrict__ keep) {
-  constexpr int T3 = T * T * T;
-  __shared__ unsigned long long acc[T3];
-  const int tid = threadIdx.x;
-  const int nt = tm.nt;
-  const unsigned ntiles = (unsigned)(nt * nt * nt);
-  const unsigned ra = 2u * blockIdx.x, rb = ra + 1u;
-  const bool has_b = rb < ntiles;  // uniform: the last workgroup may hold one tile
-  const unsigned* __restrict__ wa = tm.ranges + (size_t)ra * kRangeWords;
-  const unsigned* __restrict__ wb = tm.ranges + (size_t)(has_b ? rb : ra) * kRangeWords;
-  const unsigned tot_a = wa[13], dbase_a = wa[14];
-  const unsigned tot_b = has_b ? wb[13] : 0u, dbase_b = wb[14];
-  const unsigned rounds_a = (tot_a + NT - 1u) / NT, rounds_b = (tot_b + NT - 1u) / NT;
-  const unsigned rounds = rounds_a + rounds_b;
-  const int tile_a = (int)tm.order[ra], tile_b = has_b ? (int)tm.order[rb] : 0;
-  const int s = fixed_shift(sc, ntot);
-  const double scale = ldexp(1.0, s), unit = ldexp(1.0, -s);
-  const long long qmean = (long long)(sc->qtot / (unsigned long long)((long long)cm.nm * cm.nm * cm.nm));
-  // record of concatenated round g (tile a below rounds_a, then tile b): its
-  // range r and whether the lane has one; a wavefront whose 64 items all lie
-  // in range 0 skips the per-lane range search, as in k_deposit_tiles
-  // (the range words are read through the uniform table row of the tile, so
-  // they come from the scalar cache rather than living in registers)
-  auto fetch = [&](unsigned g, int& r, bool& live) {
-    const bool in_b = g >= rounds_a;  // uniform
-    const unsigned* __restrict__ w = in_b ? wb : wa;
-    const unsigned q = (in_b ? g - rounds_a : g) * NT + (unsigned)tid;
-    const unsigned qw = __builtin_amdgcn_readfirstlane(q);
-    unsigned dl = in_b ? dbase_b : dbase_a;
-    r = 0;
-    if (qw + 63u >= w[0]) {
-#pragma unroll
-      for (int k = 0; k < 13; ++k) {
-        const bool ge = q >= w[k];
-        r += ge ? 1 : 0;
-        dl += w[15 + k] & (0u - (unsigned)ge);
-      }
-    }
-    live = q < (in_b ? tot_b : tot_a);
-    PartRec v;
-    if (live) {
-      v = sorted[q + dl];
-    } else {
-      v.a[0] = v.a[1] = v.a[2] = 0ull;
-    }
-    return v;
-  };
-  // the accumulated tile as FP32 mass per cell minus the mean (and, with
-  // keep, unshifted), then the accumulators cleared for the next tile
-  auto write_tile = [&](int tile) {
-    const int ux = tile % nt, uy = (tile / nt) % nt, uz = tile / (nt * nt);
-    for (int c = tid; c < T3; c += NT) {
-      const int lx = c % T, ly = (c / T) % T, lz = c / (T * T);
-      const size_t row = (size_t)(uy * T + ly) * cm.nm + (ux * T + lx);
-      const long long v = (long long)acc[c];
-      rho[(size_t)(uz * T + lz) * rho_plane + row] = (float)((double)(v - qmean) * unit);
-      if (keep) keep[(size_t)(uz * T + lz) * cm.nm * cm.nm + row] = (float)((double)v * unit);
-    }
-  };
-  constexpr int kPrefetch = 3;
-  PartRec buf[kPrefetch];
-  int rbuf[kPrefetch];
-  bool lbuf[kPrefetch];
-#pragma unroll
-  for (int j = 0; j < kPrefetch; ++j) {
-    rbuf[j] = 0;
-    lbuf[j] = false;
-    if ((unsigned)j < rounds) buf[j] = fetch((unsigned)j, rbuf[j], lbuf[j]);
-  }
-  for (int c = tid; c < T3; c += NT) acc[c] = 0ull;
-  __syncthreads();
-  for (unsigned it = 0; it < rounds; it += kPrefetch) {
-#pragma unroll
-    for (int j = 0; j < kPrefetch; ++j) {
-      const unsigned g = it + (unsigned)j;
-      if (g < rounds) {  // uniform over the workgroup
-        if (g == rounds_a) {
-          // tile a is complete: write it and start tile b from zero
-          __syncthreads();
-          write_tile(tile_a);
-          __syncthreads();
-          for (int c = tid; c < T3; c += NT) acc[c] = 0ull;
-          __syncthreads();
-        }
-        const PartRec p = buf[j];
-        const int r = rbuf[j];
-        const bool live = lbuf[j];
-        if (g + kPrefetch < rounds) buf[j] = fetch(g + kPrefetch, rbuf[j], lbuf[j]);
-        deposit_record<T>(acc, p, r, live, scale);
-      }
-    }
-  }
-  __syncthreads();
-  if (rounds_b == 0u) {
-    // tile b had no records (or there is no tile b): tile a is still in acc
-    write_tile(tile_a);
-    if (!has_b) return;  // uniform
-    __syncthreads();
-    for (int c = tid; c < T3; c += NT) acc[c] = 0ull;
-    __syncthreads();
-  }
-  write_tile(tile_b);
-}
-
-template <int T, int NT = kDepositThreads>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void k_deposit_pairs(
-    const PartRec* __restrict__ sorted, const CellMap cm, const TileMap tm, const SolveScalars* sc, long long ntot,
-    float* __restrict__ rho, long long rho_plane, float* __restrict__ keep) {
-  deposit_pair_body<T, NT>(sorted, cm, tm, sc, ntot, rho, rho_plane, keep);
-}
-
-template <int T, int NT = kDepositThreads>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void k_deposit_tiles_box(const BoxArgs* __restrict__ bx, const TileMap tm) {
-  const BoxArgs& b = bx[blockIdx.z];
-  deposit_tiles_body<T, NT>(b.sorted, b.offset, b.cm, tm, b.sc, b.n, reinterpret_cast<float*>(b.P),
-                            2 * mesh_plane(b.cm.nm), nullptr);
 }
 
 }  // namespace gng

@@ -77,12 +77,11 @@ constexpr int x_rows() {
 // Deposit tile side: the largest of 16, 12, 8, 4 that divides nm.
 constexpr int deposit_tile(int nm) { return nm % 16 == 0 ? 16 : nm % 12 == 0 ? 12 : nm % 8 == 0 ? 8 : 4; }
 
-// Launch choices with more than one compiled variant.  Defaults: the
-// persistent z pass at nm = 512 (elsewhere it spills or loses occupancy) and
-// 512-thread deposit workgroups; gng_pm_autotune() times the alternatives.
+// Launch choices with more than one compiled variant; default_tuning() holds
+// the rules of the defaults, gng_pm_autotune() times the alternatives.
 struct Tuning {
   int z_persistent = 0;
-  int deposit_wide = 1;
+  int deposit_wide = 0;
   int y_fwd_persistent = 0;
   int y_inv_persistent = 0;
   int tuned = 0;  // 1 when measured (or read from the tuning cache)
@@ -91,7 +90,7 @@ struct Tuning {
   int chunk_inv = 0;      // same for the inverse y/x pass pair
   int deposit_split = 1;  // heavy deposit tiles over several workgroups
   int y_inv_narrow = 1;   // inverse y pass on the narrower tile where one is compiled
-  int deposit_pair = 0;   // unsplit deposit: two tiles per workgroup
+  int deposit_pair = 0;   // two tiles per deposit workgroup
 };
 
 // Planes per chunk when a pass pair runs chunk by chunk, so that the second
@@ -109,10 +108,27 @@ int chunk_rule(int nm, long long budget_mib) {
 // forward pair, 64 and 16 for the inverse pair
 constexpr long long kChunkFwdMiB = 256, kChunkInvMiB = 64;
 
+// Particles per slice of a heavy deposit tile in a solve of n particles: about
+// four slices per CU if every particle sat in a heavy tile, at most 32768
+// (longer slices are the tail of the largest runs) and at least 8192 (a slice
+// ends by adding up to 4096 cells to its scratch tile with global atomics, and
+// shorter slices pay more for those than they gain).  Deposit stage on MI355X,
+// least 2048 / 4096 / 8192: 0.9e6 particles on 192^3 69 / 56 / 64 us, 4.1e6 on
+// 256^3 151 / 149 / 119 us, 16.8e6 on 256^3 383 / 391 / 374 us; one fixed
+// 32768 before: 338, 343 and 673 us.
+unsigned slice_items(long long n) { return (unsigned)std::min<long long>(std::max<long long>(n / 1024, 8192), 32768); }
+
 Tuning default_tuning(int nm) {
   Tuning t;
   t.z_persistent = nm == 512;
-  t.deposit_wide = 1;
+  // 512 threads per deposit tile only where there are fewer tiles than CUs
+  // (64^3: 12 against 13 us); elsewhere four 256-thread workgroups share a
+  // CU's LDS and overlap each other's latencies (512^3, 256^3 particles: 253
+  // against 288 us).  Two tiles per workgroup pay on the largest mesh only
+  // (1024^3: 2.78 against 2.88 ms; 512^3: 260 against 253 us).
+  const int nt = nm / deposit_tile(nm);
+  t.deposit_wide = nt * nt * nt < 256;
+  t.deposit_pair = nm >= 1024;
   t.chunk_fwd = chunk_rule(nm, kChunkFwdMiB);
   // at nm >= 1024 the inverse y pass runs as two launches on full lines, and
   // whole-mesh passes measured faster (10.5 against 11.0 ms at 1024^3)
@@ -120,8 +136,6 @@ Tuning default_tuning(int nm) {
   return t;
 }
 
-// knob 8 (two tiles per deposit workgroup) only acts with the split off, so
-// it comes after knob 6 in the coordinate descent
 constexpr int kKnobs = 9;
 int& knob(Tuning& t, int k) {
   switch (k) {
@@ -294,13 +308,10 @@ struct MeshOps {
   int z_cols;  // the per-item z pass's tiles
   int z_threads;
   int tile;
-  // deposit[v][split]: workgroups of 256 (v = 0) or 512 (v = 1) threads;
-  // split: dense tiles shared by several workgroups
-  void (*deposit[2][2])(dim3, dim3, hipStream_t, const PartRec*, const unsigned*, CellMap, TileMap,
-                        const SolveScalars*, long long, float*, long long, float*, DepositSplit);
-  // deposit_pairs[v]: two tiles per workgroup (unsplit deposit only)
-  void (*deposit_pairs[2])(dim3, dim3, hipStream_t, const PartRec*, CellMap, TileMap, const SolveScalars*, long long,
-                           float*, long long, float*);
+  // deposit[v][t]: workgroups of 256 (v = 0) or 512 (v = 1) threads, each on
+  // t + 1 neighbouring tiles
+  void (*deposit[2][2])(dim3, dim3, hipStream_t, const PartRec*, CellMap, TileMap, const SolveScalars*, float*,
+                        long long, float*, DepositSplit);
   // per-cell particle moments of the sorted records, one workgroup per tile
   void (*cell_moments)(dim3, dim3, hipStream_t, const PartRec*, const unsigned*, CellMap, TileMap,
                        const SolveScalars*, long long, double*);
@@ -355,26 +366,17 @@ MeshOps make_ops() {
   o.z_cols = YZCfg<N>::CZ;
   o.z_threads = YZCfg<N>::TZ;
   o.tile = TD;
-#define GNG_DEPOSIT(V, NT, SPLIT)                                                                          \
-  o.deposit[V][SPLIT] = [](dim3 g, dim3 b, hipStream_t s, const PartRec* srt, const unsigned* off, CellMap cm,     \
-                           TileMap tm, const SolveScalars* sc, long long n, float* rho, long long rho_plane,        \
-                           float* keep, DepositSplit sp) {                                                          \
-    hipLaunchKernelGGL((k_deposit_tiles<TD, NT, SPLIT>), g, b, 0, s, srt, off, cm, tm, sc, n, rho, rho_plane, keep, \
-                       sp);                                                                                         \
+#define GNG_DEPOSIT(V, NT, TILES)                                                                               \
+  o.deposit[V][TILES - 1] = [](dim3 g, dim3 b, hipStream_t s, const PartRec* srt, CellMap cm, TileMap tm,       \
+                               const SolveScalars* sc, float* rho, long long rho_plane, float* keep,            \
+                               DepositSplit sp) {                                                               \
+    hipLaunchKernelGGL((k_deposit<TD, NT, TILES>), g, b, 0, s, srt, cm, tm, sc, rho, rho_plane, keep, sp);      \
   };
-  GNG_DEPOSIT(0, 256, false)
-  GNG_DEPOSIT(1, 512, false)
-  GNG_DEPOSIT(0, 256, true)
-  GNG_DEPOSIT(1, 512, true)
+  GNG_DEPOSIT(0, 256, 1)
+  GNG_DEPOSIT(1, 512, 1)
+  GNG_DEPOSIT(0, 256, 2)
+  GNG_DEPOSIT(1, 512, 2)
 #undef GNG_DEPOSIT
-  o.deposit_pairs[0] = [](dim3 g, dim3 b, hipStream_t s, const PartRec* srt, CellMap cm, TileMap tm,
-                          const SolveScalars* sc, long long n, float* rho, long long rho_plane, float* keep) {
-    hipLaunchKernelGGL((k_deposit_pairs<TD, 256>), g, b, 0, s, srt, cm, tm, sc, n, rho, rho_plane, keep);
-  };
-  o.deposit_pairs[1] = [](dim3 g, dim3 b, hipStream_t s, const PartRec* srt, CellMap cm, TileMap tm,
-                          const SolveScalars* sc, long long n, float* rho, long long rho_plane, float* keep) {
-    hipLaunchKernelGGL((k_deposit_pairs<TD, 512>), g, b, 0, s, srt, cm, tm, sc, n, rho, rho_plane, keep);
-  };
   o.cell_moments = [](dim3 g, dim3 b, hipStream_t s, const PartRec* srt, const unsigned* off, CellMap cm,
                       TileMap tm, const SolveScalars* sc, long long n, double* mom) {
     hipLaunchKernelGGL((k_cell_moments<TD>), g, b, 0, s, srt, off, cm, tm, sc, n, mom);
@@ -447,10 +449,10 @@ MeshOps make_ops() {
     hipLaunchKernelGGL((k_fft_x_inv<N, R, true>), g, b, 0, s, A, P, B, nullptr, tw, 0, 1.0f, codes);
   };
   o.deposit_box[0] = [](dim3 g, dim3 b, hipStream_t s, const BoxArgs* bx, TileMap tm) {
-    hipLaunchKernelGGL((k_deposit_tiles_box<TD, 256>), g, b, 0, s, bx, tm);
+    hipLaunchKernelGGL((k_deposit_box<TD, 256>), g, b, 0, s, bx, tm);
   };
   o.deposit_box[1] = [](dim3 g, dim3 b, hipStream_t s, const BoxArgs* bx, TileMap tm) {
-    hipLaunchKernelGGL((k_deposit_tiles_box<TD, 512>), g, b, 0, s, bx, tm);
+    hipLaunchKernelGGL((k_deposit_box<TD, 512>), g, b, 0, s, bx, tm);
   };
   o.x_fwd_box = [](dim3 g, dim3 b, hipStream_t s, const BoxArgs* bx, const float2* tw) {
     hipLaunchKernelGGL((k_fft_x_fwd_box<N, R>), g, b, 0, s, bx, tw);
@@ -530,11 +532,8 @@ struct gng_pm_plan {
   unsigned* d_tile_src = nullptr;    // Hilbert rank -> its 8 source tiles' first buckets
   unsigned* d_tile_ranges = nullptr; // Hilbert rank -> its flattened bucket ranges (per solve)
 
-  // split deposit of heavy tiles: per tile rank its slice count, their
-  // exclusive scan, its scratch slot; per workgroup its tile rank; the
-  // scratch tiles and finished-slice counters (zero between solves)
-  unsigned* d_slices = nullptr;
-  unsigned* d_slot = nullptr;
+  // split deposit of heavy tiles: per slice workgroup its tile rank and slice,
+  // the scratch tiles and finished-slice counters (zero between solves)
   unsigned* d_extra = nullptr;
   unsigned long long* d_split_scratch = nullptr;
   unsigned* d_split_done = nullptr;
@@ -615,10 +614,8 @@ struct StreamOrder {
 };
 
 void free_work(gng_pm_plan* p) {
-  for (void* q : {(void*)p->d_slices, (void*)p->d_slot, (void*)p->d_extra, (void*)p->d_split_scratch,
-                  (void*)p->d_split_done})
-    (void)hipFree(q);
-  p->d_slices = p->d_slot = p->d_extra = p->d_split_done = nullptr;
+  for (void* q : {(void*)p->d_extra, (void*)p->d_split_scratch, (void*)p->d_split_done}) (void)hipFree(q);
+  p->d_extra = p->d_split_done = nullptr;
   p->d_split_scratch = nullptr;
   p->split_slots = 0;
   (void)hipFree(p->d_sorted);
@@ -799,19 +796,15 @@ int ensure_work(gng_pm_plan* p, long long n) {
   GNG_HIP(hipMalloc(&p->d_perm, sizeof(unsigned) * m));
   GNG_HIP(hipMalloc(&p->d_bucket, sizeof(unsigned) * m));
   GNG_HIP(hipMalloc(&p->d_rank, sizeof(unsigned) * m));
-  // split deposit: extra workgroups (and scratch tiles) for at most 2 n /
-  // kSliceItems slices beyond one per tile
-  const long long ntiles = p->nb / 8;
-  const long long slots = 2 * n / (long long)kSliceItems + 16;
-  const size_t t3 = (size_t)p->tm.T * p->tm.T * p->tm.T;
-  GNG_HIP(hipMalloc(&p->d_slices, sizeof(unsigned) * (size_t)ntiles));
-  GNG_HIP(hipMalloc(&p->d_slot, sizeof(unsigned) * (size_t)ntiles));
+  // split deposit: slice workgroups, and half as many scratch tiles
+  const long long slots = deposit_slots(n, slice_items(n));
+  const size_t t3 = (size_t)p->tm.T * p->tm.T * p->tm.T, tiles = (size_t)slots / 2;
   GNG_HIP(hipMalloc(&p->d_extra, sizeof(unsigned) * (size_t)slots));
-  GNG_HIP(hipMalloc(&p->d_split_scratch, sizeof(unsigned long long) * t3 * (size_t)slots));
-  GNG_HIP(hipMalloc(&p->d_split_done, sizeof(unsigned) * (size_t)slots));
+  GNG_HIP(hipMalloc(&p->d_split_scratch, sizeof(unsigned long long) * t3 * tiles));
+  GNG_HIP(hipMalloc(&p->d_split_done, sizeof(unsigned) * tiles));
   // the scratch tiles and counters start at zero; every solve leaves them so
-  GNG_HIP(hipMemset(p->d_split_scratch, 0, sizeof(unsigned long long) * t3 * (size_t)slots));
-  GNG_HIP(hipMemset(p->d_split_done, 0, sizeof(unsigned) * (size_t)slots));
+  GNG_HIP(hipMemset(p->d_split_scratch, 0, sizeof(unsigned long long) * t3 * tiles));
+  GNG_HIP(hipMemset(p->d_split_done, 0, sizeof(unsigned) * tiles));
   p->split_slots = slots;
   p->work_cap = n;
   return GNG_OK;
@@ -857,34 +850,19 @@ int run_front(gng_pm_plan* p, const PartIn& in, long long n, hipStream_t s) {
   run_sort(p, in, n, p->tune.interp_sorted ? p->d_perm : nullptr, true, s);
   mark(p, 2, s);
   const unsigned ntiles = (unsigned)p->tm.nt * p->tm.nt * p->tm.nt;
-  hipLaunchKernelGGL(k_tile_ranges, dim3((ntiles + 255) / 256), dim3(256), 0, s, p->d_offset, p->tm, p->d_sc);
   DepositSplit sp{};
-  unsigned deposit_groups = ntiles;
   if (p->split_slots > 0 && p->tune.deposit_split) {
-    // heavy tiles over several workgroups: slices per tile, and the table of
-    // the extra workgroups past the ntiles primary ones
-    hipLaunchKernelGGL(k_deposit_plan, dim3((ntiles + 255) / 256), dim3(256), 0, s, p->d_offset, p->tm, p->d_slices,
-                       p->d_slot, p->d_extra, p->d_sc, (unsigned)p->split_slots);
-    sp.slices = p->d_slices;
-    sp.slot = p->d_slot;
+    sp.items = slice_items(n);
+    sp.slots = std::min<unsigned>((unsigned)p->split_slots, deposit_slots(n, sp.items));
     sp.extra = p->d_extra;
-    sp.sc = p->d_sc;
-    sp.ntiles = ntiles;
-    sp.slots = (unsigned)p->split_slots;
     sp.scratch = p->d_split_scratch;
     sp.done = p->d_split_done;
-    deposit_groups = ntiles + (unsigned)p->split_slots;
   }
-  if (!sp.slices && p->tune.deposit_pair) {
-    o.deposit_pairs[p->tune.deposit_wide](dim3((ntiles + 1u) / 2u), dim3(p->tune.deposit_wide ? 512 : 256), s,
-                                          p->d_sorted, cm, p->tm, p->d_sc, n, rho, rho_plane,
-                                          p->keep_density ? p->d_rho : nullptr);
-  } else {
-    o.deposit[p->tune.deposit_wide][sp.slices != nullptr](dim3(deposit_groups),
-                                                          dim3(p->tune.deposit_wide ? 512 : 256), s, p->d_sorted,
-                                                          p->d_offset, cm, p->tm, p->d_sc, n, rho, rho_plane,
-                                                          p->keep_density ? p->d_rho : nullptr, sp);
-  }
+  hipLaunchKernelGGL(k_tile_ranges, dim3((ntiles + 255) / 256), dim3(256), 0, s, p->d_offset, p->tm, p->d_sc, n, sp);
+  const int pair = p->tune.deposit_pair != 0;
+  o.deposit[p->tune.deposit_wide][pair](dim3(sp.slots + xcd_grid(pair ? (ntiles + 1u) / 2u : ntiles)),
+                                        dim3(p->tune.deposit_wide ? 512 : 256), s, p->d_sorted, cm, p->tm, p->d_sc,
+                                        rho, rho_plane, p->keep_density ? p->d_rho : nullptr, sp);
   mark(p, 3, s);
   const long long rows = (long long)nm * nm;
   const dim3 yz_grid((unsigned)(H / o.yz_cols), (unsigned)nm);
@@ -2266,6 +2244,7 @@ int upload_box_tables(gng_pm_batch* b, const std::vector<BoxGroup>& gs, const in
       a.sorted = p->d_sorted;
       a.bucket = p->d_bucket;
       a.rank = p->d_rank;
+      a.ranges = p->d_tile_ranges;
       a.p0 = offsets[i];
       a.n = offsets[i + 1] - offsets[i];
       h.push_back(a);
@@ -2293,21 +2272,21 @@ void launch_box_group(gng_pm_batch* b, const BoxGroup& gr, const BoxArgs* bx, lo
   const unsigned nbx = (unsigned)gr.boxes.size();
   const int nm = gr.nm, H = nm / 2;
   const PosSrc<float> src{x, y, z, 1};
-  hipLaunchKernelGGL(k_reset_scalars_box, dim3(1, 1, nbx), dim3(64), 0, s, bx);
   const long long n16 = (p0->nb + 3) / 4;
-  hipLaunchKernelGGL(k_zero_box, dim3((unsigned)((n16 + 255) / 256), 1, nbx), dim3(256), 0, s, bx, n16);
+  hipLaunchKernelGGL(k_sort_reset_box, dim3((unsigned)((n16 + 255) / 256), 1, nbx), dim3(256), 0, s, bx, n16);
   if (maxn > 0)
     hipLaunchKernelGGL(k_bucket_count_box,
                        dim3((unsigned)((maxn + 256 * kBucketPer - 1) / (256 * kBucketPer)), 1, nbx), dim3(256), 0,
                        s, bx, src, m, p0->tm);
   hipLaunchKernelGGL(k_scan_local_box, dim3((unsigned)p0->scan_blocks, 1, nbx), dim3(256), 0, s, bx, p0->nb);
-  hipLaunchKernelGGL(k_scan_partials_box, dim3(1, 1, nbx), dim3(256), 0, s, bx, p0->scan_blocks, p0->nb);
-  hipLaunchKernelGGL(k_scan_add_box, dim3((unsigned)p0->scan_blocks, 1, nbx), dim3(256), 0, s, bx, p0->nb);
+  hipLaunchKernelGGL(k_scan_add_prefix_box, dim3((unsigned)p0->scan_blocks, 1, nbx), dim3(256), 0, s, bx,
+                     p0->scan_blocks, p0->nb);
   if (maxn > 0)
     hipLaunchKernelGGL(k_scatter_box, dim3((unsigned)((maxn + 256 * kScatterPer - 1) / (256 * kScatterPer)), 1, nbx),
                        dim3(256), 0, s, bx, src, m);
   const unsigned ntiles = (unsigned)p0->tm.nt * p0->tm.nt * p0->tm.nt;
-  o.deposit_box[p0->tune.deposit_wide](dim3(ntiles, 1, nbx), dim3(p0->tune.deposit_wide ? 512 : 256), s, bx,
+  hipLaunchKernelGGL(k_tile_ranges_box, dim3((ntiles + 255) / 256, 1, nbx), dim3(256), 0, s, bx, p0->tm);
+  o.deposit_box[p0->tune.deposit_wide](dim3(xcd_grid(ntiles), 1, nbx), dim3(p0->tune.deposit_wide ? 512 : 256), s, bx,
                                        p0->tm);
   const long long rows = (long long)nm * nm;
   o.x_fwd_box(dim3((unsigned)(rows / o.x_rows), 1, nbx), dim3(256), s, bx, p0->d_tw);

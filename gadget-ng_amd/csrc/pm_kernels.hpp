@@ -170,8 +170,9 @@ constexpr int kQStride = 16;  // 64-bit words between slots
 struct SolveScalars {
   unsigned int mmax_bits;  // max |m| as float bits (non-negative floats order as integers)
   unsigned int split_budget;  // scratch tiles reserved by split deposit tiles
-  unsigned long long qtot;    // sum of the qsum slots, once the scatter is done (k_tile_ranges)
-  unsigned int pad[60];
+  long long qmean;            // integer part of the mean fixed-point mass per cell (k_tile_ranges)
+  int shift;                  // fixed_shift, once the scatter is done (k_tile_ranges)
+  unsigned int pad[59];
   unsigned long long qsum[kQSlots * kQStride];
 };
 
@@ -211,6 +212,7 @@ struct BoxArgs {
   PartRec* sorted;
   unsigned* bucket;
   unsigned* rank;
+  unsigned* ranges;
   long long n;
   long long p0;
 };
@@ -221,15 +223,6 @@ __device__ __forceinline__ void reset_scalars_body(SolveScalars* sc) {
     sc->split_budget = 0u;
   }
   if (threadIdx.x < kQSlots) sc->qsum[threadIdx.x * kQStride] = 0ull;
-}
-
-__global__ void k_reset_scalars(SolveScalars* sc) {
-  reset_scalars_body(sc);
-}
-
-__global__ void k_reset_scalars_box(const BoxArgs* __restrict__ bx) {
-  const BoxArgs& b = bx[blockIdx.z];
-  reset_scalars_body(b.sc);
 }
 
 // ---------------------------------------------------------------------------

@@ -214,7 +214,8 @@ int gng_pm_force_meshes(gng_pm_plan *p, float *out);
  * applies to this plan and to plans created later in the process with the
  * same device architecture and mesh side; with GNG_PM_TUNE_FILE set it is also
  * read from and written to that file.  Untuned plans use the persistent z pass
- * at nm = 512 only and the 512-thread deposit.  No reference counterpart.
+ * at nm = 512 only, the 512-thread deposit only below 256 tiles, and two
+ * tiles per deposit workgroup from nm = 1024 on.  No reference counterpart.
  * Synchronous; the density and potential of earlier solves are invalidated. */
 typedef struct gng_pm_tuning_t {
   int32_t z_persistent;      /* z + Green pass: persistent workgroups          */
@@ -241,9 +242,10 @@ typedef struct gng_pm_tuning_t {
                                 64 at 1024^3; inv: 64 MiB, 64 at 512^3 and 16
                                 at 1024^3, where the default is 0); none at
                                 256^3 and below */
-  int32_t deposit_split;     /* deposit: tiles holding more than 32768 particles
-                                (dense clumps) are shared by several workgroups
-                                (1, default) or each run by one (0).  Same
+  int32_t deposit_split;     /* deposit: tiles holding more than 8192 to 32768 particles
+                                (growing with n; dense clumps) are shared by
+                                several workgroups (1, default) or each run by
+                                one (0).  Same
                                 density bit for bit either way */
   int32_t y_inv_narrow;      /* inverse y pass on 8-column tiles of 512 threads
                                 (1, default) instead of 16 columns of 1024, where
@@ -251,9 +253,9 @@ typedef struct gng_pm_tuning_t {
                                 the three live fields leave a 1024-thread
                                 workgroup alone on its CU.  Same values either
                                 way */
-  int32_t deposit_pair;      /* deposit without split tiles: two tiles per
-                                workgroup (1), whose records load while the
-                                other tile is written, or one (0, default).
+  int32_t deposit_pair;      /* deposit: two tiles per workgroup (1, default from
+                                nm = 1024), whose records load while the other
+                                tile is written, or one (0).
                                 Same density bit for bit either way */
 } gng_pm_tuning_t;
 

@@ -1,6 +1,6 @@
 """CPU emulation of the GPU deposit's tile/class scheme (no GPU needed).
 
-k_deposit_tiles (gadget-ng_amd/csrc/deposit.hpp) gives each tile of T^3
+k_deposit (gadget-ng_amd/csrc/deposit.hpp) gives each tile of T^3
 cells to one workgroup.  A particle's base cell fixes its tile and a 3-bit
 class (bit a set when the base cell is on the tile's last layer along axis
 a); tile u reads its own particles and, from each lower neighbour u - d, the
