@@ -52,7 +52,7 @@ constexpr int HX = TX + 2, HY = TY + 2, HZ = TZ + 2, HC = HX * HY * HZ;
 // weight-gradient tile: 16 x 4 x 4 cells
 constexpr int WX = 16, WY = 4, WZ = 4;
 constexpr int WHX = WX + 2, WHY = WY + 2, WHZ = WZ + 2, WHC = WHX * WHY * WHZ;
-constexpr int kWgradBlocks = 512;
+constexpr int kWgradBlocks = 512;  // twice that for 8 input channels: half the columns, half the LDS
 
 // parameter layout (floats)
 constexpr int kIn = 8;  // input channels (6 used)
@@ -298,34 +298,57 @@ __global__ __launch_bounds__(kConvThreads, 4) void k_conv(const unsigned short* 
   }
 }
 
+// 8 cells x 8 channels of bf16, transposed: v[i] holds the channels of cell i,
+// row[c] receives channel c of cells 0..7.
+__device__ __forceinline__ u32x4 channel_row(const u32x4* v, int c) {
+  const unsigned sel = (c & 1) ? 0x07060302u : 0x05040100u;
+  u32x4 r;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) r[j] = __builtin_amdgcn_perm(v[2 * j + 1][c >> 1], v[2 * j][c >> 1], sel);
+  return r;
+}
+
 // Weight gradient partials.  Columns n = t*CIN + c (27*CIN of them) plus a
 // bias column of ones; rows o = output channel (< COS).  Each workgroup walks
-// tiles in a grid-stride loop and writes its D[o][n] partial sums:
+// 16x4x4-cell tiles in a grid-stride loop and writes its D[o][n] partial sums:
 //   partial[block][n / 16][o * 16 + n % 16].
+//
+// K runs over cells, so both operands are wanted channel by channel along x,
+// while the meshes are channels-last.  The staging transposes 8 cells x 8
+// channels at a time in registers (byte permutes) and keeps X three times,
+// once per x tap, so that every fragment of 8 consecutive cells of one
+// (tap, channel) is one aligned 16-byte LDS word: one ds_read_b128 per MFMA of
+// 16 outputs x 16 columns x 32 cells (two x rows).  Planes are padded to an
+// odd number of 16-byte words, so the 16 lanes of different channels hit
+// different banks.  8 boxes of 64^3, the three layers: 833 us with
+// single-element LDS reads and K = 16 products, 181 us so.
 template <int CIN, int COS>
 __global__ __launch_bounds__(256) void k_conv_wgrad(const unsigned short* __restrict__ X,
                                                     const unsigned short* __restrict__ dZ,
                                                     float* __restrict__ partial, int nm, int boxes) {
   constexpr int NCOL = 27 * CIN + 1, NB = (NCOL + 15) / 16, SPW = (NB + 3) / 4;
-  __shared__ __attribute__((aligned(16))) unsigned short xt[WHC * CIN];
-  __shared__ __attribute__((aligned(16))) unsigned short dt[WX * WY * WZ * COS];
+  constexpr int XROWS = WHY * WHZ, XPL = XROWS * WX + 8, ZROWS = WY * WZ, ZPL = ZROWS * WX + 8;  // 16-bit words
+  __shared__ __attribute__((aligned(16))) unsigned short xt[3 * CIN * XPL];
+  __shared__ __attribute__((aligned(16))) unsigned short dt[COS * ZPL];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m = lane & 15, g = lane >> 4;
 
-  int coff[SPW], cch[SPW], ckind[SPW];  // kind 0: tap column, 1: ones, 2: zero
+  // the lane's column of each of the wave's blocks: its word offset in xt for
+  // row pair 0, and the last block's kind (0: tap column, 1: ones, 2: zero)
+  int xoff[SPW], ckind = 0;
 #pragma unroll
   for (int q = 0; q < SPW; ++q) {
     const int n = 16 * (wave + 4 * q) + m;
-    coff[q] = 0;
-    cch[q] = 0;
+    xoff[q] = 0;
+    ckind = n == 27 * CIN ? 1 : 2;
     if (n < 27 * CIN) {
-      coff[q] = tap_off(n / CIN, WHX, WHY);
-      cch[q] = n % CIN;
-      ckind[q] = 0;
-    } else {
-      ckind[q] = n == 27 * CIN ? 1 : 2;
+      const int t = n / CIN, c = n % CIN;
+      xoff[q] = ((t % 3) * CIN + c) * XPL + ((t / 9) * WHY + (t / 3) % 3 + (g >> 1)) * WX + (g & 1) * 8;
+      ckind = 0;
     }
   }
+  static_assert(16 * 4 * (SPW - 1) <= 27 * CIN, "only the last block of a wave may leave the tap columns");
+  const int zoff = (m < COS ? m : 0) * ZPL + (g >> 1) * WX + (g & 1) * 8;
   f32x4 acc[SPW];
 #pragma unroll
   for (int q = 0; q < SPW; ++q) acc[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -334,51 +357,85 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(const unsigned short* __rest
   const long long per_box = (long long)ntx * nty * ntz;
   const long long tiles = per_box * boxes;
   const long long M = (long long)nm * nm * nm;
-  for (long long tt = blockIdx.x; tt < tiles; tt += gridDim.x) {
+  // Staging items.  X: one thread per (halo row, channel octet, half row): 10
+  // cells in, 8 channels of each of the three x shifts out.  dZ, on the last
+  // wavefront: one thread per (row, channel octet, half row).
+  constexpr int OCT = CIN / 8, XI = XROWS * OCT * 2;
+  static_assert(CIN % 8 == 0 && XI <= 192, "the X items leave the last wavefront to dZ");
+  constexpr int ZOCT = COS == 16 ? 2 : 1, ZI = ZROWS * ZOCT * 2, ZC = COS == 16 ? 8 : 4;
+  static_assert(ZI <= 64 && (COS == 16 || COS == 4), "dZ items fill at most one wavefront");
+  using ZW = typename std::conditional<COS == 16, u32x4, u32x2>::type;
+  const bool is_x = threadIdx.x < XI, is_z = threadIdx.x >= 192 && threadIdx.x < 192 + ZI;
+  const int item = is_x ? (int)threadIdx.x : (int)threadIdx.x - 192;
+  const int grp = item & 1, oct = (item >> 1) % (is_x ? OCT : ZOCT), row = (item >> 1) / (is_x ? OCT : ZOCT);
+  u32x4 v[10];
+  // the next tile's words load while the current tile's products run
+  auto load = [&](long long tt) {
     const long long box = tt / per_box;
     const long long rem = tt - box * per_box;
-    const int bx = (int)(rem % ntx), by = (int)((rem / ntx) % nty), bz = (int)(rem / ((long long)ntx * nty));
-    const int x0 = bx * WX, y0 = by * WY, z0 = bz * WZ;
-    __syncthreads();
-    load_halo<CIN, WHX, WHY, WHZ, 256>(xt, X + box * M * CIN, x0, y0, z0, nm);
-    {
-      constexpr int WPC = COS / 2, NW = WX * WY * WZ * WPC, PER = NW / 256;
-      static_assert(NW % 256 == 0, "gradient tile words must fill the workgroup");
-      const unsigned* src = reinterpret_cast<const unsigned*>(dZ + box * M * COS);
-      unsigned* dst = reinterpret_cast<unsigned*>(dt);
-      unsigned v[PER];
+    const int x0 = (int)(rem % ntx) * WX, y0 = (int)((rem / ntx) % nty) * WY, z0 = (int)(rem / ((long long)ntx * nty)) * WZ;
+    if (is_x) {
+      int gy = y0 + row % WHY - 1, gz = z0 + row / WHY - 1;
+      gy += gy < 0 ? nm : 0;
+      gy -= gy >= nm ? nm : 0;
+      gz += gz < 0 ? nm : 0;
+      gz -= gz >= nm ? nm : 0;
+      const u32x4* src = reinterpret_cast<const u32x4*>(X + (box * M + ((long long)gz * nm + gy) * nm) * CIN) + oct;
 #pragma unroll
-      for (int k = 0; k < PER; ++k) {
-        const int e = (int)threadIdx.x + k * 256;
-        const int c = e / WPC, w = e - c * WPC;
-        const int cx = c % WX, cy = (c / WX) % WY, cz = c / (WX * WY);
-        const long long gc = ((long long)(z0 + cz) * nm + (y0 + cy)) * nm + x0 + cx;
-        v[k] = src[gc * WPC + w];
+      for (int i = 0; i < 10; ++i) {
+        int gx = x0 + 8 * grp + i - 1;
+        gx += gx < 0 ? nm : 0;
+        gx -= gx >= nm ? nm : 0;
+        v[i] = src[gx * OCT];
       }
+    } else if (is_z) {
+      const long long c0 = box * M + ((long long)(z0 + row / WY) * nm + (y0 + row % WY)) * nm + x0 + 8 * grp;
+      const ZW* src = reinterpret_cast<const ZW*>(dZ + c0 * COS) + oct;
 #pragma unroll
-      for (int k = 0; k < PER; ++k) dst[threadIdx.x + k * 256] = v[k];
+      for (int i = 0; i < 8; ++i) {
+        const ZW z = src[i * ZOCT];
+        v[i].x = z.x;
+        v[i].y = z.y;
+        if constexpr (COS == 16) {
+          v[i].z = z.z;
+          v[i].w = z.w;
+        }
+      }
+    }
+  };
+  if (blockIdx.x < tiles) load(blockIdx.x);
+  for (long long tt = blockIdx.x; tt < tiles; tt += gridDim.x) {
+    __syncthreads();
+    if (is_x) {
+#pragma unroll
+      for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+          *reinterpret_cast<u32x4*>(xt + (dx * CIN + 8 * oct + c) * XPL + row * WX + 8 * grp) = channel_row(v + dx, c);
+    } else if (is_z) {
+#pragma unroll
+      for (int c = 0; c < ZC; ++c)
+        *reinterpret_cast<u32x4*>(dt + (8 * oct + c) * ZPL + row * WX + 8 * grp) = channel_row(v, c);
     }
     __syncthreads();
-#pragma unroll 1
-    for (int r = 0; r < WY * WZ; ++r) {
-      const int ry = r % WY, rz = r / WY;
-      bf16x4 av;
+    if (tt + gridDim.x < tiles) load(tt + gridDim.x);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) av[j] = m < COS ? (short)dt[((rz * WY + ry) * WX + 4 * g + j) * COS + m] : (short)0;
-      const int hb = ((rz + 1) * WHY + (ry + 1)) * WHX + 1 + 4 * g;
+    for (int s = 0; s < WY * WZ / 2; ++s) {
+      // rows 2s and 2s + 1 of the tile (g >> 1 picks one)
+      u32x4 aw = *reinterpret_cast<const u32x4*>(dt + zoff + 2 * s * WX);
+      if (COS < 16 && m >= COS) aw = u32x4{0u, 0u, 0u, 0u};
+      const bf16x8 av = __builtin_bit_cast(bf16x8, aw);
+      constexpr int PAIRS = WY / 2;
+      const int hrow = (s / PAIRS) * WHY + 2 * (s % PAIRS);
 #pragma unroll
       for (int q = 0; q < SPW; ++q) {
-        if (wave + 4 * q < NB) {
-          bf16x4 bv;
+        // no branch per product: blocks past the last are computed as zeros
+        u32x4 bw = *reinterpret_cast<const u32x4*>(xt + xoff[q] + hrow * WX);
+        if (q == SPW - 1) {  // the last blocks hold the ones column and zeros
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            short v = 0;
-            if (ckind[q] == 0) v = (short)xt[(hb + j + coff[q]) * CIN + cch[q]];
-            else if (ckind[q] == 1) v = (short)0x3F80;
-            bv[j] = v;
-          }
-          acc[q] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc[q], 0, 0, 0);
+          for (int k = 0; k < 4; ++k) bw[k] = ckind == 0 ? bw[k] : ckind == 1 ? 0x3F803F80u : 0u;
         }
+        acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, __builtin_bit_cast(bf16x8, bw), acc[q], 0, 0, 0);
       }
     }
   }
@@ -393,18 +450,28 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(const unsigned short* __rest
   }
 }
 
-// dW[t][c][o] (t*CIN + c = column) and db[o] from the partials, summed over
-// workgroups in order in FP64.
+// dW[t][c][o] (t*CIN + c = column) and db[o] from the partials, in FP64 in a
+// fixed order.  Workgroup (s, r) takes 64 of the 256 values of column block s;
+// 16 groups of 64 threads each add every 16th workgroup's partial (loads of
+// 256 bytes, several in flight), then the 16 sums are added in order.  One
+// thread per value and 512 dependent loads took 130 us a layer, this 6.
 template <int CIN, int COUT>
-__global__ void k_wgrad_reduce(const float* __restrict__ partial, int nblocks, float* __restrict__ gw,
-                               float* __restrict__ gb) {
+__global__ __launch_bounds__(1024) void k_wgrad_reduce(const float* __restrict__ partial, int nblocks,
+                                                       float* __restrict__ gw, float* __restrict__ gb) {
   constexpr int NCOL = 27 * CIN + 1, NB = (NCOL + 15) / 16;
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= NCOL * COUT) return;
-  const int col = e / COUT, o = e % COUT;
-  const int s = col / 16, nn = col % 16;
+  __shared__ double red[16][64];
+  const int i = threadIdx.x & 63, grp = threadIdx.x >> 6;
+  const int s = blockIdx.x, e = blockIdx.y * 64 + i;
   double sum = 0.0;
-  for (int b = 0; b < nblocks; ++b) sum += partial[((long long)b * NB + s) * 256 + o * 16 + nn];
+#pragma unroll 8
+  for (int b = grp; b < nblocks; b += 16) sum += partial[((long long)b * NB + s) * 256 + e];
+  red[grp][i] = sum;
+  __syncthreads();
+  if (grp != 0) return;
+#pragma unroll
+  for (int k = 1; k < 16; ++k) sum += red[k][i];
+  const int o = e >> 4, col = 16 * s + (e & 15);
+  if (o >= COUT || col >= NCOL) return;
   if (col < 27 * CIN) gw[col * COUT + o] = (float)sum;
   else gb[o] = (float)sum;
 }
@@ -413,35 +480,49 @@ __global__ void k_wgrad_reduce(const float* __restrict__ partial, int nblocks, f
 // (cin x cout real channels, cin_pad channels in the k layout).  With
 // mirror != 0 the fragments are those of the data-gradient convolution:
 // B[k = t*cin_pad + o][n = c] = w[26 - t][c][o].
-__global__ void k_pack(const float* __restrict__ w, int cin, int cout, int cin_pad, int ksteps, int mirror,
-                       u32x4* __restrict__ frag) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= ksteps * 64) return;
-  const int s = e / 64, l = e % 64, g = l / 16, n = l % 16;
+struct PackJob {
+  const float* w;
+  int cin, cout, cin_pad, ksteps, mirror;
+  u32x4* frag;
+};
+// Every fragment set and the padded biases in one launch: block b of 64
+// threads is k-step b of the jobs laid end to end, the last block the biases.
+constexpr int kPackJobs = 5;
+struct PackAll {
+  PackJob job[kPackJobs];
+  const float* bias[3];
+  int nbias[3];
+  float* b16;
+};
+__global__ __launch_bounds__(64) void k_pack(const PackAll all) {
+  int s = blockIdx.x, j = 0;
+  while (j < kPackJobs && s >= all.job[j].ksteps) s -= all.job[j++].ksteps;
+  if (j == kPackJobs) {
+    const int k = threadIdx.x >> 4, n = threadIdx.x & 15;
+    if (k < 3) all.b16[16 * k + n] = n < all.nbias[k] ? all.bias[k][n] : 0.0f;
+    return;
+  }
+  const PackJob& pj = all.job[j];
+  const int l = threadIdx.x, g = l / 16, n = l % 16;
   unsigned short v[8];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const int k = 32 * s + 8 * g + j;
-    const int t = k / cin_pad, c = k % cin_pad;
+  for (int q = 0; q < 8; ++q) {
+    const int k = 32 * s + 8 * g + q;
+    const int t = k / pj.cin_pad, c = k % pj.cin_pad;
     float x = 0.0f;
-    if (!mirror) {
-      if (t < 27 && c < cin && n < cout) x = w[(t * cin + c) * cout + n];
+    if (!pj.mirror) {
+      if (t < 27 && c < pj.cin && n < pj.cout) x = pj.w[(t * pj.cin + c) * pj.cout + n];
     } else {
       // data gradient: input channels are the forward outputs (c < cout),
       // outputs the forward inputs (n < cin)
-      if (t < 27 && c < cout && n < cin) x = w[((26 - t) * cin + n) * cout + c];
+      if (t < 27 && c < pj.cout && n < pj.cin) x = pj.w[((26 - t) * pj.cin + n) * pj.cout + c];
     }
-    v[j] = f2bf(x);
+    v[q] = f2bf(x);
   }
   u32x4 o;
 #pragma unroll
   for (int q = 0; q < 4; ++q) o[q] = (unsigned)v[2 * q] | ((unsigned)v[2 * q + 1] << 16);
-  frag[e] = o;
-}
-
-__global__ void k_bias16(const float* __restrict__ b, int cout, float* __restrict__ b16) {
-  const int n = threadIdx.x;
-  if (n < 16) b16[n] = n < cout ? b[n] : 0.0f;
+  pj.frag[s * 64 + l] = o;
 }
 
 __global__ void k_adam(float* __restrict__ p, const float* __restrict__ gr, float* __restrict__ m1,
@@ -456,17 +537,22 @@ __global__ void k_adam(float* __restrict__ p, const float* __restrict__ gr, floa
   p[i] -= lr * (a * c1) / (sqrtf(v * c2) + eps);
 }
 
-__global__ void k_fill(float* __restrict__ p, long long n, float v) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
+// The loss gradient mesh (n4 16-byte words) and the loss sum cleared.
+__global__ __launch_bounds__(256) void k_loss_reset(float4* __restrict__ gy, long long n4, double* __restrict__ loss) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i < n4) gy[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  if (i == 0) *loss = 0.0;
 }
 
-__global__ void k_fill_d(double* p) { *p = 0.0; }
-
 // dz3 = bf16(dL/dy), 4 channels per cell
-__global__ void k_to_bf16(const float* __restrict__ a, unsigned short* __restrict__ b, long long n) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) b[i] = f2bf(a[i]);
+__global__ __launch_bounds__(256) void k_to_bf16(const float4* __restrict__ a, u32x2* __restrict__ b, long long n4) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n4) return;
+  const float4 v = a[i];
+  u32x2 o;
+  o.x = pack_bf16(v.x, v.y);
+  o.y = pack_bf16(v.z, v.w);
+  b[i] = o;
 }
 
 // Periodic 7-point running mean along one axis (stride 1, nm or nm^2).
@@ -616,14 +702,26 @@ __device__ __forceinline__ void cic_nodes(float x, float y, float z, float cs, i
   }
 }
 
-// Loss and dL/dy.  Lanes whose particles share a base cell (training sets are
-// stored cell-sorted) form runs; a segmented suffix sum over each run leaves
-// the run total in its first lane, which alone issues the atomics.
+// Loss and dL/dy.  The mesh adds are what bounds this kernel: device-wide
+// float atomics run at some 60 G/s here, and 24 of them per particle took
+// 0.68 ms for 2^21 particles, one per cell (0.26 ms now).  A workgroup therefore first sums
+// its 256 particles' contributions by node in an LDS table (open addressing;
+// a node that finds no slot in kLossProbes tries goes to the mesh directly, as
+// most do when the records are in no spatial order) and adds each node once:
+// cell-sorted records, as training sets are stored, share most of their nodes.
+constexpr int kLossSlots = 2048, kLossProbes = 8;
 __global__ __launch_bounds__(256) void k_loss(const float4* __restrict__ pos, const float4* __restrict__ tgt,
                                               long long n, const float4* __restrict__ y, float* __restrict__ gy,
                                               double* __restrict__ loss, int nm, float cs, float out_scale,
                                               float gscale, int max_boxes) {
+  constexpr unsigned kEmpty = 0xFFFFFFFFu;  // cells number below 2^32 - 1: a cell takes over 300 bytes
+  __shared__ unsigned key[kLossSlots];
+  __shared__ float4 sum[kLossSlots];
   __shared__ double red[4];
+  for (int i = threadIdx.x; i < kLossSlots; i += 256) {
+    key[i] = kEmpty;
+    sum[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  }
   const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   const int lane = threadIdx.x & 63;
   const long long M = (long long)nm * nm * nm;
@@ -634,7 +732,6 @@ __global__ __launch_bounds__(256) void k_loss(const float4* __restrict__ pos, co
   Cic c;
   float gx = 0.0f, gyv = 0.0f, gz = 0.0f;
   double lp = 0.0;
-  long long key = -1 - lane;
   if (live) {
     const float4 t = tgt[p];
     cic_nodes(q.x, q.y, q.z, cs, nm, (long long)(int)q.w * M, c);
@@ -651,43 +748,33 @@ __global__ __launch_bounds__(256) void k_loss(const float4* __restrict__ pos, co
     gx = gscale * t.w * ex;
     gyv = gscale * t.w * ey;
     gz = gscale * t.w * ez;
-    key = c.node[0];
-  } else {
+  }
+  __syncthreads();
+  // a particle of weight 0 adds nothing (its error times 0 is 0 unless it is
+  // not finite, and then it does add)
+  if (live && !(gx == 0.0f && gyv == 0.0f && gz == 0.0f)) {
 #pragma unroll
     for (int a = 0; a < 8; ++a) {
-      c.node[a] = 0;
-      c.w[a] = 0.0f;
-    }
-  }
-  // run boundaries
-  const long long kprev = __shfl_up(key, 1);
-  const bool head = lane == 0 || kprev != key;
-  const unsigned long long heads = __ballot(head);
-  const unsigned long long above = lane == 63 ? 0ull : (heads >> (lane + 1)) << (lane + 1);
-  const int run_end = above ? __ffsll((long long)above) - 2 : 63;
-  float v[24];
-#pragma unroll
-  for (int a = 0; a < 8; ++a) {
-    v[3 * a] = c.w[a] * gx;
-    v[3 * a + 1] = c.w[a] * gyv;
-    v[3 * a + 2] = c.w[a] * gz;
-  }
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const bool take = lane + off <= run_end;
-#pragma unroll
-    for (int e = 0; e < 24; ++e) {
-      const float o = __shfl_down(v[e], off);
-      if (take) v[e] += o;
-    }
-  }
-  if (live && head) {
-#pragma unroll
-    for (int a = 0; a < 8; ++a) {
-      float* dst = gy + c.node[a] * 4;
-      atomicAdd(dst, v[3 * a]);
-      atomicAdd(dst + 1, v[3 * a + 1]);
-      atomicAdd(dst + 2, v[3 * a + 2]);
+      const unsigned node = (unsigned)c.node[a];
+      const float vx = c.w[a] * gx, vy = c.w[a] * gyv, vz = c.w[a] * gz;
+      // neighbours along x in neighbouring slots, other rows elsewhere
+      unsigned h = (node + (node >> 11) * 977u) & (kLossSlots - 1);
+      int tries = 0;
+      for (; tries < kLossProbes; ++tries) {
+        const unsigned prev = atomicCAS(&key[h], kEmpty, node);
+        if (prev == kEmpty || prev == node) break;
+        h = (h + 64u) & (kLossSlots - 1);
+      }
+      if (tries < kLossProbes) {
+        atomicAdd(&sum[h].x, vx);
+        atomicAdd(&sum[h].y, vy);
+        atomicAdd(&sum[h].z, vz);
+      } else {
+        float* dst = gy + c.node[a] * 4;
+        atomicAdd(dst, vx);
+        atomicAdd(dst + 1, vy);
+        atomicAdd(dst + 2, vz);
+      }
     }
   }
   // loss: wave then block reduction, one FP64 atomic per block
@@ -695,6 +782,13 @@ __global__ __launch_bounds__(256) void k_loss(const float4* __restrict__ pos, co
   for (int off = 32; off > 0; off >>= 1) lp += __shfl_down(lp, off);
   if (lane == 0) red[threadIdx.x >> 6] = lp;
   __syncthreads();
+  // neighbouring lanes add neighbouring components and nodes, so a wavefront's
+  // adds fall into few cache lines
+  const float* flat = reinterpret_cast<const float*>(sum);
+  for (int i = threadIdx.x; i < 4 * kLossSlots; i += 256) {
+    const unsigned node = key[i >> 2];
+    if (node != kEmpty && (i & 3) != 3) atomicAdd(gy + (size_t)node * 4 + (i & 3), flat[i]);
+  }
   if (threadIdx.x == 0) atomicAdd(loss, red[0] + red[1] + red[2] + red[3]);
 }
 
@@ -801,14 +895,15 @@ BufInfo buffer(const gng_net* t, int which) {
 int repack(gng_net* t, hipStream_t s) {
   const float* p = t->d_params;
   constexpr int K1 = KSteps<kIn>::v, K4 = KSteps<4>::v, K16 = KSteps<16>::v;
-  hipLaunchKernelGGL(k_pack, dim3(K1), dim3(64), 0, s, p + P_W1, kIn, 16, kIn, K1, 0, t->d_f1);
-  hipLaunchKernelGGL(k_pack, dim3(K16), dim3(64), 0, s, p + P_W2, 16, 16, 16, K16, 0, t->d_f2);
-  hipLaunchKernelGGL(k_pack, dim3(K16), dim3(64), 0, s, p + P_W3, 16, 3, 16, K16, 0, t->d_f3);
-  hipLaunchKernelGGL(k_pack, dim3(K4), dim3(64), 0, s, p + P_W3, 16, 3, 4, K4, 1, t->d_g3);
-  hipLaunchKernelGGL(k_pack, dim3(K16), dim3(64), 0, s, p + P_W2, 16, 16, 16, K16, 1, t->d_g2);
-  hipLaunchKernelGGL(k_bias16, dim3(1), dim3(64), 0, s, p + P_B1, 16, t->d_b16);
-  hipLaunchKernelGGL(k_bias16, dim3(1), dim3(64), 0, s, p + P_B2, 16, t->d_b16 + 16);
-  hipLaunchKernelGGL(k_bias16, dim3(1), dim3(64), 0, s, p + P_B3, 3, t->d_b16 + 32);
+  PackAll all{{{p + P_W1, kIn, 16, kIn, K1, 0, t->d_f1},
+               {p + P_W2, 16, 16, 16, K16, 0, t->d_f2},
+               {p + P_W3, 16, 3, 16, K16, 0, t->d_f3},
+               {p + P_W3, 16, 3, 4, K4, 1, t->d_g3},
+               {p + P_W2, 16, 16, 16, K16, 1, t->d_g2}},
+              {p + P_B1, p + P_B2, p + P_B3},
+              {16, 16, 3},
+              t->d_b16};
+  hipLaunchKernelGGL(k_pack, dim3(K1 + 3 * K16 + K4 + 1), dim3(64), 0, s, all);
   GNG_HIP(hipGetLastError());
   return GNG_OK;
 }
@@ -1074,16 +1169,16 @@ int gng_net_loss_grad(gng_net* net, const float* d_pos4, const float* d_tgt4, in
   GNG_HIP(hipSetDevice(net->device));
   hipStream_t s = as_stream(stream);
   const long long cells = net->M * net->max_boxes;
-  hipLaunchKernelGGL(k_fill, dim3((unsigned)((cells * 4 + 255) / 256)), dim3(256), 0, s, net->d_gy, cells * 4, 0.0f);
-  hipLaunchKernelGGL(k_fill_d, dim3(1), dim3(1), 0, s, net->d_loss);
+  const dim3 gc((unsigned)((cells + 255) / 256));
+  hipLaunchKernelGGL(k_loss_reset, gc, dim3(256), 0, s, reinterpret_cast<float4*>(net->d_gy), cells, net->d_loss);
   const float cs = (float)((double)net->nm / box_size);
   const float gscale = (float)(2.0 * out_scale / (double)n);
   hipLaunchKernelGGL(k_loss, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
                      reinterpret_cast<const float4*>(d_pos4), reinterpret_cast<const float4*>(d_tgt4), (long long)n,
                      reinterpret_cast<const float4*>(net->d_y), net->d_gy, net->d_loss, net->nm, cs, out_scale, gscale,
                      net->max_boxes);
-  hipLaunchKernelGGL(k_to_bf16, dim3((unsigned)((cells * 4 + 255) / 256)), dim3(256), 0, s, net->d_gy, net->d_dz3,
-                     cells * 4);
+  hipLaunchKernelGGL(k_to_bf16, gc, dim3(256), 0, s, reinterpret_cast<const float4*>(net->d_gy),
+                     reinterpret_cast<u32x2*>(net->d_dz3), cells);
   GNG_HIP(hipGetLastError());
   net->loss_n = n;
   return GNG_OK;
@@ -1103,22 +1198,23 @@ int gng_net_backward(gng_net* net, int32_t boxes, void* stream) {
   // layer 3: dW3 from x2 and dz3, then dz2 = conv^T(dz3) * silu'(z2)
   hipLaunchKernelGGL((k_conv_wgrad<16, 4>), dim3(wb), dim3(256), 0, s, net->d_x2, net->d_dz3, net->d_partial, nm,
                      boxes);
-  hipLaunchKernelGGL((k_wgrad_reduce<16, 3>), dim3((433 * 3 + 255) / 256), dim3(256), 0, s, net->d_partial, wb,
+  hipLaunchKernelGGL((k_wgrad_reduce<16, 3>), dim3(28, 1), dim3(1024), 0, s, net->d_partial, wb,
                      gr + P_W3, gr + P_B3);
   hipLaunchKernelGGL((k_conv<4, MODE_BWD>), g, dim3(kConvThreads), 0, s, net->d_dz3, net->d_g3, (const float*)nullptr,
                      (float*)nullptr, net->d_dz2, net->d_z2, nm);
   // layer 2
   hipLaunchKernelGGL((k_conv_wgrad<16, 16>), dim3(wb), dim3(256), 0, s, net->d_x1, net->d_dz2, net->d_partial, nm,
                      boxes);
-  hipLaunchKernelGGL((k_wgrad_reduce<16, 16>), dim3((433 * 16 + 255) / 256), dim3(256), 0, s, net->d_partial, wb,
+  hipLaunchKernelGGL((k_wgrad_reduce<16, 16>), dim3(28, 4), dim3(1024), 0, s, net->d_partial, wb,
                      gr + P_W2, gr + P_B2);
   hipLaunchKernelGGL((k_conv<16, MODE_BWD>), g, dim3(kConvThreads), 0, s, net->d_dz2, net->d_g2, (const float*)nullptr,
                      (float*)nullptr, net->d_dz1, net->d_z1, nm);
   // layer 1
-  hipLaunchKernelGGL((k_conv_wgrad<kIn, 16>), dim3(wb), dim3(256), 0, s, net->d_x0, net->d_dz1, net->d_partial, nm,
+  const int wb1 = (int)(wtiles < 2 * kWgradBlocks ? wtiles : 2 * kWgradBlocks);
+  hipLaunchKernelGGL((k_conv_wgrad<kIn, 16>), dim3(wb1), dim3(256), 0, s, net->d_x0, net->d_dz1, net->d_partial, nm,
                      boxes);
-  hipLaunchKernelGGL((k_wgrad_reduce<kIn, 16>), dim3(((27 * kIn + 1) * 16 + 255) / 256), dim3(256), 0, s,
-                     net->d_partial, wb, gr + P_W1, gr + P_B1);
+  hipLaunchKernelGGL((k_wgrad_reduce<kIn, 16>), dim3((27 * kIn + 1 + 15) / 16, 4), dim3(1024), 0, s,
+                     net->d_partial, wb1, gr + P_W1, gr + P_B1);
   GNG_HIP(hipGetLastError());
   return GNG_OK;
 }
