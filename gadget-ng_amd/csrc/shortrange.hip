@@ -7,31 +7,52 @@
 // r_cut is summed exactly, which is the quantity that walk approximates.
 //
 // Method:
-//   1. particles are counted into a chaining mesh of nc^3 cells of side
-//      L/nc >= r_cut (nc >= 3) and scanned; a stable radix sort by cell
-//      (sort.hpp) puts them in cell order with ascending particle index inside
-//      each cell, and they are gathered as float4 (position relative to the
-//      corner of their unwrapped cell, mass) plus the original index.  The
-//      order of every sum is then fixed, so the result is bit-identical from
-//      call to call;
-//   2. the work list is (cell, chunk of 256 particles); its length is read
-//      back once to size the grid, so every workgroup has one chunk and the
-//      hardware dispatcher balances cells of very different occupancy;
-//   3. a workgroup streams the 27 neighbour cells through LDS 256 particles at
-//      a time and each lane sums its particle's pairs: FP32 inside a staged
-//      chunk, FP64 across chunks.  A neighbour cell at offset d (cells, each
-//      component -1, 0 or 1) holds its particles at rel + d * L/nc from the
-//      lane's cell corner, so the displacement needs no per-pair minimum
+//   1. every particle gets its cell in a chaining mesh of nc^3 cells of side
+//      L/nc >= r_cut (nc >= 3); a stable radix sort by cell (sort.hpp) puts
+//      them in cell order with ascending particle index inside each cell; the
+//      cell offsets are looked up in the sorted cells (a binary search per
+//      cell: no atomics, which a clump's particles would all aim at one
+//      counter); the particles are gathered as float4 (position relative to
+//      the corner of their unwrapped cell, G m / r_cut^3) plus the original
+//      index.  The order of every sum is then fixed, so the
+//      result is bit-identical from call to call;
+//   2. the work list is (cell, chunk of 64 particles).  A chunk with more than
+//      kHeavy particles in reach is heavy: its workgroup's four wavefronts
+//      each take a quarter of every neighbour cell and their sums are added in
+//      order; these come first in the grid.  The other chunks are one
+//      wavefront each.  The lengths stay on the device and the grid covers the
+//      most there can be;
+//   3. one wavefront takes a chunk, one particle per lane, and walks the
+//      particles of the 27 neighbour cells: FP32 inside 256 of them, FP64
+//      across.  The neighbours are wave-uniform, so they come through the
+//      scalar cache into scalar registers and the loop needs no LDS staging,
+//      barrier or per-pair vector load.  A neighbour cell at offset d (cells,
+//      each component -1, 0 or 1) holds its particles at rel + d * side from
+//      the lane's cell corner, so the displacement needs no per-pair minimum
 //      image: every pair within r_cut <= L/nc <= L/3 is its own minimum image
 //      in that form, and no pair outside the cut comes inside it.
 //
-// The split factor uses erfc from Abramowitz & Stegun 7.1.26 (|error| <=
-// 1.5e-7), sharing exp(-x^2) with the exact-split term.
+// The pair law is bound by VALU issue, a transcendental counting as four.
+// With r in units of r_cut and u = r^2 / (2 r_s^2), S(r) / r^3 is
+//   u < 2:  1/r^3 - L(r^2),  L = (1 - S) / r^3 analytic in r^2 (the reference
+//           factor: 1/r^2 (1/r - E(r^2)), E = erf / r),
+//   else:   F(r^2) itself, smooth there and free of cancellation,
+// with L, E and F from a table of 1025 quadratics over r^2 in LDS (FP64
+// coefficients at Chebyshev nodes, relative error below 1e-7): one rsq, one
+// 16-byte LDS read and 16 other operations per accepted pair, against rsq,
+// rcp, exp and 24 others for a rational erfc of absolute error 1.5e-7.
+// 96^3 particles (30 % in Plummer spheres), r_cut = 5 r_s = 6.25 cells:
+// 17.0 ms with LDS-staged neighbours, that erfc and one workgroup per 256
+// particles; 13.3 with scalar neighbours and the table; 6.3 with heavy chunks
+// spread over four wavefronts (8.1 with the erfc formula there).
+// Beyond u = 16 (r_cut above 5.6 r_s) the table would be too coarse and the
+// device library's erfc is called.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
 #include <new>
 #include <string>
+#include <type_traits>
 
 #include "../../include/gng_learned.h"
 #include "sort.hpp"
@@ -40,18 +61,13 @@
 namespace gng {
 namespace sr {
 
-constexpr int kChunk = 256;
-
-__global__ void k_fill_u32(unsigned* __restrict__ p, long long n, unsigned v) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
-}
-
-__global__ void k_fill_u64(unsigned long long* p) { *p = 0ull; }
+constexpr int kChunk = 64;          // particles per work item: one wavefront
+constexpr unsigned kHeavy = 8192;   // particles in the 27 cells above which a chunk takes a workgroup
+constexpr int kAhead = 8;           // entries past the last particle that may be loaded (never used)
 
 // The unwrapped chaining-mesh cell floor(v nc / L) of one coordinate, in FP64
 // (cs = nc / L), and its index wrapped into [0, nc); a non-finite coordinate
-// lands in cell 0.  k_count and k_gather both start from cell_floor, so a
+// lands in cell 0.  k_cells and k_gather both start from cell_floor, so a
 // particle's cell and its in-cell offset always agree.
 __device__ __forceinline__ double cell_floor(float v, double cs) { return floor((double)v * cs); }
 
@@ -61,99 +77,176 @@ __device__ __forceinline__ int wrap_cell(double fl, int nc) {
   return c >= 0.0 && c < (double)nc ? (int)c : 0;
 }
 
-__global__ void k_count(const float* __restrict__ x, const float* __restrict__ y, const float* __restrict__ z,
-                        long long n, int nc, double cs, unsigned* __restrict__ cnt, unsigned* __restrict__ cell_of) {
+__global__ __launch_bounds__(256) void k_cells(const float* __restrict__ x, const float* __restrict__ y,
+                                               const float* __restrict__ z, long long n, int nc, double cs,
+                                               unsigned* __restrict__ cell_of) {
   const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n) return;
   const int cx = wrap_cell(cell_floor(x[p], cs), nc), cy = wrap_cell(cell_floor(y[p], cs), nc),
             cz = wrap_cell(cell_floor(z[p], cs), nc);
-  const unsigned c = (unsigned)(((long long)cz * nc + cy) * nc + cx);
-  cell_of[p] = c;
-  atomicAdd(&cnt[c], 1u);
+  cell_of[p] = (unsigned)(((long long)cz * nc + cy) * nc + cx);
 }
 
-// One workgroup of 1024 threads: exclusive scans of the counts (off) and of
-// the chunk counts ceil(cnt/kChunk) (choff), each with its total at [ncell].
-__global__ __launch_bounds__(1024) void k_scan(const unsigned* __restrict__ cnt, long long ncell,
-                                               unsigned* __restrict__ off, unsigned* __restrict__ choff) {
-  __shared__ unsigned long long s1[1024], s2[1024];
-  const int t = threadIdx.x;
-  const long long seg = (ncell + 1023) / 1024;
-  const long long a = t * seg, b = a + seg < ncell ? a + seg : ncell;
-  unsigned long long c1 = 0, c2 = 0;
-  for (long long i = a; i < b; ++i) {
-    c1 += cnt[i];
-    c2 += (cnt[i] + kChunk - 1) / kChunk;
+struct Counters {
+  unsigned long long pairs;  // evaluated pairs
+  unsigned heavy, light;     // work items of each kind
+};
+
+// off[c] = first particle of cell c in the sorted cells (off[ncell] = n), and
+// the counters reset.
+__global__ __launch_bounds__(256) void k_offsets(const unsigned* __restrict__ cells, unsigned n, long long ncell,
+                                                 unsigned* __restrict__ off, Counters* __restrict__ cnt) {
+  const long long c = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (c == 0) *cnt = Counters{0ull, 0u, 0u};
+  if (c > ncell) return;
+  unsigned lo = 0, hi = n;  // the first index whose cell is >= c
+  while (lo < hi) {
+    const unsigned mid = (lo + hi) >> 1;
+    if (cells[mid] < (unsigned)c) lo = mid + 1;
+    else hi = mid;
   }
-  s1[t] = c1;
-  s2[t] = c2;
-  __syncthreads();
-  for (int d = 1; d < 1024; d <<= 1) {
-    const unsigned long long u1 = t >= d ? s1[t - d] : 0, u2 = t >= d ? s2[t - d] : 0;
-    __syncthreads();
-    s1[t] += u1;
-    s2[t] += u2;
-    __syncthreads();
+  off[c] = lo;
+}
+
+// Most heavy and light work items n particles in ncell cells can make.  The
+// particles in reach add up to 27 n over the cells, so at most 27 n / kHeavy
+// cells are heavy.
+inline long long max_heavy(long long n) { return n / kChunk + 27 * n / kHeavy + 1; }
+inline long long max_light(long long n, long long ncell) { return n / kChunk + (n < ncell ? n : ncell); }
+
+// The work items (cell, chunk): heavy ones' from the front of items, the
+// others' from its back.  One atomic per wavefront and kind; the places are
+// arbitrary, but no result depends on them.
+__global__ __launch_bounds__(256) void k_items(const unsigned* __restrict__ off, int nc, long long ncell,
+                                               uint2* __restrict__ items, unsigned cap, Counters* __restrict__ cnt) {
+  const long long c = (long long)blockIdx.x * 256 + threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  const unsigned k = c < ncell ? off[c + 1] - off[c] : 0u;
+  const unsigned chunks = (k + kChunk - 1) / kChunk;
+  unsigned reach = 0;
+  if (k) {
+    const int cx = (int)(c % nc), cy = (int)((c / nc) % nc), cz = (int)(c / ((long long)nc * nc));
+    for (int nb = 0; nb < 27; ++nb) {
+      const int ux = (cx + nb % 3 + nc - 1) % nc, uy = (cy + nb / 3 % 3 + nc - 1) % nc, uz = (cz + nb / 9 + nc - 1) % nc;
+      const long long u = ((long long)uz * nc + uy) * nc + ux;
+      reach += off[u + 1] - off[u];
+    }
   }
-  unsigned long long r1 = s1[t] - c1, r2 = s2[t] - c2;
-  for (long long i = a; i < b; ++i) {
-    off[i] = (unsigned)r1;
-    choff[i] = (unsigned)r2;
-    r1 += cnt[i];
-    r2 += (cnt[i] + kChunk - 1) / kChunk;
-  }
-  if (t == 1023) {
-    off[ncell] = (unsigned)s1[1023];
-    choff[ncell] = (unsigned)s2[1023];
+  for (int kind = 0; kind < 2; ++kind) {
+    const unsigned mine = (reach > kHeavy) == (kind == 0) ? chunks : 0u;
+    unsigned incl = mine;
+    for (int d = 1; d < 64; d <<= 1) {
+      const unsigned t = __shfl_up(incl, d);
+      if (lane >= d) incl += t;
+    }
+    unsigned base = 0;
+    if (lane == 63 && incl != 0u) base = atomicAdd(kind == 0 ? &cnt->heavy : &cnt->light, incl);
+    base = __shfl(base, 63) + incl - mine;
+    for (unsigned q = 0; q < mine; ++q)
+      items[kind == 0 ? base + q : cap - 1u - (base + q)] = make_uint2((unsigned)c, q);
   }
 }
 
 // sorted[i] = particle order[i] (the cell-sorted permutation): its position
 // relative to the corner of its unwrapped cell, v - floor(v nc / L) L / nc,
-// formed in FP64 from the same floor as k_count's (so it is also the offset
+// formed in FP64 from the same floor as k_cells' (so it is also the offset
 // from the wrapped cell's corner, whatever image of the box v lies in), and
-// its mass
-__global__ void k_gather(const float* __restrict__ x, const float* __restrict__ y, const float* __restrict__ z,
-                         const float* __restrict__ m, long long n, const unsigned* __restrict__ order, double cs,
-                         double cside, float4* __restrict__ sorted, unsigned* __restrict__ sidx) {
+// G m / r_cut^3.  The offset stays in the caller's unit: neighbours' roundings
+// to FP32 are then mostly the same one, and cancel in their displacement
+__global__ __launch_bounds__(256) void k_gather(const float* __restrict__ x, const float* __restrict__ y,
+                                                const float* __restrict__ z, const float* __restrict__ m, long long n,
+                                                const unsigned* __restrict__ order, double cs, double cside,
+                                                double g_rc3, float4* __restrict__ sorted,
+                                                unsigned* __restrict__ sidx) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const unsigned p = order[i];
   const float vx = x[p], vy = y[p], vz = z[p];
   sorted[i] = make_float4((float)((double)vx - cell_floor(vx, cs) * cside),
                           (float)((double)vy - cell_floor(vy, cs) * cside),
-                          (float)((double)vz - cell_floor(vz, cs) * cside), m[p]);
+                          (float)((double)vz - cell_floor(vz, cs) * cside), (float)((double)m[p] * g_rc3));
   sidx[i] = p;
 }
 
 struct Params {
-  float csize, rc2, eps2, inv_s2rs, g;  // csize: chaining cell side L/nc
-  float log2e_s2rs2;                    // log2(e) / (2 r_s^2)
+  float csize;     // chaining cell side
+  float rc2;       // r_cut^2
+  // the rest with lengths in units of r_cut
+  float inv_rc2;   // to those units
+  float eps2;
+  float kappa;     // r_cut / (sqrt(2) r_s): x = kappa r
+  float e2;        // kappa^2 log2(e): exp(-x^2) = exp2(-e2 r^2)
+  float tscale;    // table entries per unit of r^2
   int nc;
-  long long ncell;
+  unsigned items;  // capacity of the work list
 };
 
+constexpr int kTable = 1024;  // entries 0 .. kTable, entry i around r^2 = i / tscale
+constexpr double kTableU = 16.0, kNearU = 2.0;
+
+// The smooth part of the pair law at r^2 = v (see the head of this file): -L
+// or E below u = kNearU (near), F above.  1 - S and erf by their power series
+// in u, which also continue them to the v < 0 of entry 0's left node.
 template <int KERNEL>
-__global__ __launch_bounds__(256) void k_force(const float4* __restrict__ sorted, const unsigned* __restrict__ sidx,
-                                               const unsigned* __restrict__ off, const unsigned* __restrict__ choff,
-                                               Params pr, float* __restrict__ ax, float* __restrict__ ay,
-                                               float* __restrict__ az, unsigned long long* __restrict__ pairs) {
-  __shared__ float4 js[kChunk];
-  // work item -> (cell, chunk): last cell with choff[c] <= blockIdx.x
-  const unsigned w = blockIdx.x;
-  long long lo = 0, hi = pr.ncell;  // invariant: choff[lo] <= w < choff[hi]
-  while (hi - lo > 1) {
-    const long long mid = (lo + hi) >> 1;
-    if (choff[mid] <= w) lo = mid;
-    else hi = mid;
+__device__ double smooth_part(double v, double kappa2, bool near) {
+  const double u = kappa2 * v, k1 = sqrt(kappa2);
+  if (near) {
+    double term = 1.0, sum = 0.0;
+    for (int m = 0; m < 40; ++m) {
+      sum += term / (double)(2 * m + (KERNEL == GNG_SR_EXACT ? 3 : 1));
+      term *= -u / (double)(m + 1);
+    }
+    // 2 / sqrt(pi); the exact split's is negated, so that it is only added
+    return KERNEL == GNG_SR_EXACT ? -2.0 * 1.1283791670955126 * sum * k1 * kappa2 : 1.1283791670955126 * sum * k1;
   }
-  const long long cell = lo;
-  const unsigned q = w - choff[cell];
-  const unsigned i = off[cell] + q * kChunk + threadIdx.x;
-  const bool live = i < off[cell + 1];
+  const double x = sqrt(u);
+  const double S = erfc(x) + (KERNEL == GNG_SR_EXACT ? 1.1283791670955126 * x * exp(-u) : 0.0);
+  return S / (v * sqrt(v));
+}
+
+// Entry i: c0 + d (c1 + d c2) with d = r^2 tscale - i in [-1/2, 1/2], through
+// the Chebyshev nodes of that interval, and 1 where the entry is near, else 0.
+template <int KERNEL>
+__global__ __launch_bounds__(256) void k_table(double kappa2, double tscale, float4* __restrict__ table) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i > kTable) return;
+  const double c = (double)i / tscale, d0 = 0.43301270189221932;  // sqrt(3) / 4
+  const bool near = kappa2 * c < kNearU;
+  const double f0 = smooth_part<KERNEL>(c, kappa2, near), fp = smooth_part<KERNEL>(c + d0 / tscale, kappa2, near),
+               fm = smooth_part<KERNEL>(c - d0 / tscale, kappa2, near);
+  table[i] = make_float4((float)f0, (float)((fp - fm) / (2.0 * d0)), (float)((fp + fm - 2.0 * f0) / (2.0 * d0 * d0)),
+                         near ? 1.0f : 0.0f);
+}
+
+// SOFT: the softening keeps a coincident pair's factor finite, so that its zero
+// displacement alone makes it vanish.
+template <int KERNEL, bool TABLE, bool SOFT>
+__global__ __launch_bounds__(256) void k_force(const float4* __restrict__ sorted, const unsigned* __restrict__ sidx,
+                                               const unsigned* __restrict__ off, const uint2* __restrict__ items,
+                                               const float4* __restrict__ table, const Params pr,
+                                               float* __restrict__ ax, float* __restrict__ ay, float* __restrict__ az,
+                                               Counters* __restrict__ cnt) {
+  constexpr int kSums = 3 * 3 * kChunk;  // doubles: three wavefronts' sums of a heavy chunk
+  __shared__ float4 tab[TABLE ? kTable + 1 : kSums / 2];
+  static_assert(kSums / 2 <= kTable, "the sums reuse the table's LDS");
+  const unsigned heavy = cnt->heavy, light = cnt->light;
+  const bool whole = blockIdx.x < heavy;  // uniform: the workgroup is one heavy chunk
+  if (!whole && (blockIdx.x - heavy) * 4u >= light) return;
+  if constexpr (TABLE) {
+    for (int e = threadIdx.x; e <= kTable; e += 256) tab[e] = table[e];
+    __syncthreads();
+  }
+  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const unsigned w = whole ? blockIdx.x : (blockIdx.x - heavy) * 4u + wave;
+  if (!whole && w >= light) return;
+  const uint2 item = items[whole ? w : pr.items - 1u - w];
+  const unsigned cell = __builtin_amdgcn_readfirstlane(item.x), i0 = off[cell] + item.y * kChunk;
+  const unsigned i = i0 + (threadIdx.x & 63u), iend = off[cell + 1];
+  const bool live = i < iend;
   const float4 pi = live ? sorted[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   const int nc = pr.nc;
-  const int cx = (int)(cell % nc), cy = (int)((cell / nc) % nc), cz = (int)(cell / ((long long)nc * nc));
+  const int cx = (int)(cell % (unsigned)nc), cy = (int)((cell / (unsigned)nc) % (unsigned)nc),
+            cz = (int)(cell / ((unsigned)nc * (unsigned)nc));
   double sx = 0.0, sy = 0.0, sz = 0.0;
   unsigned long long seen = 0;
   for (int nb = 0; nb < 27; ++nb) {
@@ -167,47 +260,87 @@ __global__ __launch_bounds__(256) void k_force(const float4* __restrict__ sorted
     uy -= uy >= nc ? nc : 0;
     uz += uz < 0 ? nc : 0;
     uz -= uz >= nc ? nc : 0;
-    const long long nbc = ((long long)uz * nc + uy) * nc + ux;
-    const unsigned j0 = off[nbc], j1 = off[nbc + 1];
+    const unsigned nbc = ((unsigned)uz * (unsigned)nc + (unsigned)uy) * (unsigned)nc + (unsigned)ux;
+    unsigned j0 = off[nbc], j1 = off[nbc + 1];
     seen += j1 - j0;
-    for (unsigned jb = j0; jb < j1; jb += kChunk) {
-      __syncthreads();
-      if (jb + threadIdx.x < j1) {
-        float4 v = sorted[jb + threadIdx.x];
-        v.w *= pr.g;  // G m, staged once per particle rather than per pair
-        js[threadIdx.x] = v;
-      }
-      __syncthreads();
-      const int cnt = (int)(j1 - jb < (unsigned)kChunk ? j1 - jb : (unsigned)kChunk);
-      float fx = 0.0f, fy = 0.0f, fz = 0.0f;
-#pragma unroll 4
-      for (int k = 0; k < cnt; ++k) {
-        const float4 pj = js[k];
-        const float dx = pj.x - px, dy = pj.y - py, dz = pj.z - pz;
-        const float r2b = dx * dx + dy * dy + dz * dz;
-        // r2b > 0 skips coincident pairs and the particle itself (for the
-        // lane's own cell the offset is 0 * csize = 0, so its displacement
-        // is exactly zero)
-        if (r2b <= pr.rc2 && r2b > 0.0f) {
-          const float r2 = r2b + pr.eps2;
-          const float rinv = rsqrtf(r2);
-          const float x = r2 * rinv * pr.inv_s2rs;
-          // exp(-x^2) with x^2 = r2 / (2 r_s^2), on the hardware exp2
-          const float e = __builtin_amdgcn_exp2f(-r2 * pr.log2e_s2rs2);
-          // hardware reciprocal (1 ulp), far below the polynomial's 1.5e-7
-          const float t = __builtin_amdgcn_rcpf(1.0f + 0.3275911f * x);
-          const float poly =
-              t * (0.254829592f + t * (-0.284496736f + t * (1.421413741f + t * (-1.453152027f + t * 1.061405429f))));
-          const float S = e * (KERNEL == GNG_SR_EXACT ? poly + 1.1283791670955126f * x : poly);
-          const float f = pj.w * S * (rinv * rinv * rinv);
-          fx += f * dx;
-          fy += f * dy;
-          fz += f * dz;
+    if (whole) {
+      const unsigned q = (j1 - j0 + 3u) / 4u;
+      j0 = min(j1, j0 + wave * q);
+      j1 = min(j1, j0 + q);
+    }
+    float fx = 0.0f, fy = 0.0f, fz = 0.0f;
+    auto pair = [&](const float4 pj) {
+      const float dx = pj.x - px, dy = pj.y - py, dz = pj.z - pz;
+      const float r2b = dx * dx + dy * dy + dz * dz;
+      // r2b > 0 skips coincident pairs and the particle itself (for the
+      // lane's own cell the offset is 0 * csize = 0, so its displacement
+      // is exactly zero)
+      if (r2b <= pr.rc2 && (SOFT || r2b > 0.0f)) {
+        const float r2 = fmaf(r2b, pr.inv_rc2, pr.eps2);
+        const float rinv = __builtin_amdgcn_rsqf(r2);
+        float f;
+        if constexpr (TABLE) {
+          // adding 1.5 * 2^23 leaves rint(t) in the low mantissa bits
+          const float tb = fmaf(r2, pr.tscale, 12582912.0f);
+          const float d = fmaf(r2, pr.tscale, -(tb - 12582912.0f));
+          const float4 q = tab[__float_as_uint(tb) - 0x4B400000u];
+          const float smooth = fmaf(d, fmaf(d, q.z, q.y), q.x);
+          if constexpr (KERNEL == GNG_SR_EXACT)
+            f = fmaf(q.w, rinv * rinv * rinv, smooth);
+          else
+            f = q.w != 0.0f ? rinv * rinv * (rinv - smooth) : smooth;
+        } else {
+          const float x = r2 * rinv * pr.kappa;
+          const float S = erfcf(x) + (KERNEL == GNG_SR_EXACT
+                                          ? 1.1283791670955126f * x * __builtin_amdgcn_exp2f(-r2 * pr.e2) : 0.0f);
+          f = S * (rinv * rinv * rinv);
         }
+        f *= pj.w;
+        fx += f * dx;
+        fy += f * dy;
+        fz += f * dz;
       }
+    };
+    // four particles at a time, the next four's scalar loads in flight
+    // (sorted has kAhead entries past the last particle)
+    unsigned j = j0;
+    float4 n0 = sorted[j], n1 = sorted[j + 1], n2 = sorted[j + 2], n3 = sorted[j + 3];
+    while (j < j1) {
+      const unsigned stop = j1 - j > 256u ? j + 256u : j1;
+      for (; j + 4 <= stop; j += 4) {
+        const float4 p0 = n0, p1 = n1, p2 = n2, p3 = n3;
+        n0 = sorted[j + 4];
+        n1 = sorted[j + 5];
+        n2 = sorted[j + 6];
+        n3 = sorted[j + 7];
+        pair(p0);
+        pair(p1);
+        pair(p2);
+        pair(p3);
+      }
+      for (; j < stop; ++j) pair(sorted[j]);  // only before the end of the cell
       sx += fx;
       sy += fy;
       sz += fz;
+      fx = fy = fz = 0.0f;
+    }
+  }
+  if (whole) {
+    double* sums = reinterpret_cast<double*>(tab);
+    __syncthreads();
+    if (wave != 0u) {
+      double* q = sums + (wave - 1u) * 3 * kChunk + (threadIdx.x & 63u);
+      q[0] = sx;
+      q[kChunk] = sy;
+      q[2 * kChunk] = sz;
+    }
+    __syncthreads();
+    if (wave != 0u) return;
+    for (int k = 0; k < 3; ++k) {
+      const double* q = sums + k * 3 * kChunk + threadIdx.x;
+      sx += q[0];
+      sy += q[kChunk];
+      sz += q[2 * kChunk];
     }
   }
   if (live) {
@@ -217,11 +350,8 @@ __global__ __launch_bounds__(256) void k_force(const float4* __restrict__ sorted
     az[o] = (float)sz;
   }
   // evaluated pairs: live lanes x particles seen
-  if (threadIdx.x == 0) {
-    const unsigned nlive = off[cell + 1] - (off[cell] + q * kChunk);
-    const unsigned nl = nlive < (unsigned)kChunk ? nlive : (unsigned)kChunk;
-    atomicAdd(pairs, (unsigned long long)nl * seen);
-  }
+  if ((threadIdx.x & 63u) == 0u)
+    atomicAdd(&cnt->pairs, (unsigned long long)(iend - i0 < kChunk ? iend - i0 : kChunk) * seen);
 }
 
 }  // namespace sr
@@ -241,10 +371,11 @@ struct gng_sr {
   void* d_temp = nullptr;  // radix-sort work space (sized for cap_n)
   size_t temp_bytes = 0;
   long long cap_cells = 0;
-  unsigned* d_cnt = nullptr;
   unsigned* d_off = nullptr;
-  unsigned* d_choff = nullptr;
-  unsigned long long* d_pairs = nullptr;
+  long long cap_items = 0;
+  uint2* d_items = nullptr;
+  float4* d_table = nullptr;
+  Counters* d_count = nullptr;
   long long last_pairs = -1;
   bool pairs_pending = false;
 };
@@ -258,19 +389,18 @@ void free_sr(gng_sr* s) {
   (void)hipFree(s->d_cell_sorted);
   (void)hipFree(s->d_order);
   (void)hipFree(s->d_temp);
-  (void)hipFree(s->d_cnt);
   (void)hipFree(s->d_off);
-  (void)hipFree(s->d_choff);
-  (void)hipFree(s->d_pairs);
+  (void)hipFree(s->d_items);
+  (void)hipFree(s->d_table);
+  (void)hipFree(s->d_count);
 }
 
 }  // namespace
 
 namespace {
 
-// Chaining-mesh bookkeeping shared by the entry points: cell of every
-// particle, per-cell counts and offsets, chunk offsets, and the stable
-// cell-sorted permutation d_order.  Returns nc through *nc_out.
+// Chaining-mesh bookkeeping shared by the entry points: cell of every particle
+// and the stable cell-sorted permutation d_order (cells in d_cell_sorted).  Returns nc through *nc_out.
 int cell_sort(gng_sr* sr, const float* d_x, const float* d_y, const float* d_z, int64_t n, double box_size,
               double r_cut, hipStream_t s, int* nc_out) {
   int nc = (int)std::floor(box_size / r_cut);
@@ -287,7 +417,7 @@ int cell_sort(gng_sr* sr, const float* d_x, const float* d_y, const float* d_z, 
     sr->d_sidx = sr->d_cell_of = sr->d_cell_sorted = sr->d_order = nullptr;
     sr->d_temp = nullptr;
     sr->cap_n = 0;
-    GNG_HIP(hipMalloc(&sr->d_sorted, sizeof(float4) * (size_t)n));
+    GNG_HIP(hipMalloc(&sr->d_sorted, sizeof(float4) * ((size_t)n + kAhead)));
     GNG_HIP(hipMalloc(&sr->d_sidx, sizeof(unsigned) * (size_t)n));
     GNG_HIP(hipMalloc(&sr->d_cell_of, sizeof(unsigned) * (size_t)n));
     GNG_HIP(hipMalloc(&sr->d_cell_sorted, sizeof(unsigned) * (size_t)n));
@@ -296,22 +426,14 @@ int cell_sort(gng_sr* sr, const float* d_x, const float* d_y, const float* d_z, 
     sr->cap_n = n;
   }
   if (ncell > sr->cap_cells) {
-    (void)hipFree(sr->d_cnt);
     (void)hipFree(sr->d_off);
-    (void)hipFree(sr->d_choff);
-    sr->d_cnt = sr->d_off = sr->d_choff = nullptr;
+    sr->d_off = nullptr;
     sr->cap_cells = 0;
-    GNG_HIP(hipMalloc(&sr->d_cnt, sizeof(unsigned) * (size_t)ncell));
     GNG_HIP(hipMalloc(&sr->d_off, sizeof(unsigned) * (size_t)(ncell + 1)));
-    GNG_HIP(hipMalloc(&sr->d_choff, sizeof(unsigned) * (size_t)(ncell + 1)));
     sr->cap_cells = ncell;
   }
-  const unsigned cb = (unsigned)((ncell + 255) / 256), pb = (unsigned)((n + 255) / 256);
-  hipLaunchKernelGGL(k_fill_u32, dim3(cb), dim3(256), 0, s, sr->d_cnt, ncell, 0u);
-  const double cs = (double)nc / box_size;
-  hipLaunchKernelGGL(k_count, dim3(pb), dim3(256), 0, s, d_x, d_y, d_z, (long long)n, nc, cs, sr->d_cnt,
-                     sr->d_cell_of);
-  hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, sr->d_cnt, ncell, sr->d_off, sr->d_choff);
+  hipLaunchKernelGGL(k_cells, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, d_x, d_y, d_z, (long long)n, nc,
+                     (double)nc / box_size, sr->d_cell_of);
   GNG_HIP(hipGetLastError());
   // stable LSD radix sort over the bits a cell index needs
   int end_bit = 1;
@@ -343,7 +465,9 @@ int gng_sr_create(int32_t device, gng_sr** out) {
   gng_sr* s = new (std::nothrow) gng_sr();
   if (!s) return fail(GNG_ERR_OOM, "host allocation failed");
   s->device = device;
-  if (hipMalloc(&s->d_pairs, sizeof(unsigned long long)) != hipSuccess) {
+  if (hipMalloc(&s->d_count, sizeof(Counters)) != hipSuccess ||
+      hipMalloc(&s->d_table, sizeof(float4) * (kTable + 1)) != hipSuccess) {
+    free_sr(s);
     delete s;
     return fail(GNG_ERR_OOM, "short-range counters");
   }
@@ -388,33 +512,49 @@ int gng_sr_accelerations(gng_sr* sr, const float* d_x, const float* d_y, const f
   int nc = 0;
   if (int e = cell_sort(sr, d_x, d_y, d_z, n, box_size, r_cut, s, &nc)) return e;
   const long long ncell = (long long)nc * nc * nc;
-  const unsigned pb = (unsigned)((n + 255) / 256);
-  hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(1), 0, s, sr->d_pairs);
-  // the same cs as the cell count (cell_sort), and the cell side
-  const double cs = (double)nc / box_size, cside = box_size / (double)nc;
-  const float csize = (float)cside;
-  hipLaunchKernelGGL(k_gather, dim3(pb), dim3(256), 0, s, d_x, d_y, d_z, d_m, (long long)n, sr->d_order, cs, cside,
-                     sr->d_sorted, sr->d_sidx);
-  GNG_HIP(hipGetLastError());
-  unsigned chunks = 0;
-  GNG_HIP(hipMemcpyAsync(&chunks, sr->d_choff + ncell, sizeof(unsigned), hipMemcpyDeviceToHost, s));
-  GNG_HIP(hipStreamSynchronize(s));
-  if (chunks == 0) return fail(GNG_ERR_HIP, "short-range work list is empty");
+  const long long cap = max_heavy(n) + max_light(n, ncell);
+  if (cap > sr->cap_items) {
+    (void)hipFree(sr->d_items);
+    sr->d_items = nullptr;
+    sr->cap_items = 0;
+    GNG_HIP(hipMalloc(&sr->d_items, sizeof(uint2) * (size_t)cap));
+    sr->cap_items = cap;
+  }
+  // the same cs as the cell lookup (cell_sort), and the cell side
+  const double cs = (double)nc / box_size, cside = box_size / (double)nc, inv_rc = 1.0 / r_cut;
+  hipLaunchKernelGGL(k_offsets, dim3((unsigned)((ncell + 256) / 256)), dim3(256), 0, s, sr->d_cell_sorted, (unsigned)n,
+                     ncell, sr->d_off, sr->d_count);
+  hipLaunchKernelGGL(k_items, dim3((unsigned)((ncell + 255) / 256)), dim3(256), 0, s, sr->d_off, nc, ncell, sr->d_items,
+                     (unsigned)cap, sr->d_count);
+  hipLaunchKernelGGL(k_gather, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, d_x, d_y, d_z, d_m, (long long)n,
+                     sr->d_order, cs, cside, g * inv_rc * inv_rc * inv_rc, sr->d_sorted, sr->d_sidx);
+  const double kappa2 = 0.5 * (r_cut / r_split) * (r_cut / r_split), e2 = eps2 * inv_rc * inv_rc;
+  // the table covers r^2 <= 1 + eps^2, with room for rounding at its end
+  const bool table = kappa2 * (1.0 + e2) <= kTableU;
   Params pr;
-  pr.csize = csize;
+  pr.csize = (float)cside;
   pr.rc2 = (float)(r_cut * r_cut);
-  pr.eps2 = (float)eps2;
-  pr.inv_s2rs = (float)(1.0 / (std::sqrt(2.0) * r_split));
-  pr.g = (float)g;
-  pr.log2e_s2rs2 = (float)(1.4426950408889634 / (2.0 * r_split * r_split));
+  pr.inv_rc2 = (float)(inv_rc * inv_rc);
+  pr.eps2 = (float)e2;
+  pr.kappa = (float)std::sqrt(kappa2);
+  pr.e2 = (float)(kappa2 * 1.4426950408889634);
+  pr.tscale = (float)((kTable - 0.6) / (1.0 + e2));
   pr.nc = nc;
-  pr.ncell = ncell;
-  if (kernel == GNG_SR_EXACT)
-    hipLaunchKernelGGL((k_force<GNG_SR_EXACT>), dim3(chunks), dim3(256), 0, s, sr->d_sorted, sr->d_sidx, sr->d_off,
-                       sr->d_choff, pr, d_ax, d_ay, d_az, sr->d_pairs);
-  else
-    hipLaunchKernelGGL((k_force<GNG_SR_REFERENCE>), dim3(chunks), dim3(256), 0, s, sr->d_sorted, sr->d_sidx,
-                       sr->d_off, sr->d_choff, pr, d_ax, d_ay, d_az, sr->d_pairs);
+  pr.items = (unsigned)cap;
+  const bool exact = kernel == GNG_SR_EXACT;
+  if (table)
+    hipLaunchKernelGGL(exact ? k_table<GNG_SR_EXACT> : k_table<GNG_SR_REFERENCE>, dim3((kTable + 256) / 256), dim3(256),
+                       0, s, kappa2, (double)pr.tscale, sr->d_table);
+  // a coincident pair's 1 / r^3 stays below 1e18
+  const bool soft = e2 >= 1e-12;
+  const auto pick = [&](auto k) {
+    constexpr int K = decltype(k)::value;
+    return table ? (soft ? k_force<K, true, true> : k_force<K, true, false>) : k_force<K, false, false>;
+  };
+  const auto force = exact ? pick(std::integral_constant<int, GNG_SR_EXACT>())
+                           : pick(std::integral_constant<int, GNG_SR_REFERENCE>());
+  hipLaunchKernelGGL(force, dim3((unsigned)(max_heavy(n) + (max_light(n, ncell) + 3) / 4)), dim3(256), 0, s,
+                     sr->d_sorted, sr->d_sidx, sr->d_off, sr->d_items, sr->d_table, pr, d_ax, d_ay, d_az, sr->d_count);
   GNG_HIP(hipGetLastError());
   sr->pairs_pending = true;
   return GNG_OK;
@@ -426,7 +566,7 @@ int64_t gng_sr_last_pair_count(const gng_sr* sr) {
   if (m->pairs_pending) {
     unsigned long long v = 0;
     if (hipSetDevice(m->device) != hipSuccess || hipDeviceSynchronize() != hipSuccess ||
-        hipMemcpy(&v, m->d_pairs, sizeof(v), hipMemcpyDeviceToHost) != hipSuccess)
+        hipMemcpy(&v, &m->d_count->pairs, sizeof(v), hipMemcpyDeviceToHost) != hipSuccess)
       return -1;
     m->last_pairs = (long long)v;
     m->pairs_pending = false;

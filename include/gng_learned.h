@@ -57,8 +57,8 @@ void gng_sr_destroy(gng_sr* sr);
 
 /* Device-resident short-range accelerations of all n particles (float32 SoA
  * device arrays), written (not added) to d_ax/d_ay/d_az on `stream`.
- * Requires box_size >= 3 r_cut.  Synchronises `stream` once (the work-list
- * size is read back). */
+ * Requires box_size >= 3 r_cut.  Enqueued; nothing is synchronised (but a
+ * first call, or one with more particles or cells, allocates). */
 int gng_sr_accelerations(gng_sr* sr, const float* d_x, const float* d_y, const float* d_z, const float* d_m,
                          int64_t n, double box_size, double r_split, double r_cut, double eps2, double g,
                          int32_t kernel, float* d_ax, float* d_ay, float* d_az, void* stream);
