@@ -712,89 +712,152 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void k_
                          nullptr, DepositSplit{});
 }
 
-// LDS fixed-point add with wavefront aggregation: the lanes whose cell equals
-// the first valid lane's cell sum their contributions in registers and one
-// lane adds the total; the others add directly.
-// Integer sums keep the result independent of the grouping.
-__device__ __forceinline__ void lds_add_aggregated(unsigned long long* acc, int cell, long long q, bool valid) {
-  const unsigned long long vmask = __ballot(valid);
-  if (vmask == 0ull) return;
-  const int lane = threadIdx.x & 63;
-  const int leader = __ffsll((long long)vmask) - 1;
-  const int lcell = __shfl(cell, leader);
-  const bool mine = valid && cell == lcell;
-  const unsigned long long mm = __ballot(mine);
-  if (__popcll(mm) > 1) {
-    long long v = mine ? q : 0ll;
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    if (lane == leader) atomicAdd(acc + lcell, (unsigned long long)v);
-    valid = valid && !mine;
-  }
-  if (valid) atomicAdd(acc + cell, (unsigned long long)q);
+// Particle moments per cell from the sorted cell records of the last sort: for
+// the particles whose base cell is c, mom[5c + a] = sum m (f_a - 1/2)
+// (a = x, y, z), mom[5c + 3] = sum m |f - 1/2|^2, mom[5c + 4] = sum m, with f
+// the 43-bit in-cell fraction of the record.  The sums are 64-bit fixed point
+// (the deposit's scale), so they do not depend on the particle order.
+//
+// kCellMomParts workgroups per tile, one for each part of its z layers (5
+// int64 LDS accumulators per cell of the part), write every cell of the tile
+// once (zero for an empty cell), so no clearing pass and no global atomics are
+// needed.  A tile above sp.items particles (a Plummer core holds 10^5) is
+// shared by slices as in the deposit: they add their sums into the tile's own
+// words of mom as int64, which k_moments_plan has cleared, and the last of
+// them converts the words in place.  256^3 particles, 30 % in 250 Plummer
+// spheres: 1.38 ms with one workgroup a part and a shuffle reduction of the
+// most common cell, 0.54 so (0.30 for a plain lattice).
+constexpr int kCellMoments = 5;
+constexpr int kCellMomThreads = 512;
+constexpr int kCellMomParts = 2;
+
+// Linear index of cell c of tile (ux, uy, uz).
+template <int T>
+__device__ __forceinline__ size_t tile_cell(int c, int ux, int uy, int uz, int nm) {
+  return ((size_t)(uz * T + c / (T * T)) * nm + (uy * T + (c / T) % T)) * nm + (ux * T + c % T);
 }
 
-// Particle moments per cell from the sorted cell records of the last sort,
-// kCellMomParts workgroups per tile, one for each part of its z layers
-// (5 int64 LDS accumulators per cell of the part), 1024 threads each, so that
-// a dense tile (a Plummer core holds 10^5 particles) is read by several
-// workgroups at once and in few rounds: for the particles whose base cell c is in the tile,
-// mom[5c + a] = sum m (f_a - 1/2) (a = x, y, z), mom[5c + 3] =
-// sum m |f - 1/2|^2, mom[5c + 4] = sum m, with f the 43-bit in-cell fraction
-// of the record.  The sums are 64-bit fixed point (the deposit's scale), so
-// they do not depend on the particle order; every cell of the tile is
-// written once (zero for an empty cell), so no clearing pass and no global
-// atomics are needed.
-constexpr int kCellMoments = 5;
-constexpr int kCellMomThreads = 1024;
-constexpr int kCellMomParts = 2;
+__global__ void k_moments_reset(SolveScalars* sc) { sc->moment_budget = 0u; }
+
+// One workgroup per tile: words 30 (slices, 1: not split) and 31 (finished
+// counter) of its range row, the slice table, and the cleared words of a split
+// tile.
+template <int T>
+__global__ __launch_bounds__(256) void k_moments_plan(const unsigned* __restrict__ offset, const TileMap tm, int nm,
+                                                      SolveScalars* sc, const DepositSplit sp,
+                                                      double* __restrict__ mom) {
+  __shared__ unsigned slices;
+  const int tile = blockIdx.x, nt = tm.nt;
+  const unsigned rank = tm.rank[tile], w = offset[rank * 8u + 8u] - offset[rank * 8u];
+  if (threadIdx.x == 0) {
+    unsigned S = 1u, slot = 0u;
+    if (sp.slots != 0u && w > sp.items) {
+      S = min((w + sp.items - 1u) / sp.items, kMaxSlices);
+      const unsigned base = atomicAdd(&sc->moment_budget, S);
+      if (base + S > sp.slots) {
+        for (unsigned e = base; e < sp.slots; ++e) sp.extra[e] = kNoSlice;
+        S = 1u;
+      } else {
+        slot = base / 2u;
+        for (unsigned k = 0; k < S; ++k) sp.extra[base + k] = (unsigned)tile | (k << 20);
+      }
+    }
+    tm.ranges[(size_t)rank * kRangeWords + 30] = S;
+    tm.ranges[(size_t)rank * kRangeWords + 31] = slot;
+    slices = S;
+  }
+  __syncthreads();
+  if (slices == 1u) return;
+  const int ux = tile % nt, uy = (tile / nt) % nt, uz = tile / (nt * nt);
+  for (int c = threadIdx.x; c < T * T * T; c += 256)
+#pragma unroll
+    for (int k = 0; k < kCellMoments; ++k) mom[tile_cell<T>(c, ux, uy, uz, nm) * kCellMoments + k] = 0.0;
+}
+
 template <int T>
 __global__ __launch_bounds__(kCellMomThreads) void k_cell_moments(const PartRec* __restrict__ sorted,
                                                                   const unsigned* __restrict__ offset,
                                                                   const CellMap cm, const TileMap tm,
                                                                   const SolveScalars* sc, long long ntot,
-                                                                  double* __restrict__ mom) {
+                                                                  const DepositSplit sp, double* __restrict__ mom) {
   constexpr int HL = T / kCellMomParts, HC = T * T * HL, NT = kCellMomThreads;
   static_assert(T % kCellMomParts == 0, "tiles split into parts of whole layers");
   __shared__ unsigned long long acc[kCellMoments][HC];
   const int tid = threadIdx.x;
   const int nt = tm.nt;
-  const int tile = blockIdx.x, half = blockIdx.y;
-  const int ux = tile % nt, uy = (tile / nt) % nt, uz = tile / (nt * nt);
-  const unsigned b0 = tm.rank[tile] * 8u;
-  const unsigned beg = offset[b0], end = offset[b0 + 8];
+  const int part = blockIdx.y;
+  // the first sp.slots workgroups of a part are slices, the others whole tiles
+  const bool slice = blockIdx.x < sp.slots;
+  unsigned tile = blockIdx.x - sp.slots, k_slice = 0;
+  if (slice) {
+    if (blockIdx.x >= sc->moment_budget) return;  // uniform
+    const unsigned v = sp.extra[blockIdx.x];
+    if (v == kNoSlice) return;
+    tile = v & 0xfffffu;
+    k_slice = v >> 20;
+  }
+  const int ux = (int)tile % nt, uy = ((int)tile / nt) % nt, uz = (int)tile / (nt * nt);
+  const unsigned rank = tm.rank[tile], b0 = rank * 8u;
+  const unsigned S = tm.ranges[(size_t)rank * kRangeWords + 30], slot = tm.ranges[(size_t)rank * kRangeWords + 31];
+  if (!slice && S > 1u) return;
+  unsigned beg = offset[b0], end = offset[b0 + 8];
+  if (slice) {
+    const unsigned share = (end - beg + S - 1u) / S;
+    beg = min(end, beg + k_slice * share);
+    end = min(end, beg + share);
+  }
   const int s = fixed_shift(sc, ntot);
   const double scale = ldexp(1.0, s), unit = ldexp(1.0, -s);
-  const unsigned rounds = (end - beg + NT - 1u) / NT;
-  {
-    for (int c = tid; c < HC; c += NT)
+  for (int c = tid; c < HC; c += NT)
 #pragma unroll
-      for (int k = 0; k < kCellMoments; ++k) acc[k][c] = 0ull;
-    __syncthreads();
-    // every lane runs the same rounds, so the aggregation ballots see whole waves
-    for (unsigned it = 0; it < rounds; ++it) {
-      const unsigned q = beg + it * NT + (unsigned)tid;
-      bool live = q < end;
-      PartRec p;
-      p.a[0] = p.a[1] = p.a[2] = 0ull;
-      if (live) p = sorted[q];
-      const int lx = rec_cell(p, 0) % T, ly = rec_cell(p, 1) % T, lz = rec_cell(p, 2) % T;
-      live = live && lz / HL == half;
-      const int c = ((lz - half * HL) * T + ly) * T + lx;
-      const double fx = rec_frac(p, 0) - 0.5, fy = rec_frac(p, 1) - 0.5, fz = rec_frac(p, 2) - 0.5;
-      const double ms = (double)rec_mass(p) * scale;
-      const long long v[kCellMoments] = {rint_small(ms * fx), rint_small(ms * fy), rint_small(ms * fz),
-                                          rint_small(ms * (fx * fx + fy * fy + fz * fz)), rint_small(ms)};
+    for (int k = 0; k < kCellMoments; ++k) acc[k][c] = 0ull;
+  __syncthreads();
+  // two records in flight per thread
+  PartRec next;
+  if (beg + (unsigned)tid < end) next = sorted[beg + (unsigned)tid];
+  for (unsigned q = beg + (unsigned)tid; q < end; q += NT) {
+    const PartRec p = next;
+    if (end - q > NT) next = sorted[q + NT];
+    const int lx = rec_cell(p, 0) % T, ly = rec_cell(p, 1) % T, lz = rec_cell(p, 2) % T;
+    if (lz / HL != part) continue;
+    const int c = ((lz - part * HL) * T + ly) * T + lx;
+    const double fx = rec_frac(p, 0) - 0.5, fy = rec_frac(p, 1) - 0.5, fz = rec_frac(p, 2) - 0.5;
+    const double ms = (double)rec_mass(p) * scale;
+    const long long v[kCellMoments] = {rint_small(ms * fx), rint_small(ms * fy), rint_small(ms * fz),
+                                        rint_small(ms * (fx * fx + fy * fy + fz * fz)), rint_small(ms)};
 #pragma unroll
-      for (int k = 0; k < kCellMoments; ++k) lds_add_aggregated(acc[k], live ? c : 0, live ? v[k] : 0ll, live);
-    }
-    __syncthreads();
-    for (int c = tid; c < HC; c += NT) {
-      const int lx = c % T, ly = (c / T) % T, lz = c / (T * T) + half * HL;
-      const size_t cell = ((size_t)(uz * T + lz) * cm.nm + (uy * T + ly)) * cm.nm + (ux * T + lx);
-#pragma unroll
-      for (int k = 0; k < kCellMoments; ++k) mom[cell * kCellMoments + k] = (double)(long long)acc[k][c] * unit;
-    }
+    for (int k = 0; k < kCellMoments; ++k) atomicAdd(&acc[k][c], (unsigned long long)v[k]);
   }
+  __syncthreads();
+  // consecutive threads take consecutive words of a cell row
+  constexpr int W = HC * kCellMoments;
+  if (!slice) {
+    for (int e = tid; e < W; e += NT) {
+      const int c = e / kCellMoments, k = e % kCellMoments;
+      mom[tile_cell<T>(c + part * HC, ux, uy, uz, cm.nm) * kCellMoments + k] = (double)(long long)acc[k][c] * unit;
+    }
+    return;
+  }
+  unsigned long long* sums = reinterpret_cast<unsigned long long*>(mom);
+  for (int e = tid; e < W; e += NT) {
+    const int c = e / kCellMoments, k = e % kCellMoments;
+    const unsigned long long v = acc[k][c];
+    if (v) atomicAdd(sums + tile_cell<T>(c + part * HC, ux, uy, uz, cm.nm) * kCellMoments + k, v);
+  }
+  __threadfence();
+  __syncthreads();
+  unsigned* const last = reinterpret_cast<unsigned*>(&acc[0][0]);  // read above
+  if (tid == 0) *last = atomicAdd(sp.done + slot, 1u) == S * kCellMomParts - 1u;
+  __syncthreads();
+  if (!*last) return;
+  __threadfence();
+  for (int e = tid; e < W * kCellMomParts; e += NT) {
+    const int c = e / kCellMoments, k = e % kCellMoments;
+    unsigned long long* p = sums + tile_cell<T>(c, ux, uy, uz, cm.nm) * kCellMoments + k;
+    const long long v = (long long)__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *reinterpret_cast<double*>(p) = (double)v * unit;
+  }
+  if (tid == 0) sp.done[slot] = 0u;
 }
 
 }  // namespace gng

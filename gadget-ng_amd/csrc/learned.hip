@@ -555,23 +555,37 @@ __global__ __launch_bounds__(256) void k_to_bf16(const float4* __restrict__ a, u
   b[i] = o;
 }
 
-// Periodic 7-point running mean along one axis (stride 1, nm or nm^2).
+// Periodic 7-point running means along x, then y: one pass over the mesh, the
+// 64 x 16 tile and its three-cell halo in LDS (three one-axis passes read and
+// wrote the mesh three times: 200 us at 256^3; 60 with the z mean in k_input,
+// which takes no longer for it).
 constexpr int kHalfWidth = 3;
-__global__ void k_boxmean(const float* __restrict__ in, float* __restrict__ out, int nm, long long stride) {
-  const long long M = (long long)nm * nm * nm;
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= M) return;
-  const int c = (int)((i / stride) % nm);
-  const long long base = i - (long long)c * stride;
-  float s = 0.0f;
-#pragma unroll
-  for (int d = -kHalfWidth; d <= kHalfWidth; ++d) {
-    int j = c + d;
-    j += j < 0 ? nm : 0;
-    j -= j >= nm ? nm : 0;
-    s += in[base + (long long)j * stride];
+constexpr int kBmX = 64, kBmY = 16, kBmHX = kBmX + 2 * kHalfWidth, kBmHY = kBmY + 2 * kHalfWidth;
+__global__ __launch_bounds__(256) void k_boxmean_xy(const float* __restrict__ in, float* __restrict__ out, int nm) {
+  __shared__ float a[kBmHY][kBmHX], b[kBmHY][kBmX];
+  const int x0 = blockIdx.x * kBmX, y0 = blockIdx.y * kBmY;
+  const float* plane = in + (long long)blockIdx.z * nm * nm;
+  for (int e = threadIdx.x; e < kBmHX * kBmHY; e += 256) {
+    const int hx = e % kBmHX, hy = e / kBmHX;
+    a[hy][hx] = plane[(y0 + hy - kHalfWidth + nm) % nm * nm + (x0 + hx - kHalfWidth + nm) % nm];
   }
-  out[i] = s * (1.0f / (2 * kHalfWidth + 1));
+  __syncthreads();
+  for (int e = threadIdx.x; e < kBmX * kBmHY; e += 256) {
+    const int x = e % kBmX, hy = e / kBmX;
+    float s = 0.0f;
+#pragma unroll
+    for (int d = 0; d <= 2 * kHalfWidth; ++d) s += a[hy][x + d];
+    b[hy][x] = s * (1.0f / (2 * kHalfWidth + 1));
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < kBmX * kBmY; e += 256) {
+    const int x = e % kBmX, y = e / kBmX;
+    float s = 0.0f;
+#pragma unroll
+    for (int d = 0; d <= 2 * kHalfWidth; ++d) s += b[y + d][x];
+    if (x0 + x < nm && y0 + y < nm)
+      out[((long long)blockIdx.z * nm + y0 + y) * nm + x0 + x] = s * (1.0f / (2 * kHalfWidth + 1));
+  }
 }
 
 // Particle moments per cell, as 64-bit fixed point (value * 2^shift) summed
@@ -646,12 +660,30 @@ __global__ void k_fill_u64(unsigned long long* __restrict__ p, long long n) {
 // The moments come as 64-bit fixed-point sums (mom, times mom_unit =
 // 2^-shift / rho_mean) or as doubles (momd, times mom_unit = 1 / rho_mean),
 // five per cell in the order of k_moments.
-__global__ void k_input(const float* __restrict__ rho, const float* __restrict__ phi,
-                        const float* __restrict__ phi_mean, const unsigned long long* __restrict__ mom,
-                        const double* __restrict__ momd, double mom_unit, long long M, float inv_rho,
-                        float inv_phi, u32x4* __restrict__ x0) {
+// phi_xy is the potential's mean along x and y (k_boxmean_xy); the mean along z
+// is taken here, from planes that neighbouring workgroups have in L2.
+__global__ __launch_bounds__(256) void k_input(const float* __restrict__ rho, const float* __restrict__ phi,
+                                               const float* __restrict__ phi_xy,
+                                               const unsigned long long* __restrict__ mom,
+                                               const double* __restrict__ momd, double mom_unit, int nm,
+                                               float inv_rho, float inv_phi, u32x4* __restrict__ x0) {
+  const long long plane = (long long)nm * nm, M = plane * nm;
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= M) return;
+  const int z = (int)(i / plane);
+  float mean = 0.0f;
+#pragma unroll
+  for (int d = -kHalfWidth; d <= kHalfWidth; ++d) {
+    int j = z + d;
+    j += j < 0 ? nm : 0;
+    j -= j >= nm ? nm : 0;
+    mean += phi_xy[i + (j - z) * plane];
+  }
+  {
+#pragma clang fp contract(off)
+    mean = mean * (1.0f / (2 * kHalfWidth + 1));
+    mean = phi[i] - mean;  // both rounded by themselves, as the x and y means are
+  }
   float c2 = 0.0f, c3 = 0.0f, c4 = 0.0f, c5 = 0.0f;
   if (mom || momd) {
     double v[kMoments];
@@ -671,7 +703,7 @@ __global__ void k_input(const float* __restrict__ rho, const float* __restrict__
     c5 = (float)(spread > 0.0 ? spread : 0.0);
   }
   u32x4 v;
-  v.x = pack_bf16(rho[i] * inv_rho - 1.0f, (phi[i] - phi_mean[i]) * inv_phi);
+  v.x = pack_bf16(rho[i] * inv_rho - 1.0f, mean * inv_phi);
   v.y = pack_bf16(c2, c3);
   v.z = pack_bf16(c4, c5);
   v.w = 0u;
@@ -853,7 +885,7 @@ struct gng_net {
   float* d_partial = nullptr;
   double* d_loss = nullptr;
   long long loss_n = 0;
-  float* d_tmp = nullptr;  // 2 x M floats for the input's box means
+  float* d_tmp = nullptr;  // M floats for the input's box means
   unsigned long long* d_mom = nullptr;  // kMoments x M fixed-point particle moments (allocated on first use)
 };
 
@@ -927,12 +959,9 @@ int net_input(gng_net* net, int32_t box, const float* d_rho, const float* d_phi,
               const unsigned long long* mom, const double* momd, double mom_unit, hipStream_t s) {
   const dim3 g((unsigned)((net->M + 255) / 256));
   const int nm = net->nm;
-  float* t0 = net->d_tmp;
-  float* t1 = net->d_tmp + net->M;
-  hipLaunchKernelGGL(k_boxmean, g, dim3(256), 0, s, d_phi, t0, nm, 1LL);
-  hipLaunchKernelGGL(k_boxmean, g, dim3(256), 0, s, t0, t1, nm, (long long)nm);
-  hipLaunchKernelGGL(k_boxmean, g, dim3(256), 0, s, t1, t0, nm, (long long)nm * nm);
-  hipLaunchKernelGGL(k_input, g, dim3(256), 0, s, d_rho, d_phi, t0, mom, momd, mom_unit, net->M, 1.0f / rho_mean,
+  hipLaunchKernelGGL(k_boxmean_xy, dim3((unsigned)((nm + kBmX - 1) / kBmX), (unsigned)(nm / kBmY), (unsigned)nm),
+                     dim3(256), 0, s, d_phi, net->d_tmp, nm);
+  hipLaunchKernelGGL(k_input, g, dim3(256), 0, s, d_rho, d_phi, net->d_tmp, mom, momd, mom_unit, nm, 1.0f / rho_mean,
                      1.0f / phi_scale, reinterpret_cast<u32x4*>(net->d_x0) + (long long)box * net->M);
   GNG_HIP(hipGetLastError());
   return GNG_OK;
@@ -987,7 +1016,7 @@ int gng_net_create(int32_t grid_size, int32_t max_boxes, int32_t device, gng_net
   A(&t->d_dz1, cells * 32);
   A(&t->d_partial, (size_t)kWgradBlocks * 28 * 256 * 4);
   A(&t->d_loss, 8);
-  A(&t->d_tmp, t->M * 2 * 4);
+  A(&t->d_tmp, t->M * 4);
   if (e != hipSuccess) {
     free_net(t);
     delete t;

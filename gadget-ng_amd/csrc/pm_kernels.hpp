@@ -172,7 +172,8 @@ struct SolveScalars {
   unsigned int split_budget;  // scratch tiles reserved by split deposit tiles
   long long qmean;            // integer part of the mean fixed-point mass per cell (k_tile_ranges)
   int shift;                  // fixed_shift, once the scatter is done (k_tile_ranges)
-  unsigned int pad[59];
+  unsigned int moment_budget; // slices reserved by the moments' heavy tiles (k_moments_plan)
+  unsigned int pad[58];
   unsigned long long qsum[kQSlots * kQStride];
 };
 

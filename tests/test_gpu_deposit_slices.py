@@ -35,3 +35,26 @@ def test_slices_at_their_limits(pm, oracle_mod, nm, count, corner, threads, pair
     # the density is stored as FP32: half an ulp of each cell, and the
     # fixed-point unit (below 2^-40 of the largest sum) of each contribution
     assert np.abs(d0 - ref).max() <= 2.0 ** -24 * ref.max() * 1.01
+
+
+@pytest.mark.parametrize("nm,count", [(16, 32768), (16, 32769), (48, 3 * 32768 + 5)])
+def test_moments_of_heavy_tiles(pm, nm, count):
+    """Cell moments at and past the slice length, twice (the cleared words and
+    counters are left as they were found), against sums in FP64: the fixed
+    point has over 2^40 units per mass."""
+    print(f"case moments nm={nm} count={count}", flush=True)
+    rng = np.random.default_rng(count)
+    box = float(nm)
+    pos = (8.0 + rng.normal(0.0, 1.5, (count, 3)).clip(-7.5, 7.5)) % box
+    pos = np.concatenate([pos, rng.uniform(0.0, box, (300, 3))])
+    mass = rng.uniform(0.5, 1.5, pos.shape[0]).astype(np.float32).astype(np.float64)
+    plan = pm.Plan(nm, box)
+    plan.accelerations_f64(pos, mass, 1.0)
+    i = np.floor(pos).astype(np.int64) % nm
+    c = (i[:, 2] * nm + i[:, 1]) * nm + i[:, 0]
+    f = pos - np.floor(pos) - 0.5
+    vals = np.concatenate([mass[:, None] * f, (mass * (f ** 2).sum(1))[:, None], mass[:, None]], axis=1)
+    ref = np.stack([np.bincount(c, weights=vals[:, k], minlength=nm ** 3) for k in range(5)], axis=1)
+    for _ in range(2):
+        got = plan.cell_moments().reshape(-1, 5)
+        assert np.abs(got - ref).max() <= count * 2.0 ** -38
