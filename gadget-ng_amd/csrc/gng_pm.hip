@@ -335,7 +335,8 @@ struct MeshOps {
                   unsigned long long*);
   // initial conditions: generated modes through the inverse z pass, and the
   // inverse y and x passes with mode multipliers (second derivatives)
-  void (*ic_z)(dim3, dim3, hipStream_t, IcParams, float2*, float2*, const float2*, int2);
+  // (ic_z[src]: the modes generated, generated and kept, or read back)
+  void (*ic_z[3])(dim3, dim3, hipStream_t, IcParams, float2*, float2*, float2*, const float2*, int2);
   void (*y_inv_mul)(dim3, dim3, hipStream_t, float2*, float2*, float2*, const float2*, int3);
   void (*x_inv_mul)(dim3, dim3, hipStream_t, float2*, float2*, float2*, const float2*, int3);
   // ensembles: every stage for all boxes of this mesh side in one launch
@@ -442,9 +443,13 @@ MeshOps make_ops() {
                  long long nblk, long long base, unsigned long long* modes) {
     hipLaunchKernelGGL((k_pk_col0<N>), g, b, 0, s, P, tw, w, part, nblk, base, modes);
   };
-  o.ic_z = [](dim3 g, dim3 b, hipStream_t s, IcParams ip, float2* A, float2* B, const float2* tw, int2 zc) {
-    hipLaunchKernelGGL((k_ic_z<N, C, TY>), g, b, 0, s, ip, A, B, tw, zc);
-  };
+#define GNG_IC_Z(SRC)                                                                                            \
+  o.ic_z[SRC] = [](dim3 g, dim3 b, hipStream_t s, IcParams ip, float2* modes, float2* A, float2* B, const float2* tw, \
+                   int2 zc) { hipLaunchKernelGGL((k_ic_z<N, C, TY, SRC>), g, b, 0, s, ip, modes, A, B, tw, zc); };
+  GNG_IC_Z(0)
+  GNG_IC_Z(1)
+  GNG_IC_Z(2)
+#undef GNG_IC_Z
   o.y_inv_mul = [](dim3 g, dim3 b, hipStream_t s, float2* A, float2* B, float2* P, const float2* tw, int3 codes) {
     hipLaunchKernelGGL((k_fft_y_inv<N, C, TY, true>), g, b, 0, s, A, B, P, tw, codes);
   };
@@ -584,6 +589,7 @@ struct gng_pm_plan {
   double* d_ic_sigma = nullptr;
   long long ic_sigma_cap = 0;
   float* d_ic_mask = nullptr;  // 1 per axis index, 0 at the Nyquist index (second order)
+  float2* d_ic_mesh[3] = {};   // meshes of the second order beside P, A, B (allocated on its first use)
   // Stage timing: every solve records kStages+1 events into the next slot of
   // a ring; nothing synchronises until gng_pm_stage_times() reads them.
   bool timing = false;
@@ -639,7 +645,8 @@ void free_plan(gng_pm_plan* p) {
                   (void*)p->d_idx, (void*)p->d_tile_rank, (void*)p->d_tile_order, (void*)p->d_tile_src, (void*)p->d_tile_ranges,
                   (void*)p->d_pk_w,
                   (void*)p->d_pk_part, (void*)p->d_pk_modes, (void*)p->d_pk_msum, (void*)p->d_pk_out,
-                  (void*)p->d_ic_sigma, (void*)p->d_ic_mask, (void*)p->d_part64})
+                  (void*)p->d_ic_sigma, (void*)p->d_ic_mask, (void*)p->d_ic_mesh[0], (void*)p->d_ic_mesh[1],
+                  (void*)p->d_ic_mesh[2], (void*)p->d_part64})
     (void)hipFree(q);
   if (p->done_ev) (void)hipEventDestroy(p->done_ev);
   for (int t = 0; t < 8; ++t) {
@@ -1352,37 +1359,36 @@ int ic_upload_sigma(gng_pm_plan* p, const double* sigma, long long sigma_len, hi
 // the z pass generates the modes, the force pipeline's inverse y and x passes
 // finish the three displacement transforms, then the lattice kernel.
 int run_ic(gng_pm_plan* p, const IcParams& ip, double vel_factor, double scale, long long lo, long long cnt,
-           double* pos, double* vel, hipStream_t s, int wrap = 1) {
+           double* pos, double* vel, hipStream_t s) {
   const int nm = p->cfg.grid_size, H = nm / 2;
   const MeshOps& o = *p->ops;
   const long long rows = (long long)nm * nm;
   const dim3 yz_grid((unsigned)(H / o.yz_cols), (unsigned)nm);
   const dim3 yz_block((unsigned)o.yz_threads);
-  o.ic_z(yz_grid, yz_block, s, ip, p->d_A, p->d_B, p->d_tw, make_int2(0, 1));  // a, -i n_z a
+  o.ic_z[0](yz_grid, yz_block, s, ip, nullptr, p->d_A, p->d_B, p->d_tw, make_int2(0, 1));  // a, -i n_z a
   o.y_inv(yz_grid, yz_block, s, p->d_A, p->d_B, p->d_P, p->d_tw);
   o.x_inv(dim3((unsigned)(rows / o.x_rows), 3), dim3(256), s, p->d_A, p->d_P, p->d_B, nullptr, p->d_tw, 0, 1.0f);
   p->density_valid = false;
   p->potential_valid = false;
   if (cnt > 0) {
-    const double L = p->cfg.box_size;
-    const double d = L / (double)nm;
-    const double ifft_norm = 1.0 / (double)((long long)nm * nm * nm);
-    hipLaunchKernelGGL(k_ic_particles, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s,
-                       reinterpret_cast<const float*>(p->d_B), reinterpret_cast<const float*>(p->d_P),
-                       reinterpret_cast<const float*>(p->d_A), 2 * mesh_plane(nm), nm, d, L, ifft_norm * d, scale,
-                       vel_factor, lo, cnt, pos, vel, wrap);
+    const double L = p->cfg.box_size, d = L / (double)nm, ifft_norm = 1.0 / (double)(rows * nm);
+    const IcField psi{(const float*)p->d_B, (const float*)p->d_P, (const float*)p->d_A};
+    hipLaunchKernelGGL(k_ic_particles<1>, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s, psi, IcField{},
+                       2 * mesh_plane(nm), nm, d, L, ifft_norm * d, scale, vel_factor, 0.0, 0.0, lo, cnt, pos, vel);
   }
   GNG_HIP(hipGetLastError());
   return GNG_OK;
 }
 
-// Second-order (2LPT) particles (ic_2lpt.rs:348-553): the first-order part as
-// above without the wrap; then the six second derivatives of phi in two
-// rounds of three fields through the z, y and x passes with mode multipliers
-// (round 0: xx yy zz, round 1: xz yz xy), accumulated into the source S; then
-// S through the force pipeline with G = 1/|n|^2 and every mode with a Nyquist
-// component masked, which leaves Psi2 = Re IFFT(-i n S-hat / |n|^2) in the
-// force meshes; then the second-order particle kernel.
+// Second-order (2LPT) particles (ic_2lpt.rs:348-553): the six second
+// derivatives of phi in two rounds of three fields through the z, y and x
+// passes with mode multipliers (round 0: xx yy zz, round 1: xz yz xy),
+// accumulated into the source S; S through the force pipeline with
+// G = 1/|n|^2 and every mode with a Nyquist component masked, which leaves
+// Psi2 = Re IFFT(-i n S-hat / |n|^2) in the force meshes; the first-order
+// displacement in three further meshes; then the particle kernel, which reads
+// all six.  Round 0 generates the modes and keeps them in the first of those
+// meshes; the other z passes read them back.
 int run_ic_2lpt(gng_pm_plan* p, const IcParams& ip, double vel1, double vel2, double d2, double scale, long long lo,
                 long long cnt, double* pos, double* vel, hipStream_t s) {
   const int nm = p->cfg.grid_size, H = nm / 2;
@@ -1403,23 +1409,25 @@ int run_ic_2lpt(gng_pm_plan* p, const IcParams& ip, double vel1, double vel2, do
       return fail(GNG_ERR_HIP, std::string("2LPT mask upload: ") + hipGetErrorString(e));
     }
   }
-  int rc = run_ic(p, ip, vel1, scale, lo, cnt, pos, vel, s, 0);
-  if (rc) return rc;
-  float* S = nullptr;  // the source, an unpadded real mesh
-  GNG_HIP(hipMalloc(&S, sizeof(float) * (size_t)nm3));
+  for (float2*& m : p->d_ic_mesh)
+    if (!m) GNG_HIP(hipMalloc(&m, sizeof(float2) * (size_t)nm * (size_t)mesh_plane(nm)));
+  float2 *modes = p->d_ic_mesh[0], *a1 = p->d_ic_mesh[1], *b1 = p->d_ic_mesh[2];
+  float* S = reinterpret_cast<float*>(a1);  // the source, an unpadded real mesh
+  p->density_valid = false;
+  p->potential_valid = false;
   const float* fa = reinterpret_cast<const float*>(p->d_A);
   const float* fp = reinterpret_cast<const float*>(p->d_P);
   const float* fb = reinterpret_cast<const float*>(p->d_B);
   const double inv_n6 = 1.0 / ((double)nm3 * (double)nm3);  // two unnormalised inverse transforms per factor
   const dim3 xg((unsigned)(rows / o.x_rows), 3);
   // round 0: (a, n_z^2 a) -> y (1, n_y^2, 1) -> x (n_x^2, 1, 1) = xx, yy, zz (mesh axes)
-  o.ic_z(yz_grid, yz_block, s, ip, p->d_A, p->d_B, p->d_tw, make_int2(0, 3));
+  o.ic_z[1](yz_grid, yz_block, s, ip, modes, p->d_A, p->d_B, p->d_tw, make_int2(0, 3));
   o.y_inv_mul(yz_grid, yz_block, s, p->d_A, p->d_B, p->d_P, p->d_tw, make_int3(0, 3, 0));
   o.x_inv_mul(xg, dim3(256), s, p->d_A, p->d_P, p->d_B, p->d_tw, make_int3(3, 0, 0));
   hipLaunchKernelGGL(k_ic_source, dim3((unsigned)((nm3 + 255) / 256)), dim3(256), 0, s, fa, fp, fb, S, fplane,
                      (long long)rows, nm, inv_n6, 0);
   // round 1: (n_z a, a) -> y (1, n_y, n_y) -> x (n_x, 1, n_x) = xz, yz, xy
-  o.ic_z(yz_grid, yz_block, s, ip, p->d_A, p->d_B, p->d_tw, make_int2(2, 0));
+  o.ic_z[2](yz_grid, yz_block, s, ip, modes, p->d_A, p->d_B, p->d_tw, make_int2(2, 0));
   o.y_inv_mul(yz_grid, yz_block, s, p->d_A, p->d_B, p->d_P, p->d_tw, make_int3(0, 2, 2));
   o.x_inv_mul(xg, dim3(256), s, p->d_A, p->d_P, p->d_B, p->d_tw, make_int3(2, 0, 2));
   hipLaunchKernelGGL(k_ic_source, dim3((unsigned)((nm3 + 255) / 256)), dim3(256), 0, s, fa, fp, fb, S, fplane,
@@ -1438,17 +1446,19 @@ int run_ic_2lpt(gng_pm_plan* p, const IcParams& ip, double vel1, double vel2, do
   o.z_green_col0(dim3((unsigned)(H + 1)), dim3(256), s, p->d_P, p->d_A, p->d_B, p->d_tw, gp);
   o.y_inv(yz_grid, yz_block, s, p->d_A, p->d_B, p->d_P, p->d_tw);
   o.x_inv(xg, dim3(256), s, p->d_A, p->d_P, p->d_B, nullptr, p->d_tw, 0, 1.0f);
+  // the first order: (a, -i n_z a), the y pass's third field over the modes
+  o.ic_z[2](yz_grid, yz_block, s, ip, modes, a1, b1, p->d_tw, make_int2(0, 1));
+  o.y_inv(yz_grid, yz_block, s, a1, b1, modes, p->d_tw);
+  o.x_inv(xg, dim3(256), s, a1, modes, b1, nullptr, p->d_tw, 0, 1.0f);
   if (cnt > 0) {
-    const double L = p->cfg.box_size;
-    const double d = L / (double)nm;
-    const double ifft_norm = 1.0 / (double)nm3;
-    hipLaunchKernelGGL(k_ic_particles_2lpt, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s, fb, fp, fa, fplane,
-                       nm, L, ifft_norm * d, scale * scale, d2, vel2, lo, cnt, pos, vel);
+    const double L = p->cfg.box_size, d = L / (double)nm, ifft_norm = 1.0 / (double)nm3;
+    const IcField psi{(const float*)b1, (const float*)modes, (const float*)a1}, psi2{fb, fp, fa};
+    hipLaunchKernelGGL(k_ic_particles<2>, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s, psi, psi2, fplane, nm, d,
+                       L, ifft_norm * d, scale, vel1, d2, vel2, lo, cnt, pos, vel);
   }
+  // returns when done, like the other synchronous parts of this call
   hipError_t e = hipGetLastError();
-  // S must outlive the kernels that read it
   if (e == hipSuccess) e = hipStreamSynchronize(s);
-  (void)hipFree(S);
   if (e != hipSuccess)
     return fail(e == hipErrorOutOfMemory ? GNG_ERR_OOM : GNG_ERR_HIP, std::string("2LPT: ") + hipGetErrorString(e));
   return GNG_OK;

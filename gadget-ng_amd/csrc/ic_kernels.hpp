@@ -103,7 +103,8 @@ __device__ __forceinline__ double ic_gaussian(unsigned long long s) {
   double u1 = (double)(a >> 11) / 9007199254740992.0;
   const double u2 = (double)(b >> 11) / 9007199254740992.0;
   u1 = u1 > 1e-300 ? u1 : 1e-300;
-  return sqrt(-2.0 * log(u1)) * cos(6.283185307179586 * u2);
+  // cos(2 pi u2) without the general argument reduction (u2 in [0, 1))
+  return sqrt(-2.0 * log(u1)) * cospi(2.0 * u2);
 }
 
 // delta-hat of mode (ix, iy, iz) in the reference's index order, and |n|^2.
@@ -139,14 +140,18 @@ __global__ __launch_bounds__(256) void k_ic_delta(IcParams ip, int n, double2* _
   out[e] = ic_mode(ip, n, (int)(r / n), (int)(r % n), iz, n2);
 }
 
-// One (column tile, ky) item: the modes of C columns along all kz generated
-// into LDS as a = -delta-hat / |n|^2, then the inverse z transforms of
-// m_A(n_z) a and m_B(n_z) a (multiplier codes of ic_mul: zc.x, zc.y; the
-// displacement takes 1 and -i n_z), written to the plan's A and B meshes in
-// the layout the inverse y pass reads.  Mode (column kx, row ky, plane kz) is
-// the reference's (ix, iy, iz) = (kz, ky, kx).
-template <int N, int C, int T>
-__global__ __launch_bounds__(T) void k_ic_z(const IcParams ip, float2* __restrict__ A, float2* __restrict__ B,
+// One (column tile, ky) item: the modes a = -delta-hat / |n|^2 of C columns
+// along all kz, then the inverse z transforms of m_A(n_z) a and m_B(n_z) a
+// (multiplier codes of ic_mul: zc.x, zc.y; the displacement takes 1 and
+// -i n_z), written to the A and B meshes in the layout the inverse y pass
+// reads.  Mode (column kx, row ky, plane kz) is the reference's (ix, iy, iz) =
+// (kz, ky, kx).  The modes are generated (SRC 0), generated and kept in `modes`
+// (SRC 1), or read back from there (SRC 2; modes may be A or B: a workgroup
+// reads its columns whole before it writes them).  Generating costs 2100
+// vector-issue slots a mode (over half of them the two ChaCha blocks), so the
+// three passes of the second order generate once: 256^3 441 us, read back 44.
+template <int N, int C, int T, int SRC>
+__global__ __launch_bounds__(T) void k_ic_z(const IcParams ip, float2* modes, float2* A, float2* B,
                                             const float2* __restrict__ tw_g, const int2 zc) {
   constexpr int H = N / 2, IS = C + 1;
   using F = RegFft<N, true, false, C, T, 1, IS, true, N>;
@@ -157,24 +162,31 @@ __global__ __launch_bounds__(T) void k_ic_z(const IcParams ip, float2* __restric
   const int tile = line_tile<C, H / C>(blockIdx.x), ky = blockIdx.y;
   const unsigned plane = (unsigned)mesh_plane(N);
   const size_t col0 = (size_t)ky * H + (size_t)tile * C;
-#pragma unroll 1
-  for (int e = tid; e < C * N; e += T) {
-    const int l = e % C, i = e / C;
-    int n2;
-    const double2 d = ic_mode(ip, N, i, ky, tile * C + l, n2);
-    const double dn = n2 > 0 ? (double)n2 : 1.0;  // delta-hat is 0 at n2 = 0
-    buf[i * IS + l] = make_float2((float)(-d.x / dn), (float)(-d.y / dn));
-  }
-  __syncthreads();
   float2 a[F::PER0][F::R0], w[F::PER0][F::R0], out[F::PERL][F::RL];
-  for_edge<N, F::R0, C, T, true>(tid, [&](int p, int r, int l, int i, bool ok) {
-    a[p][r] = ok ? buf[i * IS + l] : make_float2(0.f, 0.f);
-  });
+  if constexpr (SRC == 2) {
+    for_edge<N, F::R0, C, T, true>(tid, [&](int p, int r, int l, int i, bool ok) {
+      a[p][r] = ok ? modes[col0 + (unsigned)i * plane + l] : make_float2(0.f, 0.f);
+    });
+  } else {
+#pragma unroll 1
+    for (int e = tid; e < C * N; e += T) {
+      const int l = e % C, i = e / C;
+      int n2;
+      const double2 d = ic_mode(ip, N, i, ky, tile * C + l, n2);
+      const double inv = n2 > 0 ? -1.0 / (double)n2 : -1.0;  // delta-hat is 0 at n2 = 0
+      buf[i * IS + l] = make_float2((float)(d.x * inv), (float)(d.y * inv));
+    }
+    __syncthreads();
+    for_edge<N, F::R0, C, T, true>(tid, [&](int p, int r, int l, int i, bool ok) {
+      a[p][r] = ok ? buf[i * IS + l] : make_float2(0.f, 0.f);
+      if (SRC == 1 && ok) modes[col0 + (unsigned)i * plane + l] = a[p][r];
+    });
+  }
   for_edge<N, F::R0, C, T, true>(tid, [&](int p, int r, int l, int i, bool ok) {
     const float nze = (i == N / 2) ? 0.0f : (float)freq_of(i, N);
     w[p][r] = ic_mul(zc.x, nze, a[p][r]);
   });
-  // begins with a barrier: every thread has read its values from LDS
+  // begins with a barrier: every thread has its values
   F::run(w, out, buf, twl, tid);
   for_edge<N, F::RL, C, T, true>(tid, [&](int p, int r, int l, int i, bool ok) {
     if (ok) A[col0 + (unsigned)i * plane + l] = out[p][r];
@@ -196,15 +208,27 @@ __device__ __forceinline__ double ic_rem_euclid(double x, double l) {
   return r < 0.0 ? r + fabs(l) : r;
 }
 
+// The three displacement components as real fields in the plan's row layout
+// (row (z, y) at float 2 z plane + y n): the reference's x, y, z are the mesh's
+// B, P, A.
+struct IcField {
+  const float* x;
+  const float* y;
+  const float* z;
+};
+
 // Particles lo .. lo + cnt of the n^3 lattice (global id ix n^2 + iy n + iz):
-// pos and vel as n x 3 interleaved f64 (Vec3).  psi_x, psi_y, psi_z are the
-// reference's components (the mesh's B, P and A), real fields in the plan's
-// layout (row (z, y) at float 2 z plane + y n); norm = d / n^3.
-__global__ __launch_bounds__(256) void k_ic_particles(const float* __restrict__ psi_x, const float* __restrict__ psi_y,
-                                                      const float* __restrict__ psi_z, long long fplane, int n,
+// pos and vel as n x 3 interleaved f64 (Vec3); norm = d / n^3.  With ORDER 2
+// the second order is added in the reference's order of sums: D2/D1^2 s^2 Psi2
+// to the positions before the wrap and s^2 Psi2 v2 to the momenta
+// (ic_2lpt.rs:536-550), so the particle arrays are written once and read never
+// (as two kernels, 256^3: 172 + 314 us; in one 203).
+template <int ORDER>
+__global__ __launch_bounds__(256) void k_ic_particles(const IcField psi, const IcField psi2, long long fplane, int n,
                                                       double d, double box, double norm, double scale,
-                                                      double vel_factor, long long lo, long long cnt,
-                                                      double* __restrict__ pos, double* __restrict__ vel, int wrap) {
+                                                      double vel_factor, double d2, double vel2, long long lo,
+                                                      long long cnt, double* __restrict__ pos,
+                                                      double* __restrict__ vel) {
 #pragma clang fp contract(off)
   // the workgroup's 256 particles are staged in LDS so that the interleaved
   // f64 outputs go out as contiguous, coalesced stores
@@ -219,22 +243,29 @@ __global__ __launch_bounds__(256) void k_ic_particles(const float* __restrict__ 
     const long long rem = gid % nn;
     const int iy = (int)(rem / n), iz = (int)(rem % n);
     const long long off = (long long)ix * fplane + (long long)iy * n + iz;
-    double p0 = (double)psi_x[off] * norm, p1 = (double)psi_y[off] * norm, p2 = (double)psi_z[off] * norm;
-    if (scale != 1.0) {
-      p0 *= scale;
-      p1 *= scale;
-      p2 *= scale;
+    double p[3] = {(double)psi.x[off] * norm, (double)psi.y[off] * norm, (double)psi.z[off] * norm};
+    double p2[3] = {0.0, 0.0, 0.0};
+    if constexpr (ORDER == 2) {
+      p2[0] = (double)psi2.x[off] * norm;
+      p2[1] = (double)psi2.y[off] * norm;
+      p2[2] = (double)psi2.z[off] * norm;
     }
-    const double q0 = ((double)ix + 0.5) * d, q1 = ((double)iy + 0.5) * d, q2 = ((double)iz + 0.5) * d;
+    const int g[3] = {ix, iy, iz};
     double* P = sp + 3 * threadIdx.x;
     double* V = sv + 3 * threadIdx.x;
-    // without wrap: q + Psi, for the second-order kernel to complete
-    P[0] = wrap ? ic_rem_euclid(q0 + p0, box) : q0 + p0;
-    P[1] = wrap ? ic_rem_euclid(q1 + p1, box) : q1 + p1;
-    P[2] = wrap ? ic_rem_euclid(q2 + p2, box) : q2 + p2;
-    V[0] = p0 * vel_factor;
-    V[1] = p1 * vel_factor;
-    V[2] = p2 * vel_factor;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      if (scale != 1.0) p[c] *= scale;
+      double x = ((double)g[c] + 0.5) * d + p[c], v = p[c] * vel_factor;
+      if constexpr (ORDER == 2) {
+        const double scale2 = scale * scale;
+        if (scale2 != 1.0) p2[c] *= scale2;
+        x = x + d2 * p2[c];
+        v = v + p2[c] * vel2;
+      }
+      P[c] = ic_rem_euclid(x, box);
+      V[c] = v;
+    }
   }
   __syncthreads();
   for (int e = threadIdx.x; e < 3 * nloc; e += 256) {
@@ -266,51 +297,6 @@ __global__ __launch_bounds__(256) void k_ic_source(const float* __restrict__ f0,
     S[so] = (float)((a * b + b * c + c * a) * scale);
   else
     S[so] = (float)((double)S[so] - (a * a + b * b + c * c) * scale);
-}
-
-// Second-order particles: adds D2/D1^2 s^2 Psi2 to the first-order positions
-// q + s Psi1 that k_ic_particles left unwrapped (wrap = 0), wraps them, and
-// adds s^2 Psi2 v2 to the first-order momenta (ic_2lpt.rs:536-550; the sums
-// run in the reference's order).  psi2_* as in k_ic_particles.
-__global__ __launch_bounds__(256) void k_ic_particles_2lpt(const float* __restrict__ psi_x,
-                                                           const float* __restrict__ psi_y,
-                                                           const float* __restrict__ psi_z, long long fplane, int n,
-                                                           double box, double norm, double scale2, double d2,
-                                                           double vel2, long long lo, long long cnt,
-                                                           double* __restrict__ pos, double* __restrict__ vel) {
-#pragma clang fp contract(off)
-  // first-order values in and results out through LDS, coalesced
-  __shared__ double sp[3 * 256], sv[3 * 256];
-  const long long base = (long long)blockIdx.x * 256;
-  const long long t = base + threadIdx.x;
-  const int nloc = (int)(cnt - base < 256 ? cnt - base : 256);
-  for (int e = threadIdx.x; e < 3 * nloc; e += 256) {
-    sp[e] = pos[3 * base + e];
-    sv[e] = vel[3 * base + e];
-  }
-  __syncthreads();
-  if (t < cnt) {
-    const long long gid = lo + t;
-    const long long nn = (long long)n * n;
-    const int ix = (int)(gid / nn);
-    const long long rem = gid % nn;
-    const int iy = (int)(rem / n), iz = (int)(rem % n);
-    const long long off = (long long)ix * fplane + (long long)iy * n + iz;
-    double p[3] = {(double)psi_x[off] * norm, (double)psi_y[off] * norm, (double)psi_z[off] * norm};
-    double* P = sp + 3 * threadIdx.x;
-    double* V = sv + 3 * threadIdx.x;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      if (scale2 != 1.0) p[c] *= scale2;
-      P[c] = ic_rem_euclid(P[c] + d2 * p[c], box);
-      V[c] = V[c] + p[c] * vel2;
-    }
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < 3 * nloc; e += 256) {
-    pos[3 * base + e] = sp[e];
-    vel[3 * base + e] = sv[e];
-  }
 }
 
 }  // namespace gng
