@@ -748,7 +748,8 @@ __global__ __launch_bounds__(256) void k_moments_plan(const unsigned* __restrict
                                                       double* __restrict__ mom) {
   __shared__ unsigned slices;
   const int tile = blockIdx.x, nt = tm.nt;
-  const unsigned rank = tm.rank[tile], w = offset[rank * 8u + 8u] - offset[rank * 8u];
+  const bool plain = sc->plain != 0u;  // no offsets, and never split: at most kSmallN records
+  const unsigned rank = tm.rank[tile], w = plain ? 0u : offset[rank * 8u + 8u] - offset[rank * 8u];
   if (threadIdx.x == 0) {
     unsigned S = 1u, slot = 0u;
     if (sp.slots != 0u && w > sp.items) {
@@ -800,7 +801,10 @@ __global__ __launch_bounds__(kCellMomThreads) void k_cell_moments(const PartRec*
   const unsigned rank = tm.rank[tile], b0 = rank * 8u;
   const unsigned S = tm.ranges[(size_t)rank * kRangeWords + 30], slot = tm.ranges[(size_t)rank * kRangeWords + 31];
   if (!slice && S > 1u) return;
-  unsigned beg = offset[b0], end = offset[b0 + 8];
+  // records in the caller's order (a small problem's deposit does not sort):
+  // every tile looks through all of them
+  const unsigned plain = sc->plain;
+  unsigned beg = plain ? 0u : offset[b0], end = plain ? plain : offset[b0 + 8];
   if (slice) {
     const unsigned share = (end - beg + S - 1u) / S;
     beg = min(end, beg + k_slice * share);
@@ -820,6 +824,7 @@ __global__ __launch_bounds__(kCellMomThreads) void k_cell_moments(const PartRec*
     if (end - q > NT) next = sorted[q + NT];
     const int lx = rec_cell(p, 0) % T, ly = rec_cell(p, 1) % T, lz = rec_cell(p, 2) % T;
     if (lz / HL != part) continue;
+    if (plain && (rec_cell(p, 0) / T != ux || rec_cell(p, 1) / T != uy || rec_cell(p, 2) / T != uz)) continue;
     const int c = ((lz - part * HL) * T + ly) * T + lx;
     const double fx = rec_frac(p, 0) - 0.5, fy = rec_frac(p, 1) - 0.5, fz = rec_frac(p, 2) - 0.5;
     const double ms = (double)rec_mass(p) * scale;

@@ -33,6 +33,7 @@
 #include "ic_kernels.hpp"
 #include "pk_kernels.hpp"
 #include "pm_kernels.hpp"
+#include "small.hpp"
 #include "status.hpp"
 
 using namespace gng;
@@ -315,6 +316,17 @@ struct MeshOps {
   // per-cell particle moments of the sorted records
   void (*cell_moments)(unsigned ntiles, hipStream_t, const PartRec*, const unsigned*, CellMap, TileMap, SolveScalars*,
                        long long, DepositSplit, double*);
+  // small problems (small.hpp): the plane kernels are null above kPlaneMax, and
+  // run the force solve's passes, whatever the tuning, up to there, where the
+  // persistent and ensemble forms of the single passes are null
+  void (*deposit_small)(dim3, hipStream_t, const PartRec*, const unsigned*, const float*, const float*, int, CellMap,
+                        int, SolveScalars*, float*, long long, float*);
+  void (*plane_fwd)(hipStream_t, float2*, const float2*);
+  void (*z_small)(hipStream_t, float2*, float2*, float2*, const float2*, GreenParams);
+  void (*plane_inv)(hipStream_t, int, float2*, float2*, float2*, float2*, const float2*, int, float);
+  void (*plane_fwd_box)(unsigned, hipStream_t, const BoxArgs*, const float2*);
+  void (*z_small_box)(unsigned, hipStream_t, const BoxArgs*, const float2*);
+  void (*plane_inv_box)(unsigned, hipStream_t, const BoxArgs*, const float2*);
   void (*x_fwd)(dim3, dim3, hipStream_t, const float*, float2*, const float2*, long long);
   void (*y_fwd)(dim3, dim3, hipStream_t, float2*, const float2*);
   void (*z_green)(dim3, dim3, hipStream_t, const float2*, float2*, float2*, const float2*, GreenParams);
@@ -359,7 +371,7 @@ MeshOps make_ops() {
   static_assert(N % TD == 0, "deposit tiles must cover the mesh");
   static_assert((long long)(N / TD) * (N / TD) * (N / TD) <= (1LL << 20),
                 "the split deposit's extra-workgroup table keeps a tile rank in 20 bits");
-  MeshOps o;
+  MeshOps o{};
   o.nm = N;
   o.x_rows = R;
   o.yz_cols = C;
@@ -385,6 +397,34 @@ MeshOps make_ops() {
     hipLaunchKernelGGL((k_cell_moments<TD>), dim3(sp.slots + ntiles, kCellMomParts), dim3(kCellMomThreads), 0, s, srt,
                        off, cm, tm, sc, n, sp, mom);
   };
+  o.deposit_small = [](dim3 g, hipStream_t s, const PartRec* rec, const unsigned* cell, const float* mass,
+                       const float* mpart, int n, CellMap cm, int nt, SolveScalars* sc, float* rho, long long rho_plane,
+                       float* keep) {
+    hipLaunchKernelGGL((k_deposit_small<TD>), g, dim3(kSmallThreads), 0, s, rec, cell, mass, mpart, n, cm, nt, sc, rho,
+                       rho_plane, keep);
+  };
+  if constexpr (N <= kPlaneMax) {
+    constexpr int TP = PlaneCfg<N>::T;
+    o.plane_fwd = [](hipStream_t s, float2* P, const float2* tw) {
+      hipLaunchKernelGGL((k_plane_fwd<N>), dim3(N), dim3(TP), 0, s, P, tw);
+    };
+    o.z_small = [](hipStream_t s, float2* P, float2* A, float2* B, const float2* tw, GreenParams gp) {
+      hipLaunchKernelGGL((k_z_small<N>), dim3(N + N / 2 + 1), dim3(TP), 0, s, P, A, B, tw, gp);
+    };
+    o.plane_inv = [](hipStream_t s, int fields, float2* A, float2* P, float2* B, float2* pot, const float2* tw,
+                     int field0, float pot_scale) {
+      hipLaunchKernelGGL((k_plane_inv<N>), dim3(N, fields), dim3(TP), 0, s, A, P, B, pot, tw, field0, pot_scale);
+    };
+    o.plane_fwd_box = [](unsigned boxes, hipStream_t s, const BoxArgs* bx, const float2* tw) {
+      hipLaunchKernelGGL((k_plane_fwd_box<N>), dim3(N, 1, boxes), dim3(TP), 0, s, bx, tw);
+    };
+    o.z_small_box = [](unsigned boxes, hipStream_t s, const BoxArgs* bx, const float2* tw) {
+      hipLaunchKernelGGL((k_z_small_box<N>), dim3(N + N / 2 + 1, 1, boxes), dim3(TP), 0, s, bx, tw);
+    };
+    o.plane_inv_box = [](unsigned boxes, hipStream_t s, const BoxArgs* bx, const float2* tw) {
+      hipLaunchKernelGGL((k_plane_inv_box<N>), dim3(N, 3, boxes), dim3(TP), 0, s, bx, tw);
+    };
+  }
 
   o.x_fwd = [](dim3 g, dim3 b, hipStream_t s, const float* rho, float2* P, const float2* tw, long long rho_plane) {
     hipLaunchKernelGGL((k_fft_x_fwd<N, R>), g, b, 0, s, rho, P, tw, rho_plane);
@@ -398,16 +438,18 @@ MeshOps make_ops() {
   };
   o.z_green_col0 = [](dim3 g, dim3 b, hipStream_t s, const float2* P, float2* A, float2* B, const float2* tw,
                       GreenParams gp) { hipLaunchKernelGGL((k_fft_z_green_col0<N>), g, b, 0, s, P, A, B, tw, gp); };
-  o.z_green_persist = [](dim3 g, dim3 b, hipStream_t s, const float2* P, float2* A, float2* B, const float2* tw,
-                         GreenParams gp) {
-    hipLaunchKernelGGL((k_fft_z_green_persist<N, C, TY>), g, b, 0, s, P, A, B, tw, gp);
-  };
-  o.y_fwd_persist = [](dim3 g, dim3 b, hipStream_t s, float2* P, const float2* tw) {
-    hipLaunchKernelGGL((k_fft_y_fwd_persist<N, C, TY>), g, b, 0, s, P, tw);
-  };
-  o.y_inv_persist = [](dim3 g, dim3 b, hipStream_t s, float2* A, float2* B, float2* P, const float2* tw) {
-    hipLaunchKernelGGL((k_fft_y_inv_persist<N, C, TY>), g, b, 0, s, A, B, P, tw);
-  };
+  if constexpr (N > kPlaneMax) {
+    o.z_green_persist = [](dim3 g, dim3 b, hipStream_t s, const float2* P, float2* A, float2* B, const float2* tw,
+                           GreenParams gp) {
+      hipLaunchKernelGGL((k_fft_z_green_persist<N, C, TY>), g, b, 0, s, P, A, B, tw, gp);
+    };
+    o.y_fwd_persist = [](dim3 g, dim3 b, hipStream_t s, float2* P, const float2* tw) {
+      hipLaunchKernelGGL((k_fft_y_fwd_persist<N, C, TY>), g, b, 0, s, P, tw);
+    };
+    o.y_inv_persist = [](dim3 g, dim3 b, hipStream_t s, float2* A, float2* B, float2* P, const float2* tw) {
+      hipLaunchKernelGGL((k_fft_y_inv_persist<N, C, TY>), g, b, 0, s, A, B, P, tw);
+    };
+  }
   o.y_inv = [](dim3 g, dim3 b, hipStream_t s, float2* A, float2* B, float2* P, const float2* tw) {
     if constexpr (YZCfg<N>::YSPLIT) {
       // full-line tiles of the z pass's width; the caller's grid counts C-wide tiles
@@ -462,31 +504,33 @@ MeshOps make_ops() {
   o.deposit_box[1] = [](dim3 g, dim3 b, hipStream_t s, const BoxArgs* bx, TileMap tm) {
     hipLaunchKernelGGL((k_deposit_box<TD, 512>), g, b, 0, s, bx, tm);
   };
-  o.x_fwd_box = [](dim3 g, dim3 b, hipStream_t s, const BoxArgs* bx, const float2* tw) {
-    hipLaunchKernelGGL((k_fft_x_fwd_box<N, R>), g, b, 0, s, bx, tw);
-  };
-  o.y_fwd_box = [](dim3 g, dim3 b, hipStream_t s, const BoxArgs* bx, const float2* tw) {
-    hipLaunchKernelGGL((k_fft_y_fwd_box<N, C, TY>), g, b, 0, s, bx, tw);
-  };
-  o.z_green_box = [](dim3 g, dim3 b, hipStream_t s, const BoxArgs* bx, const float2* tw) {
-    hipLaunchKernelGGL((k_fft_z_green_box<N, YZCfg<N>::CZ, YZCfg<N>::TZ>), g, b, 0, s, bx, tw);
-  };
-  o.z_green_col0_box = [](dim3 g, dim3 b, hipStream_t s, const BoxArgs* bx, const float2* tw) {
-    hipLaunchKernelGGL((k_fft_z_green_col0_box<N>), g, b, 0, s, bx, tw);
-  };
-  o.y_inv_box = [](dim3 g, dim3 b, hipStream_t s, const BoxArgs* bx, const float2* tw) {
-    if constexpr (YZCfg<N>::YSPLIT) {
-      constexpr int CS = YZCfg<N>::CZ, TS = YZCfg<N>::TZ;
-      const dim3 gs((unsigned)(N / 2 / CS), g.y, g.z);
-      hipLaunchKernelGGL((k_fft_y_inv_box<N, CS, TS, 1>), gs, dim3(TS), 0, s, bx, tw);
-      hipLaunchKernelGGL((k_fft_y_inv_box<N, CS, TS, 2>), gs, dim3(TS), 0, s, bx, tw);
-    } else {
-      hipLaunchKernelGGL((k_fft_y_inv_box<N, C, TY>), g, b, 0, s, bx, tw);
-    }
-  };
-  o.x_inv_box = [](dim3 g, dim3 b, hipStream_t s, const BoxArgs* bx, const float2* tw) {
-    hipLaunchKernelGGL((k_fft_x_inv_box<N, R>), g, b, 0, s, bx, tw);
-  };
+  if constexpr (N > kPlaneMax) {
+    o.x_fwd_box = [](dim3 g, dim3 b, hipStream_t s, const BoxArgs* bx, const float2* tw) {
+      hipLaunchKernelGGL((k_fft_x_fwd_box<N, R>), g, b, 0, s, bx, tw);
+    };
+    o.y_fwd_box = [](dim3 g, dim3 b, hipStream_t s, const BoxArgs* bx, const float2* tw) {
+      hipLaunchKernelGGL((k_fft_y_fwd_box<N, C, TY>), g, b, 0, s, bx, tw);
+    };
+    o.z_green_box = [](dim3 g, dim3 b, hipStream_t s, const BoxArgs* bx, const float2* tw) {
+      hipLaunchKernelGGL((k_fft_z_green_box<N, YZCfg<N>::CZ, YZCfg<N>::TZ>), g, b, 0, s, bx, tw);
+    };
+    o.z_green_col0_box = [](dim3 g, dim3 b, hipStream_t s, const BoxArgs* bx, const float2* tw) {
+      hipLaunchKernelGGL((k_fft_z_green_col0_box<N>), g, b, 0, s, bx, tw);
+    };
+    o.y_inv_box = [](dim3 g, dim3 b, hipStream_t s, const BoxArgs* bx, const float2* tw) {
+      if constexpr (YZCfg<N>::YSPLIT) {
+        constexpr int CS = YZCfg<N>::CZ, TS = YZCfg<N>::TZ;
+        const dim3 gs((unsigned)(N / 2 / CS), g.y, g.z);
+        hipLaunchKernelGGL((k_fft_y_inv_box<N, CS, TS, 1>), gs, dim3(TS), 0, s, bx, tw);
+        hipLaunchKernelGGL((k_fft_y_inv_box<N, CS, TS, 2>), gs, dim3(TS), 0, s, bx, tw);
+      } else {
+        hipLaunchKernelGGL((k_fft_y_inv_box<N, C, TY>), g, b, 0, s, bx, tw);
+      }
+    };
+    o.x_inv_box = [](dim3 g, dim3 b, hipStream_t s, const BoxArgs* bx, const float2* tw) {
+      hipLaunchKernelGGL((k_fft_x_inv_box<N, R>), g, b, 0, s, bx, tw);
+    };
+  }
   return o;
 }
 
@@ -576,7 +620,7 @@ struct gng_pm_plan {
 
   long long last_n = 0;
   bool density_valid = false;
-  long long sorted_n = -1;  // particles of the last counting sort (its records are in d_sorted)
+  long long sorted_n = -1;  // particles of the last solve or sort (its records are in d_sorted)
 
   // power spectrum work space (allocated on first use)
   double* d_pk_w = nullptr;     // 1 / sinc(freq(i) / nm)^2, nm values
@@ -857,6 +901,38 @@ DepositSplit deposit_split(const gng_pm_plan* p, long long n, unsigned longer = 
   return sp;
 }
 
+template <typename T, typename M>
+void launch_cells_small_t(const PartIn& in, long long n, const CellMap& cm, PartRec* rec, unsigned* cell, float* mass,
+                          float* mpart, hipStream_t s) {
+  hipLaunchKernelGGL((k_cells_small<T, M>), dim3((unsigned)((n + kSmallBlock - 1) / kSmallBlock)), dim3(kSmallBlock), 0,
+                     s, pos_src<T>(in), (const M*)in.m, (int)n, cm, rec, cell, mass, mpart);
+}
+
+// The small problems' deposit: no sort, two launches.  The sort's buffers hold
+// the packed cells (bucket), the masses (rank) and the partial maxima (count).
+void run_deposit_small(gng_pm_plan* p, const PartIn& in, long long n, float* rho, long long rho_plane, hipStream_t s) {
+  const CellMap cm = cell_map(p);
+  float *mass = reinterpret_cast<float*>(p->d_rank), *mpart = reinterpret_cast<float*>(p->d_count);
+  (in.pos64 ? (in.mass64 ? launch_cells_small_t<double, double> : launch_cells_small_t<double, float>)
+            : (in.mass64 ? launch_cells_small_t<float, double> : launch_cells_small_t<float, float>))(
+      in, n, cm, p->d_sorted, p->d_bucket, mass, mpart, s);
+  mark(p, 1, s);
+  mark(p, 2, s);
+  const unsigned ntiles = (unsigned)(p->nb / 8);
+  p->ops->deposit_small(dim3(ntiles), s, p->d_sorted, p->d_bucket, mass, mpart, (int)n, cm, p->tm.nt, p->d_sc, rho,
+                        rho_plane, p->keep_density ? p->d_rho : nullptr);
+  p->sorted_n = n;
+}
+
+// Whether a solve takes the sort-free deposit: few particles (kSmallN), no more
+// tiles than about two workgroups a CU (each looks at every particle), room for
+// the partial maxima, and a gather in the caller's order (the other one walks
+// sorted records).
+bool small_deposit(const gng_pm_plan* p, long long n) {
+  return n > 0 && n <= kSmallN && p->nb / 8 <= 512 && (n + kSmallBlock - 1) / kSmallBlock <= p->nb &&
+         !p->tune.interp_sorted;
+}
+
 int run_front(gng_pm_plan* p, const PartIn& in, long long n, hipStream_t s) {
   int rc = ensure_work(p, n > 0 ? n : 1);
   if (rc) return rc;
@@ -871,16 +947,27 @@ int run_front(gng_pm_plan* p, const PartIn& in, long long n, hipStream_t s) {
   const long long rho_plane = fplane;
 
   mark(p, 0, s);
-  run_sort(p, in, n, p->tune.interp_sorted ? p->d_perm : nullptr, true, s);
-  mark(p, 2, s);
-  const unsigned ntiles = (unsigned)p->tm.nt * p->tm.nt * p->tm.nt;
-  const DepositSplit sp = p->tune.deposit_split ? deposit_split(p, n) : DepositSplit{};
-  hipLaunchKernelGGL(k_tile_ranges, dim3((ntiles + 255) / 256), dim3(256), 0, s, p->d_offset, p->tm, p->d_sc, n, sp);
-  const int pair = p->tune.deposit_pair != 0;
-  o.deposit[p->tune.deposit_wide][pair](dim3(sp.slots + xcd_grid(pair ? (ntiles + 1u) / 2u : ntiles)),
-                                        dim3(p->tune.deposit_wide ? 512 : 256), s, p->d_sorted, cm, p->tm, p->d_sc,
-                                        rho, rho_plane, p->keep_density ? p->d_rho : nullptr, sp);
+  if (small_deposit(p, n)) {
+    run_deposit_small(p, in, n, rho, rho_plane, s);
+  } else {
+    run_sort(p, in, n, p->tune.interp_sorted ? p->d_perm : nullptr, true, s);
+    mark(p, 2, s);
+    const unsigned ntiles = (unsigned)p->tm.nt * p->tm.nt * p->tm.nt;
+    const DepositSplit sp = p->tune.deposit_split ? deposit_split(p, n) : DepositSplit{};
+    hipLaunchKernelGGL(k_tile_ranges, dim3((ntiles + 255) / 256), dim3(256), 0, s, p->d_offset, p->tm, p->d_sc, n, sp);
+    const int pair = p->tune.deposit_pair != 0;
+    o.deposit[p->tune.deposit_wide][pair](dim3(sp.slots + xcd_grid(pair ? (ntiles + 1u) / 2u : ntiles)),
+                                          dim3(p->tune.deposit_wide ? 512 : 256), s, p->d_sorted, cm, p->tm, p->d_sc,
+                                          rho, rho_plane, p->keep_density ? p->d_rho : nullptr, sp);
+  }
   mark(p, 3, s);
+  if (o.plane_fwd) {
+    o.plane_fwd(s, p->d_P, p->d_tw);
+    // the two stages share one timing slot (the x stage's)
+    mark(p, 4, s);
+    mark(p, 5, s);
+    return GNG_OK;
+  }
   const long long rows = (long long)nm * nm;
   const dim3 yz_grid((unsigned)(H / o.yz_cols), (unsigned)nm);
   const dim3 yz_block((unsigned)o.yz_threads);
@@ -909,28 +996,20 @@ int run_front(gng_pm_plan* p, const PartIn& in, long long n, hipStream_t s) {
   return GNG_OK;
 }
 
-// The whole pipeline on device pointers.
-int run_pipeline(gng_pm_plan* p, const PartIn& in, long long n, const long long* idx, long long k, double g,
-                 const AccOut& out, hipStream_t s) {
-  int rc = run_front(p, in, n, s);
-  if (rc) return rc;
-  const int nm = p->cfg.grid_size;
-  const int H = nm / 2;
+// The z, inverse y and inverse x passes, one launch each or in plane chunks:
+// rho-hat in P to the three force fields in A, P and B.
+void run_back(gng_pm_plan* p, const GreenParams& gp, hipStream_t s) {
+  const int nm = p->cfg.grid_size, H = nm / 2;
   const MeshOps& o = *p->ops;
-  const CellMap cm = cell_map(p);
   const long long rows = (long long)nm * nm;
-  const long long fplane = 2 * mesh_plane(nm);
   const dim3 yz_grid((unsigned)(H / o.yz_cols), (unsigned)nm);
   const dim3 yz_block((unsigned)o.yz_threads);
-  const GreenParams gp = green_params(p, g);
-  {
-    // persistent z pass (one workgroup per CU) or one workgroup per item
-    if (p->tune.z_persistent && p->cus > 0)
-      o.z_green_persist(dim3((unsigned)p->cus), yz_block, s, p->d_P, p->d_A, p->d_B, p->d_tw, gp);
-    else
-      o.z_green(dim3((unsigned)(H / o.z_cols), (unsigned)nm), dim3((unsigned)o.z_threads), s, p->d_P, p->d_A, p->d_B,
-                p->d_tw, gp);
-  }
+  // persistent z pass (one workgroup per CU) or one workgroup per item
+  if (p->tune.z_persistent && p->cus > 0)
+    o.z_green_persist(dim3((unsigned)p->cus), yz_block, s, p->d_P, p->d_A, p->d_B, p->d_tw, gp);
+  else
+    o.z_green(dim3((unsigned)(H / o.z_cols), (unsigned)nm), dim3((unsigned)o.z_threads), s, p->d_P, p->d_A, p->d_B,
+              p->d_tw, gp);
   o.z_green_col0(dim3((unsigned)(H + 1)), dim3(256), s, p->d_P, p->d_A, p->d_B, p->d_tw, gp);
   mark(p, 6, s);
   const auto y_inv = p->tune.y_inv_narrow ? o.y_inv_narrow : o.y_inv;
@@ -947,7 +1026,8 @@ int run_pipeline(gng_pm_plan* p, const PartIn& in, long long n, const long long*
     // the two stages share one timing slot (the y stage's)
     mark(p, 7, s);
     mark(p, 8, s);
-  } else {
+    return;
+  }
   if (p->tune.y_inv_persistent && p->cus > 0)
     o.y_inv_persist(dim3((unsigned)p->cus), yz_block, s, p->d_A, p->d_B, p->d_P, p->d_tw);
   else
@@ -959,6 +1039,31 @@ int run_pipeline(gng_pm_plan* p, const PartIn& in, long long n, const long long*
             reinterpret_cast<float2*>(p->d_pot), p->d_tw, 3, (float)(p->cfg.box_size / (2.0 * M_PI)));
   o.x_inv(dim3((unsigned)(rows / o.x_rows), 3), dim3(256), s, p->d_A, p->d_P, p->d_B, nullptr, p->d_tw, 0, 1.0f);
   mark(p, 8, s);
+}
+
+// The whole pipeline on device pointers.
+int run_pipeline(gng_pm_plan* p, const PartIn& in, long long n, const long long* idx, long long k, double g,
+                 const AccOut& out, hipStream_t s) {
+  int rc = run_front(p, in, n, s);
+  if (rc) return rc;
+  const int nm = p->cfg.grid_size;
+  const MeshOps& o = *p->ops;
+  const CellMap cm = cell_map(p);
+  const long long fplane = 2 * mesh_plane(nm);
+  const GreenParams gp = green_params(p, g);
+  if (o.plane_fwd) {
+    o.z_small(s, p->d_P, p->d_A, p->d_B, p->d_tw, gp);
+    mark(p, 6, s);
+    if (p->keep_potential)
+      // the potential reads A before the force fields below overwrite it
+      o.plane_inv(s, 1, p->d_A, p->d_P, p->d_B, reinterpret_cast<float2*>(p->d_pot), p->d_tw, 3,
+                  (float)(p->cfg.box_size / (2.0 * M_PI)));
+    o.plane_inv(s, 3, p->d_A, p->d_P, p->d_B, nullptr, p->d_tw, 0, 1.0f);
+    // the two stages share one timing slot (the y stage's)
+    mark(p, 7, s);
+    mark(p, 8, s);
+  } else {
+    run_back(p, gp, s);
   }
   const float* fx = reinterpret_cast<const float*>(p->d_A);
   const float* fy = reinterpret_cast<const float*>(p->d_P);
@@ -1987,6 +2092,8 @@ int autotune_impl(gng_pm_plan* p, const PartIn& in, long long n, const AccOut& o
   constexpr float kMargin = 0.995f;
   for (int k = 0; k < kKnobs && rc == GNG_OK; ++k) {
     if (k == 7 && !p->ops->has_narrow_y_inv) continue;  // one tile width compiled
+    // the plane kernels have one form of every pass
+    if (p->ops->plane_fwd && (k == 0 || (k >= 2 && k <= 5))) continue;
     Tuning trial = best;
     if (k == 4 || k == 5) {
       // chunked or whole-mesh pass pairs
@@ -2310,13 +2417,19 @@ void launch_box_group(gng_pm_batch* b, const BoxGroup& gr, const BoxArgs* bx, lo
   hipLaunchKernelGGL(k_tile_ranges_box, dim3((ntiles + 255) / 256, 1, nbx), dim3(256), 0, s, bx, p0->tm);
   o.deposit_box[p0->tune.deposit_wide](dim3(xcd_grid(ntiles), 1, nbx), dim3(p0->tune.deposit_wide ? 512 : 256), s, bx,
                                        p0->tm);
-  const long long rows = (long long)nm * nm;
-  o.x_fwd_box(dim3((unsigned)(rows / o.x_rows), 1, nbx), dim3(256), s, bx, p0->d_tw);
-  o.y_fwd_box(dim3((unsigned)(H / o.yz_cols), (unsigned)nm, nbx), dim3((unsigned)o.yz_threads), s, bx, p0->d_tw);
-  o.z_green_box(dim3((unsigned)(H / o.z_cols), (unsigned)nm, nbx), dim3((unsigned)o.z_threads), s, bx, p0->d_tw);
-  o.z_green_col0_box(dim3((unsigned)(H + 1), 1, nbx), dim3(256), s, bx, p0->d_tw);
-  o.y_inv_box(dim3((unsigned)(H / o.yz_cols), (unsigned)nm, nbx), dim3((unsigned)o.yz_threads), s, bx, p0->d_tw);
-  o.x_inv_box(dim3((unsigned)(rows / o.x_rows), 3, nbx), dim3(256), s, bx, p0->d_tw);
+  if (o.plane_fwd) {
+    o.plane_fwd_box(nbx, s, bx, p0->d_tw);
+    o.z_small_box(nbx, s, bx, p0->d_tw);
+    o.plane_inv_box(nbx, s, bx, p0->d_tw);
+  } else {
+    const long long rows = (long long)nm * nm;
+    o.x_fwd_box(dim3((unsigned)(rows / o.x_rows), 1, nbx), dim3(256), s, bx, p0->d_tw);
+    o.y_fwd_box(dim3((unsigned)(H / o.yz_cols), (unsigned)nm, nbx), dim3((unsigned)o.yz_threads), s, bx, p0->d_tw);
+    o.z_green_box(dim3((unsigned)(H / o.z_cols), (unsigned)nm, nbx), dim3((unsigned)o.z_threads), s, bx, p0->d_tw);
+    o.z_green_col0_box(dim3((unsigned)(H + 1), 1, nbx), dim3(256), s, bx, p0->d_tw);
+    o.y_inv_box(dim3((unsigned)(H / o.yz_cols), (unsigned)nm, nbx), dim3((unsigned)o.yz_threads), s, bx, p0->d_tw);
+    o.x_inv_box(dim3((unsigned)(rows / o.x_rows), 3, nbx), dim3(256), s, bx, p0->d_tw);
+  }
   if (maxn > 0)
     hipLaunchKernelGGL(k_interp_box, dim3((unsigned)((maxn + 255) / 256), 1, nbx), dim3(256), 0, s, bx, src,
                        AccDst<float>{ax, ay, az, 1});

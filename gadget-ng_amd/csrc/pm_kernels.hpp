@@ -173,7 +173,8 @@ struct SolveScalars {
   long long qmean;            // integer part of the mean fixed-point mass per cell (k_tile_ranges)
   int shift;                  // fixed_shift, once the scatter is done (k_tile_ranges)
   unsigned int moment_budget; // slices reserved by the moments' heavy tiles (k_moments_plan)
-  unsigned int pad[58];
+  unsigned int plain;         // records in the caller's order (k_deposit_small: their number); 0: sorted
+  unsigned int pad[57];
   unsigned long long qsum[kQSlots * kQStride];
 };
 
@@ -181,12 +182,14 @@ struct SolveScalars {
 // so no cell sum can overflow int64 whatever the clustering, and with
 // max|m|*2^s < 2^51 (binding only below about 2^11 particles), so every
 // single contribution (w <= 1) converts with rint_small.
-__device__ __forceinline__ int fixed_shift(const SolveScalars* sc, long long ntot) {
-  const float mmax = __uint_as_float(sc->mmax_bits);
+__device__ __forceinline__ int fixed_shift(float mmax, long long ntot) {
   int e = 0, em = 0;
   (void)frexp((double)ntot * (double)mmax, &e);
   (void)frexp((double)mmax, &em);
   return min(62 - e, 51 - em);
+}
+__device__ __forceinline__ int fixed_shift(const SolveScalars* sc, long long ntot) {
+  return fixed_shift(__uint_as_float(sc->mmax_bits), ntot);
 }
 
 struct GreenParams {
@@ -222,6 +225,7 @@ __device__ __forceinline__ void reset_scalars_body(SolveScalars* sc) {
   if (threadIdx.x == 0) {
     sc->mmax_bits = 0u;
     sc->split_budget = 0u;
+    sc->plain = 0u;
   }
   if (threadIdx.x < kQSlots) sc->qsum[threadIdx.x * kQStride] = 0ull;
 }
@@ -494,10 +498,12 @@ __device__ __forceinline__ int freq_of(int j, int n) { return j <= n / 2 ? j : j
 // registers, the Green's function is applied there, and the inverse runs on
 // the reversed radix plan so it starts from those registers.  The packed
 // kx = 0 column is done by k_fft_z_green_col0.
+// Column tile `tile` of row ky.  Y, when not null, receives a second copy of A
+// (and may be P: a workgroup reads its columns whole before it writes them).
 template <int N, int C, int T>
-__device__ __forceinline__ void fft_z_green_body(const float2* __restrict__ P, float2* __restrict__ A,
-                                                   float2* __restrict__ B, const float2* __restrict__ tw_g,
-                                                   const GreenParams gp) {
+__device__ __forceinline__ void fft_z_green_body(const float2* P, float2* __restrict__ A, float2* __restrict__ B,
+                                                 const float2* __restrict__ tw_g, const GreenParams gp, int tile,
+                                                 int ky, float2* Y) {
   constexpr int H = N / 2, IS = C + 1;
   using FF = RegFft<N, false, false, C, T, 1, IS, true, N>;
   using FI = RegFft<N, true, true, C, T, 1, IS, true, N>;
@@ -509,12 +515,12 @@ __device__ __forceinline__ void fft_z_green_body(const float2* __restrict__ P, f
   __shared__ float2 twl[N];
   for (int e = tid; e < N; e += (int)blockDim.x) twl[e] = tw_g[e];
   const float2* tw = twl;
-  const int tile = line_tile<C, H / C>(blockIdx.x), ky = blockIdx.y;
   const unsigned plane = (unsigned)mesh_plane(N);
   const size_t col0 = (size_t)ky * H + (size_t)tile * C;
   float2 vin[FF::PER0][FF::R0], ph[FF::PERL][FF::RL];
   for_edge<N, FF::R0, C, T, true>(tid, [&](int p, int r, int l, int i, bool ok) {
-    if (ok) vin[p][r] = P[col0 + (unsigned)i * plane + l];
+    // (with Y, the packed column's workgroups may be writing column 0)
+    if (ok) vin[p][r] = Y && !(tile | l) ? make_float2(0.0f, 0.0f) : P[col0 + (unsigned)i * plane + l];
   });
   FF::run(vin, ph, buf, tw, tid);
   const int ny = freq_of(ky, N);
@@ -538,7 +544,10 @@ __device__ __forceinline__ void fft_z_green_body(const float2* __restrict__ P, f
     float2 out[FI::PERL][FI::RL];
     FI::run(w, out, buf, tw, tid);
     for_edge<N, FI::RL, C, T, true>(tid, [&](int p, int r, int l, int i, bool ok) {
-      if (ok && (tile | l)) A[col0 + (unsigned)i * plane + l] = out[p][r];
+      if (ok && (tile | l)) {
+        A[col0 + (unsigned)i * plane + l] = out[p][r];
+        if (Y) Y[col0 + (unsigned)i * plane + l] = out[p][r];
+      }
     });
   }
   for_edge<N, FI::R0, C, T, true>(tid, [&](int p, int r, int l, int i, bool ok) {
@@ -558,13 +567,13 @@ template <int N, int C, int T>
 __global__ __launch_bounds__(T) void k_fft_z_green(const float2* __restrict__ P, float2* __restrict__ A,
                                                    float2* __restrict__ B, const float2* __restrict__ tw_g,
                                                    const GreenParams gp) {
-  fft_z_green_body<N, C, T>(P, A, B, tw_g, gp);
+  fft_z_green_body<N, C, T>(P, A, B, tw_g, gp, line_tile<C, N / 2 / C>(blockIdx.x), blockIdx.y, nullptr);
 }
 
 template <int N, int C, int T>
 __global__ __launch_bounds__(T) void k_fft_z_green_box(const BoxArgs* __restrict__ bx, const float2* __restrict__ tw_g) {
   const BoxArgs& b = bx[blockIdx.z];
-  fft_z_green_body<N, C, T>(b.P, b.A, b.B, tw_g, b.gp);
+  fft_z_green_body<N, C, T>(b.P, b.A, b.B, tw_g, b.gp, line_tile<C, N / 2 / C>(blockIdx.x), blockIdx.y, nullptr);
 }
 
 // Persistent form of k_fft_z_green for large meshes: gridDim.x workgroups (one
@@ -658,14 +667,14 @@ __global__ __launch_bounds__(T) void k_fft_z_green_persist(const float2* __restr
 //   phi(ky, kz) = (G0 + GN)/2 Z(ky, kz) + (G0 - GN)/2 conj(Z(-ky, -kz)).
 // One workgroup per pair {ky, N - ky} transforms both z lines, combines them
 // with FP64 Green's factors and writes A and B of both.
-template <int N>
-__device__ __forceinline__ void fft_z_green_col0_body(const float2* __restrict__ P, float2* __restrict__ A,
-                                                          float2* __restrict__ B, const float2* __restrict__ tw,
-                                                          const GreenParams gp) {
-  constexpr int H = N / 2, T = 256, LS = N + 1;
+template <int N, int T>
+__device__ __forceinline__ void fft_z_green_col0_body(const float2* P, float2* __restrict__ A, float2* __restrict__ B,
+                                                      const float2* __restrict__ tw, const GreenParams gp, int ky,
+                                                      float2* Y) {
+  constexpr int H = N / 2, LS = N + 1;
   __shared__ float2 buf[4 * LS];
   const int tid = threadIdx.x;
-  const int ky = blockIdx.x, kym = (N - ky) % N;
+  const int kym = (N - ky) % N;
   const size_t plane = (size_t)mesh_plane(N);
   for (int e = tid; e < 2 * N; e += T) {
     const int l = e / N, z = e % N;
@@ -715,7 +724,9 @@ __device__ __forceinline__ void fft_z_green_col0_body(const float2* __restrict__
     const int l = e / N, z = e % N;
     if ((l & 1) && ky == kym) continue;  // self-paired row: written once
     float2* dst = l < 2 ? A : B;
-    dst[(size_t)z * plane + (size_t)((l & 1) ? kym : ky) * H] = buf[l * LS + z];
+    const size_t at = (size_t)z * plane + (size_t)((l & 1) ? kym : ky) * H;
+    dst[at] = buf[l * LS + z];
+    if (Y && l < 2) Y[at] = buf[l * LS + z];
   }
 }
 
@@ -723,13 +734,13 @@ template <int N>
 __global__ __launch_bounds__(256) void k_fft_z_green_col0(const float2* __restrict__ P, float2* __restrict__ A,
                                                           float2* __restrict__ B, const float2* __restrict__ tw,
                                                           const GreenParams gp) {
-  fft_z_green_col0_body<N>(P, A, B, tw, gp);
+  fft_z_green_col0_body<N, 256>(P, A, B, tw, gp, blockIdx.x, nullptr);
 }
 
 template <int N>
 __global__ __launch_bounds__(256) void k_fft_z_green_col0_box(const BoxArgs* __restrict__ bx, const float2* __restrict__ tw_g) {
   const BoxArgs& b = bx[blockIdx.z];
-  fft_z_green_col0_body<N>(b.P, b.A, b.B, tw_g, b.gp);
+  fft_z_green_col0_body<N, 256>(b.P, b.A, b.B, tw_g, b.gp, blockIdx.x, nullptr);
 }
 
 // Inverse y transforms: A -> A, -i n_y A -> P, B -> B, one after the other,

@@ -215,7 +215,12 @@ int gng_pm_force_meshes(gng_pm_plan *p, float *out);
  * same device architecture and mesh side; with GNG_PM_TUNE_FILE set it is also
  * read from and written to that file.  Untuned plans use the persistent z pass
  * at nm = 512 only, the 512-thread deposit only below 256 tiles, and two
- * tiles per deposit workgroup from nm = 1024 on.  No reference counterpart.
+ * tiles per deposit workgroup from nm = 1024 on.  Up to nm = 128 the force
+ * solve transforms whole z planes in one kernel each way; the choices of its x,
+ * y and z passes are kept but have no effect there.  Solves of at most 16384
+ * particles on at most 512 deposit tiles do not sort, and the deposit's choices
+ * have no effect on them (interp_sorted, which needs the sort, turns it back
+ * on).  No reference counterpart.
  * Synchronous; the density and potential of earlier solves are invalidated. */
 typedef struct gng_pm_tuning_t {
   int32_t z_persistent;      /* z + Green pass: persistent workgroups          */
