@@ -13,9 +13,9 @@
 //      cell offsets are looked up in the sorted cells (a binary search per
 //      cell: no atomics, which a clump's particles would all aim at one
 //      counter); the particles are gathered as float4 (position relative to
-//      the corner of their unwrapped cell, G m / r_cut^3) plus the original
-//      index.  The order of every sum is then fixed, so the
-//      result is bit-identical from call to call;
+//      the corner of their unwrapped cell, m) plus the original index.  The
+//      order of every sum is then fixed, so the result is bit-identical from
+//      call to call;
 //   2. the work list is (cell, chunk of 64 particles).  A chunk with more than
 //      kHeavy particles in reach is heavy: its workgroup's four wavefronts
 //      each take a quarter of every neighbour cell and their sums are added in
@@ -35,7 +35,7 @@
 // The pair law is bound by VALU issue, a transcendental counting as four.
 // With r in units of r_cut and u = r^2 / (2 r_s^2), S(r) / r^3 is
 //   u < 2:  1/r^3 - L(r^2),  L = (1 - S) / r^3 analytic in r^2 (the reference
-//           factor: 1/r^2 (1/r - E(r^2)), E = erf / r),
+//           factor, u < 1.25: 1/r^2 (1/r - E(r^2)), E = erf / r),
 //   else:   F(r^2) itself, smooth there and free of cancellation,
 // with L, E and F from a table of 1025 quadratics over r^2 in LDS (FP64
 // coefficients at Chebyshev nodes, relative error below 1e-7): one rsq, one
@@ -150,31 +150,33 @@ __global__ __launch_bounds__(256) void k_items(const unsigned* __restrict__ off,
 // sorted[i] = particle order[i] (the cell-sorted permutation): its position
 // relative to the corner of its unwrapped cell, v - floor(v nc / L) L / nc,
 // formed in FP64 from the same floor as k_cells' (so it is also the offset
-// from the wrapped cell's corner, whatever image of the box v lies in), and
-// G m / r_cut^3.  The offset stays in the caller's unit: neighbours' roundings
+// from the wrapped cell's corner, whatever image of the box v lies in), and m.
+// The offset stays in the caller's unit: neighbours' roundings
 // to FP32 are then mostly the same one, and cancel in their displacement
 __global__ __launch_bounds__(256) void k_gather(const float* __restrict__ x, const float* __restrict__ y,
                                                 const float* __restrict__ z, const float* __restrict__ m, long long n,
                                                 const unsigned* __restrict__ order, double cs, double cside,
-                                                double g_rc3, float4* __restrict__ sorted,
-                                                unsigned* __restrict__ sidx) {
+                                                float4* __restrict__ sorted, unsigned* __restrict__ sidx) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const unsigned p = order[i];
   const float vx = x[p], vy = y[p], vz = z[p];
   sorted[i] = make_float4((float)((double)vx - cell_floor(vx, cs) * cside),
                           (float)((double)vy - cell_floor(vy, cs) * cside),
-                          (float)((double)vz - cell_floor(vz, cs) * cside), (float)((double)m[p] * g_rc3));
+                          (float)((double)vz - cell_floor(vz, cs) * cside), m[p]);
   sidx[i] = p;
 }
 
 struct Params {
   float csize;     // chaining cell side
   float rc2;       // r_cut^2
-  // the rest with lengths in units of r_cut
-  float inv_rc2;   // to those units
+  // the rest with lengths in the unit r_u, r_cut up to the rounding of inv_rc2
+  // = 1 / r_u^2 (r_u and not r_cut, so that r^2's conversion has no error that
+  // all pairs share)
+  float inv_rc2;
+  double g;        // G / r_u^3, taken into the sums
   float eps2;
-  float kappa;     // r_cut / (sqrt(2) r_s): x = kappa r
+  float kappa;     // r_u / (sqrt(2) r_s): x = kappa r
   float e2;        // kappa^2 log2(e): exp(-x^2) = exp2(-e2 r^2)
   float tscale;    // table entries per unit of r^2
   int nc;
@@ -182,7 +184,12 @@ struct Params {
 };
 
 constexpr int kTable = 1024;  // entries 0 .. kTable, entry i around r^2 = i / tscale
-constexpr double kTableU = 16.0, kNearU = 2.0;
+constexpr double kTableU = 16.0;
+// where the law passes from the subtraction to F: the subtraction loses 1 / S of
+// a rounding (4 at u = 2 for the exact split; erfc falls faster: 9 at 1.25, 22
+// at 2), the quadratics of F get worse as u^-3 (6e-8 at 1.25 with u to 12.5)
+template <int KERNEL>
+constexpr double kNearU = KERNEL == GNG_SR_EXACT ? 2.0 : 1.25;
 
 // The smooth part of the pair law at r^2 = v (see the head of this file): -L
 // or E below u = kNearU (near), F above.  1 - S and erf by their power series
@@ -211,7 +218,7 @@ __global__ __launch_bounds__(256) void k_table(double kappa2, double tscale, flo
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i > kTable) return;
   const double c = (double)i / tscale, d0 = 0.43301270189221932;  // sqrt(3) / 4
-  const bool near = kappa2 * c < kNearU;
+  const bool near = kappa2 * c < kNearU<KERNEL>;
   const double f0 = smooth_part<KERNEL>(c, kappa2, near), fp = smooth_part<KERNEL>(c + d0 / tscale, kappa2, near),
                fm = smooth_part<KERNEL>(c - d0 / tscale, kappa2, near);
   table[i] = make_float4((float)f0, (float)((fp - fm) / (2.0 * d0)), (float)((fp + fm - 2.0 * f0) / (2.0 * d0 * d0)),
@@ -345,9 +352,9 @@ __global__ __launch_bounds__(256) void k_force(const float4* __restrict__ sorted
   }
   if (live) {
     const unsigned o = sidx[i];
-    ax[o] = (float)sx;
-    ay[o] = (float)sy;
-    az[o] = (float)sz;
+    ax[o] = (float)(sx * pr.g);
+    ay[o] = (float)(sy * pr.g);
+    az[o] = (float)(sz * pr.g);
   }
   // evaluated pairs: live lanes x particles seen
   if ((threadIdx.x & 63u) == 0u)
@@ -521,20 +528,23 @@ int gng_sr_accelerations(gng_sr* sr, const float* d_x, const float* d_y, const f
     sr->cap_items = cap;
   }
   // the same cs as the cell lookup (cell_sort), and the cell side
-  const double cs = (double)nc / box_size, cside = box_size / (double)nc, inv_rc = 1.0 / r_cut;
+  const double cs = (double)nc / box_size, cside = box_size / (double)nc;
+  const float inv_rc2 = (float)(1.0 / (r_cut * r_cut));
+  const double inv_ru2 = (double)inv_rc2, inv_ru = std::sqrt(inv_ru2);
   hipLaunchKernelGGL(k_offsets, dim3((unsigned)((ncell + 256) / 256)), dim3(256), 0, s, sr->d_cell_sorted, (unsigned)n,
                      ncell, sr->d_off, sr->d_count);
   hipLaunchKernelGGL(k_items, dim3((unsigned)((ncell + 255) / 256)), dim3(256), 0, s, sr->d_off, nc, ncell, sr->d_items,
                      (unsigned)cap, sr->d_count);
   hipLaunchKernelGGL(k_gather, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, d_x, d_y, d_z, d_m, (long long)n,
-                     sr->d_order, cs, cside, g * inv_rc * inv_rc * inv_rc, sr->d_sorted, sr->d_sidx);
-  const double kappa2 = 0.5 * (r_cut / r_split) * (r_cut / r_split), e2 = eps2 * inv_rc * inv_rc;
+                     sr->d_order, cs, cside, sr->d_sorted, sr->d_sidx);
+  const double kappa2 = 0.5 / (inv_ru2 * r_split * r_split), e2 = eps2 * inv_ru2;
   // the table covers r^2 <= 1 + eps^2, with room for rounding at its end
   const bool table = kappa2 * (1.0 + e2) <= kTableU;
   Params pr;
   pr.csize = (float)cside;
   pr.rc2 = (float)(r_cut * r_cut);
-  pr.inv_rc2 = (float)(inv_rc * inv_rc);
+  pr.inv_rc2 = inv_rc2;
+  pr.g = g * inv_ru2 * inv_ru;
   pr.eps2 = (float)e2;
   pr.kappa = (float)std::sqrt(kappa2);
   pr.e2 = (float)(kappa2 * 1.4426950408889634);
