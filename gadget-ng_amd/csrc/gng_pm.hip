@@ -614,6 +614,7 @@ struct gng_pm_plan {
   hipStream_t pipe_stream[8] = {};
   hipEvent_t pipe_ev[8][2] = {};
   unsigned char* pipe_slot[8][2] = {};
+  unsigned char* small_stage = nullptr;  // small calls' transfers (kSmallStage bytes, mapped)
   long long idx_cap = 0;
   long long* d_idx = nullptr;
   hipStream_t stream = nullptr;
@@ -700,6 +701,7 @@ void free_plan(gng_pm_plan* p) {
     }
     if (p->pipe_stream[t]) (void)hipStreamDestroy(p->pipe_stream[t]);
   }
+  if (p->small_stage) (void)hipHostFree(p->small_stage);
   free_work(p);
   for (auto& slot : p->ev)
     for (auto& e : slot)
@@ -1173,10 +1175,88 @@ struct Xfer {
   int kind;
 };
 
+// Transfers of a small call: packed into one mapped buffer, which a kernel on
+// the solve's own stream reads (or fills) over the bus.  Below about this size
+// the threads' start, their streams' events and a DMA per array cost more than
+// one thread's copies: 1024 particles on 32^3 took 157 us through them and take
+// 59 this way; 26000 with an index list on 64^3, just below it, take 136 us, and
+// 32768, just above, 193 through the threads.  The first call takes 0.2 ms, and 9
+// where it pins the threads' slots.
+constexpr size_t kSmallStage = 1u << 20;
+constexpr int kSmallSegs = 5;
+struct StageSegs {
+  unsigned* dev[kSmallSegs];
+  unsigned off[kSmallSegs], end[kSmallSegs];  // words in the buffer; last word of the running total
+  int n;
+};
+__global__ __launch_bounds__(256) void k_stage(const StageSegs sg, unsigned* host, int down) {
+  const unsigned e = blockIdx.x * 256u + threadIdx.x;
+  int k = 0;
+  unsigned beg = 0;
+  while (k < sg.n && e >= sg.end[k]) beg = sg.end[k++];
+  if (k == sg.n) return;
+  unsigned* const d = sg.dev[k] + (e - beg);
+  unsigned* const h = host + sg.off[k] + (e - beg);
+  if (down) *h = *d;
+  else *d = *h;
+}
+
+size_t staged_bytes(const Xfer& x) { return x.kind == 0 || x.kind == 3 ? x.count : x.count * sizeof(float); }
+
+// Whether the transfers fit the small buffer (each segment on its own line).
+bool small_xfers(const std::vector<Xfer>& xs) {
+  size_t total = 0;
+  for (const Xfer& x : xs) total += (staged_bytes(x) + 127) / 128 * 128;
+  return xs.size() <= (size_t)kSmallSegs && total <= kSmallStage;
+}
+
+// Uploads are enqueued on s; downloads are complete on return.
+int run_small_xfers(gng_pm_plan* p, const std::vector<Xfer>& xs, hipStream_t s, bool down) {
+  if (!p->small_stage)
+    GNG_HIP(hipHostMalloc(reinterpret_cast<void**>(&p->small_stage), kSmallStage,
+                          hipHostMallocMapped | hipHostMallocCoherent));
+  StageSegs sg{};
+  unsigned words = 0, off = 0;
+  for (const Xfer& x : xs) {
+    const unsigned w = (unsigned)(staged_bytes(x) / 4);
+    unsigned char* const buf = p->small_stage + 4 * (size_t)off;
+    if (x.kind == 0) {
+      std::memcpy(buf, x.src, x.count);
+    } else if (x.kind == 1) {
+      const double* src = static_cast<const double*>(x.src);
+      float* f = reinterpret_cast<float*>(buf);
+      for (size_t j = 0; j < x.count; ++j) f[j] = (float)src[j];
+    }
+    sg.dev[sg.n] = static_cast<unsigned*>(x.dev);
+    sg.off[sg.n] = off;
+    sg.end[sg.n++] = words += w;
+    off += (w + 31) / 32 * 32;
+  }
+  if (words == 0) return GNG_OK;
+  hipLaunchKernelGGL(k_stage, dim3((words + 255) / 256), dim3(256), 0, s, sg,
+                     reinterpret_cast<unsigned*>(p->small_stage), down ? 1 : 0);
+  GNG_HIP(hipGetLastError());
+  if (!down) return GNG_OK;
+  GNG_HIP(hipStreamSynchronize(s));
+  for (size_t k = 0; k < xs.size(); ++k) {
+    const unsigned char* buf = p->small_stage + 4 * (size_t)sg.off[k];
+    if (xs[k].kind == 3) {
+      std::memcpy(xs[k].dst, buf, xs[k].count);
+    } else {
+      const float* src = reinterpret_cast<const float*>(buf);
+      double* dst = static_cast<double*>(xs[k].dst);
+      for (size_t j = 0; j < xs[k].count; ++j) dst[j] = (double)src[j];
+    }
+  }
+  return GNG_OK;
+}
+
 // Splits the transfers into slot-sized chunks and runs them on the worker
 // threads; for downloads, `after` (recorded on the compute stream) gates
 // every DMA; for uploads, s waits for every worker stream when they are done.
 int run_xfers(gng_pm_plan* p, const std::vector<Xfer>& xs, hipStream_t s, hipEvent_t after) {
+  if (small_xfers(xs)) return run_small_xfers(p, xs, s, after != nullptr);
+  if (int rc = ensure_pipe(p)) return rc;
   struct Chunk {
     const Xfer* x;
     size_t off, n;  // in elements of the transfer (bytes for kind 0)
@@ -1334,7 +1414,6 @@ int solve_host_soa(gng_pm_plan* p, const float* x, const float* y, const float* 
   if (idx)
     for (long long j = 0; j < k; ++j)
       if (idx[j] < 0 || idx[j] >= n) return fail(GNG_ERR_INVALID, "index out of range");
-  if ((rc = ensure_pipe(p))) return rc;
   const size_t nb = sizeof(float) * (size_t)n;
   std::vector<Xfer> up;
   if (n > 0)
@@ -1746,7 +1825,6 @@ int gng_pm_accelerations_f64(gng_pm_plan* p, const double* pos, const double* ma
   StreamOrder order(p, s);
   if ((rc = ensure_part64(p, n, k))) return rc;
   if (idx && (rc = ensure_idx(p, k))) return rc;
-  if ((rc = ensure_pipe(p))) return rc;
   // device layout: f64 positions (3 cap64), f32 masses (cap64 floats), f32
   // accelerations (3 cap64 floats, interleaved like the output)
   double* dpos = p->d_part64;
