@@ -33,7 +33,7 @@
 //      in that form, and no pair outside the cut comes inside it.
 //
 // The pair law is bound by VALU issue, a transcendental counting as four.
-// With r in units of r_cut and u = r^2 / (2 r_s^2), S(r) / r^3 is
+// With r in units of r_u (r_cut^2 to the next power of two) and u = r^2 / (2 r_s^2), S(r) / r^3 is
 //   u < 2:  1/r^3 - L(r^2),  L = (1 - S) / r^3 analytic in r^2 (the reference
 //           factor, u < 1.25: 1/r^2 (1/r - E(r^2)), E = erf / r),
 //   else:   F(r^2) itself, smooth there and free of cancellation,
@@ -170,10 +170,9 @@ __global__ __launch_bounds__(256) void k_gather(const float* __restrict__ x, con
 struct Params {
   float csize;     // chaining cell side
   float rc2;       // r_cut^2
-  // the rest with lengths in the unit r_u, r_cut up to the rounding of inv_rc2
-  // = 1 / r_u^2 (r_u and not r_cut, so that r^2's conversion has no error that
-  // all pairs share)
-  float inv_rc2;
+  // the rest with lengths in the unit r_u: r_u^2 = 1 / inv_ru2, the power of two
+  // next to r_cut^2, so that the scaled r^2 and eps^2 round like the unscaled
+  float inv_ru2;
   double g;        // G / r_u^3, taken into the sums
   float eps2;
   float kappa;     // r_u / (sqrt(2) r_s): x = kappa r
@@ -283,7 +282,7 @@ __global__ __launch_bounds__(256) void k_force(const float4* __restrict__ sorted
       // lane's own cell the offset is 0 * csize = 0, so its displacement
       // is exactly zero)
       if (r2b <= pr.rc2 && (SOFT || r2b > 0.0f)) {
-        const float r2 = fmaf(r2b, pr.inv_rc2, pr.eps2);
+        const float r2 = fmaf(r2b, pr.inv_ru2, pr.eps2);
         const float rinv = __builtin_amdgcn_rsqf(r2);
         float f;
         if constexpr (TABLE) {
@@ -529,8 +528,7 @@ int gng_sr_accelerations(gng_sr* sr, const float* d_x, const float* d_y, const f
   }
   // the same cs as the cell lookup (cell_sort), and the cell side
   const double cs = (double)nc / box_size, cside = box_size / (double)nc;
-  const float inv_rc2 = (float)(1.0 / (r_cut * r_cut));
-  const double inv_ru2 = (double)inv_rc2, inv_ru = std::sqrt(inv_ru2);
+  const double inv_ru2 = std::exp2(-std::round(2.0 * std::log2(r_cut))), inv_ru = std::sqrt(inv_ru2);
   hipLaunchKernelGGL(k_offsets, dim3((unsigned)((ncell + 256) / 256)), dim3(256), 0, s, sr->d_cell_sorted, (unsigned)n,
                      ncell, sr->d_off, sr->d_count);
   hipLaunchKernelGGL(k_items, dim3((unsigned)((ncell + 255) / 256)), dim3(256), 0, s, sr->d_off, nc, ncell, sr->d_items,
@@ -538,17 +536,18 @@ int gng_sr_accelerations(gng_sr* sr, const float* d_x, const float* d_y, const f
   hipLaunchKernelGGL(k_gather, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, d_x, d_y, d_z, d_m, (long long)n,
                      sr->d_order, cs, cside, sr->d_sorted, sr->d_sidx);
   const double kappa2 = 0.5 / (inv_ru2 * r_split * r_split), e2 = eps2 * inv_ru2;
-  // the table covers r^2 <= 1 + eps^2, with room for rounding at its end
-  const bool table = kappa2 * (1.0 + e2) <= kTableU;
+  // the table covers r^2 <= r_cut^2 + eps^2, with room for rounding at its end
+  const double r2max = r_cut * r_cut * inv_ru2 + e2;
+  const bool table = kappa2 * r2max <= kTableU;
   Params pr;
   pr.csize = (float)cside;
   pr.rc2 = (float)(r_cut * r_cut);
-  pr.inv_rc2 = inv_rc2;
+  pr.inv_ru2 = (float)inv_ru2;
   pr.g = g * inv_ru2 * inv_ru;
   pr.eps2 = (float)e2;
   pr.kappa = (float)std::sqrt(kappa2);
   pr.e2 = (float)(kappa2 * 1.4426950408889634);
-  pr.tscale = (float)((kTable - 0.6) / (1.0 + e2));
+  pr.tscale = (float)((kTable - 0.6) / r2max);
   pr.nc = nc;
   pr.items = (unsigned)cap;
   const bool exact = kernel == GNG_SR_EXACT;
