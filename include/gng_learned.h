@@ -57,8 +57,10 @@ void gng_sr_destroy(gng_sr* sr);
 
 /* Device-resident short-range accelerations of all n particles (float32 SoA
  * device arrays), written (not added) to d_ax/d_ay/d_az on `stream`.
- * Requires box_size >= 3 r_cut.  Enqueued; nothing is synchronised (but a
- * first call, or one with more particles or cells, allocates). */
+ * Requires box_size >= 3 r_cut.  Any system of units: lengths are taken over
+ * r_cut and masses over the largest one (to a power of two), so only masses
+ * below 1e-38 of the largest lose digits.  Enqueued; nothing is synchronised
+ * (but a first call, or one with more particles or cells, allocates). */
 int gng_sr_accelerations(gng_sr* sr, const float* d_x, const float* d_y, const float* d_z, const float* d_m,
                          int64_t n, double box_size, double r_split, double r_cut, double eps2, double g,
                          int32_t kernel, float* d_ax, float* d_ay, float* d_az, void* stream);
