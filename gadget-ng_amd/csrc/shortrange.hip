@@ -55,6 +55,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <mutex>
 #include <new>
 #include <string>
 #include <type_traits>
@@ -418,6 +419,10 @@ struct gng_sr {
   Counters* d_count = nullptr;
   long long last_pairs = -1;
   bool pairs_pending = false;
+  std::mutex mu;
+  hipEvent_t done_ev = nullptr;  // end of the last call's work, on done_stream
+  hipStream_t done_stream = nullptr;
+  bool done_valid = false;
 };
 
 namespace {
@@ -433,7 +438,30 @@ void free_sr(gng_sr* s) {
   (void)hipFree(s->d_items);
   (void)hipFree(s->d_table);
   (void)hipFree(s->d_count);
+  if (s->done_ev) (void)hipEventDestroy(s->done_ev);
 }
+
+// Stream order for one call's work in the context's buffers: construction
+// makes s wait for the previous call's work when that ran on another stream,
+// destruction records the point the next call waits for.  Construct it under
+// the context's lock.  A stream that is being captured cannot wait for work
+// outside its graph: the caller orders the graph's launches.
+struct SrOrder {
+  gng_sr* sr;
+  hipStream_t s;
+  bool eager = true;
+  hipError_t e = hipSuccess;
+  SrOrder(gng_sr* sr_, hipStream_t s_) : sr(sr_), s(s_) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (s && hipStreamIsCapturing(s, &st) == hipSuccess) eager = st == hipStreamCaptureStatusNone;
+    if (eager && sr->done_valid && sr->done_stream != s) e = hipStreamWaitEvent(s, sr->done_ev, 0);
+  }
+  ~SrOrder() {
+    if (!eager || hipEventRecord(sr->done_ev, s) != hipSuccess) return;
+    sr->done_valid = true;
+    sr->done_stream = s;
+  }
+};
 
 }  // namespace
 
@@ -505,7 +533,8 @@ int gng_sr_create(int32_t device, gng_sr** out) {
   gng_sr* s = new (std::nothrow) gng_sr();
   if (!s) return fail(GNG_ERR_OOM, "host allocation failed");
   s->device = device;
-  if (hipMalloc(&s->d_count, sizeof(Counters)) != hipSuccess ||
+  if (hipEventCreateWithFlags(&s->done_ev, hipEventDisableTiming) != hipSuccess ||
+      hipMalloc(&s->d_count, sizeof(Counters)) != hipSuccess ||
       hipMalloc(&s->d_table, sizeof(float4) * (kTable + 1)) != hipSuccess) {
     free_sr(s);
     delete s;
@@ -530,8 +559,11 @@ int gng_sr_cell_order(gng_sr* sr, const float* d_x, const float* d_y, const floa
   if (int e = check_geometry(n, box_size, r_cut)) return e;
   if (n == 0) return GNG_OK;
   if (!d_x || !d_y || !d_z || !d_order) return fail(GNG_ERR_INVALID, "null array");
+  std::lock_guard<std::mutex> lk(sr->mu);
   GNG_HIP(hipSetDevice(sr->device));
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  SrOrder order(sr, s);
+  GNG_HIP(order.e);
   int nc = 0;
   if (int e = cell_sort(sr, d_x, d_y, d_z, n, box_size, r_cut, s, &nc)) return e;
   GNG_HIP(hipMemcpyAsync(d_order, sr->d_order, sizeof(unsigned) * (size_t)n, hipMemcpyDeviceToDevice, s));
@@ -547,8 +579,11 @@ int gng_sr_accelerations(gng_sr* sr, const float* d_x, const float* d_y, const f
   if (kernel != GNG_SR_EXACT && kernel != GNG_SR_REFERENCE) return fail(GNG_ERR_INVALID, "unknown split kernel");
   if (n == 0) return GNG_OK;
   if (!d_x || !d_y || !d_z || !d_m || !d_ax || !d_ay || !d_az) return fail(GNG_ERR_INVALID, "null array");
+  std::lock_guard<std::mutex> lk(sr->mu);
   GNG_HIP(hipSetDevice(sr->device));
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  SrOrder order(sr, s);
+  GNG_HIP(order.e);
   int nc = 0;
   if (int e = cell_sort(sr, d_x, d_y, d_z, n, box_size, r_cut, s, &nc)) return e;
   const long long ncell = (long long)nc * nc * nc;
@@ -607,6 +642,7 @@ int gng_sr_accelerations(gng_sr* sr, const float* d_x, const float* d_y, const f
 int64_t gng_sr_last_pair_count(const gng_sr* sr) {
   if (!sr) return -1;
   gng_sr* m = const_cast<gng_sr*>(sr);
+  std::lock_guard<std::mutex> lk(m->mu);
   if (m->pairs_pending) {
     unsigned long long v = 0;
     if (hipSetDevice(m->device) != hipSuccess || hipDeviceSynchronize() != hipSuccess ||

@@ -35,7 +35,7 @@
  * Training particles are two float4 arrays: pos4 = (x, y, z, box index) and
  * tgt4 = (target residual x, y, z, weight w_p); the loss is
  *   L = (1/n) sum_p w_p |out_scale * CIC(y)(x_p) - target_p|^2.
- * Every call on one object must be ordered (one stream, or synchronised).
+ * Every call on one network must be ordered (one stream, or synchronised).
  */
 #ifndef GNG_LEARNED_H
 #define GNG_LEARNED_H
@@ -59,8 +59,13 @@ void gng_sr_destroy(gng_sr* sr);
  * device arrays), written (not added) to d_ax/d_ay/d_az on `stream`.
  * Requires box_size >= 3 r_cut.  Any system of units: lengths are taken over
  * r_cut and masses over the largest one (to a power of two), so only masses
- * below 1e-38 of the largest lose digits.  Enqueued; nothing is synchronised
- * (but a first call, or one with more particles or cells, allocates). */
+ * below 1e-38 of the largest lose digits.
+ * Enqueued; nothing is synchronised (but a first call, or one with more
+ * particles or cells, allocates): the arrays must stay as they are until
+ * `stream` has done this work, so a caller that fills or frees them from
+ * elsewhere first waits for it.  Calls on one context may come from several
+ * streams and threads: each starts after the one before it (calls into a
+ * stream under capture excepted, whose graph the caller orders). */
 int gng_sr_accelerations(gng_sr* sr, const float* d_x, const float* d_y, const float* d_z, const float* d_m,
                          int64_t n, double box_size, double r_split, double r_cut, double eps2, double g,
                          int32_t kernel, float* d_ax, float* d_ay, float* d_az, void* stream);
