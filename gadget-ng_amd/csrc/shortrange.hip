@@ -71,6 +71,11 @@ constexpr int kChunk = 64;          // particles per work item: one wavefront
 constexpr unsigned kHeavy = 8192;   // particles in the 27 cells above which a chunk takes a workgroup
 constexpr int kAhead = 8;           // entries past the last particle that may be loaded (never used)
 
+// Workgroups per row of the force launch.  A launch dimension is cut, without
+// an error, at 2^32 work items, 2^24 of these workgroups, which 7e8 particles
+// can make.
+constexpr long long kRow = 1 << 16;
+
 // The unwrapped chaining-mesh cell floor(v nc / L) of one coordinate, in FP64
 // (cs = nc / L), and its index wrapped into [0, nc); a non-finite coordinate
 // lands in cell 0.  k_cells and k_gather both start from cell_floor, so a
@@ -264,15 +269,15 @@ __global__ __launch_bounds__(256) void k_force(const float4* __restrict__ sorted
   constexpr int kSums = 3 * 3 * kChunk;  // doubles: three wavefronts' sums of a heavy chunk
   __shared__ float4 tab[TABLE ? kTable + 1 : kSums / 2];
   static_assert(kSums / 2 <= kTable, "the sums reuse the table's LDS");
-  const unsigned heavy = cnt->heavy, light = cnt->light;
-  const bool whole = blockIdx.x < heavy;  // uniform: the workgroup is one heavy chunk
-  if (!whole && (blockIdx.x - heavy) * 4u >= light) return;
+  const unsigned heavy = cnt->heavy, light = cnt->light, group = blockIdx.y * gridDim.x + blockIdx.x;
+  const bool whole = group < heavy;  // uniform: the workgroup is one heavy chunk
+  if (!whole && (group - heavy) * 4u >= light) return;
   if constexpr (TABLE) {
     for (int e = threadIdx.x; e <= kTable; e += 256) tab[e] = table[e];
     __syncthreads();
   }
   const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const unsigned w = whole ? blockIdx.x : (blockIdx.x - heavy) * 4u + wave;
+  const unsigned w = whole ? group : (group - heavy) * 4u + wave;
   if (!whole && w >= light) return;
   const uint2 item = items[whole ? w : pr.items - 1u - w];
   const unsigned cell = __builtin_amdgcn_readfirstlane(item.x), i0 = off[cell] + item.y * kChunk;
@@ -632,8 +637,9 @@ int gng_sr_accelerations(gng_sr* sr, const float* d_x, const float* d_y, const f
   };
   const auto force = exact ? pick(std::integral_constant<int, GNG_SR_EXACT>())
                            : pick(std::integral_constant<int, GNG_SR_REFERENCE>());
-  hipLaunchKernelGGL(force, dim3((unsigned)(max_heavy(n) + (max_light(n, ncell) + 3) / 4)), dim3(256), 0, s,
-                     sr->d_sorted, sr->d_sidx, sr->d_off, sr->d_items, sr->d_table, pr, d_ax, d_ay, d_az, sr->d_count);
+  const long long groups = max_heavy(n) + (max_light(n, ncell) + 3) / 4;
+  hipLaunchKernelGGL(force, dim3((unsigned)std::min(groups, kRow), (unsigned)((groups + kRow - 1) / kRow)), dim3(256), 0,
+                     s, sr->d_sorted, sr->d_sidx, sr->d_off, sr->d_items, sr->d_table, pr, d_ax, d_ay, d_az, sr->d_count);
   GNG_HIP(hipGetLastError());
   sr->pairs_pending = true;
   return GNG_OK;
