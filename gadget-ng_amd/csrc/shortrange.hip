@@ -136,20 +136,31 @@ inline long long max_light(long long n, long long ncell) { return n / kChunk + (
 
 // The work items (cell, chunk): heavy ones' from the front of items, the
 // others' from its back.  One atomic per wavefront and kind; the places are
-// arbitrary, but no result depends on them.  The workgroups also look through
-// the n masses for the largest.
+// arbitrary, but no result depends on them.  The first workgroups also look
+// through the n masses for the largest: one atomic each, since all of them go
+// to one word, some 10 ns apart.
+constexpr unsigned kMassGroups = 256;
 __global__ __launch_bounds__(256) void k_items(const unsigned* __restrict__ off, int nc, long long ncell,
                                                const float* __restrict__ m, long long n, uint2* __restrict__ items,
                                                unsigned cap, Counters* __restrict__ cnt) {
-  unsigned top = 0, odd = 0;
-  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) {
-    const unsigned b = __float_as_uint(fabsf(m[i]));
-    if (b >= 0x7F800000u) odd = 1u;
-    else top = max(top, b);
+  if (blockIdx.x < kMassGroups) {
+    __shared__ unsigned tops[4];
+    unsigned top = 0, odd = 0;
+    const unsigned groups = min(gridDim.x, kMassGroups);
+    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += groups * 256LL) {
+      const unsigned b = __float_as_uint(fabsf(m[i]));
+      if (b >= 0x7F800000u) odd = 1u;
+      else top = max(top, b);
+    }
+    if (odd) cnt->odd = 1u;
+    for (int d = 32; d > 0; d >>= 1) top = max(top, __shfl_xor(top, d));
+    if ((threadIdx.x & 63) == 0) tops[threadIdx.x >> 6] = top;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      top = max(max(tops[0], tops[1]), max(tops[2], tops[3]));
+      if (top) atomicMax(&cnt->mmax, top);
+    }
   }
-  if (odd) cnt->odd = 1u;
-  for (int d = 32; d > 0; d >>= 1) top = max(top, __shfl_xor(top, d));
-  if ((threadIdx.x & 63) == 0 && top > __atomic_load_n(&cnt->mmax, __ATOMIC_RELAXED)) atomicMax(&cnt->mmax, top);
   const long long c = (long long)blockIdx.x * 256 + threadIdx.x;
   const int lane = threadIdx.x & 63;
   const unsigned k = c < ncell ? off[c + 1] - off[c] : 0u;
@@ -538,7 +549,7 @@ int gng_sr_create(int32_t device, gng_sr** out) {
   gng_sr* s = new (std::nothrow) gng_sr();
   if (!s) return fail(GNG_ERR_OOM, "host allocation failed");
   s->device = device;
-  if (hipEventCreateWithFlags(&s->done_ev, hipEventDisableTiming) != hipSuccess ||
+  if (hipEventCreateWithFlags(&s->done_ev, hipEventDisableTiming | hipEventDisableSystemFence) != hipSuccess ||
       hipMalloc(&s->d_count, sizeof(Counters)) != hipSuccess ||
       hipMalloc(&s->d_table, sizeof(float4) * (kTable + 1)) != hipSuccess) {
     free_sr(s);
@@ -606,7 +617,7 @@ int gng_sr_accelerations(gng_sr* sr, const float* d_x, const float* d_y, const f
   hipLaunchKernelGGL(k_offsets, dim3((unsigned)((ncell + 256) / 256)), dim3(256), 0, s, sr->d_cell_sorted, (unsigned)n,
                      ncell, sr->d_off, sr->d_count);
   // a workgroup for every 256 cells, and enough of them for the masses
-  const long long item_groups = std::max((ncell + 255) / 256, std::min<long long>((n + 2047) / 2048, 512));
+  const long long item_groups = std::max((ncell + 255) / 256, std::min<long long>((n + 2047) / 2048, kMassGroups));
   hipLaunchKernelGGL(k_items, dim3((unsigned)item_groups), dim3(256), 0, s, sr->d_off, nc, ncell, d_m, (long long)n,
                      sr->d_items, (unsigned)cap, sr->d_count);
   hipLaunchKernelGGL(k_gather, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, d_x, d_y, d_z, d_m, (long long)n,
