@@ -49,8 +49,11 @@
 // 17.0 ms with LDS-staged neighbours, that erfc and one workgroup per 256
 // particles; 13.3 with scalar neighbours and the table; 6.3 with heavy chunks
 // spread over four wavefronts (8.1 with the erfc formula there).
-// Beyond u = 16 (r_cut above 5.6 r_s) the table would be too coarse and the
-// device library's erfc is called.
+// Beyond u = 16 (r_cut above 5.6 r_s) a table uniform in r^2 would be too coarse
+// where F is steep, below u = 4; there it has 2049 entries uniform in r, for five
+// operations a pair more, and ends at the latest where F leaves FP32, at x = 9.3.
+// 2e5 particles at r_cut = 6 r_s: 1.64 ms with the device library's erfc in the
+// place of a table, 0.91 so (at 5.6 r_s 0.87).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -218,15 +221,16 @@ struct Params {
   float rc2;       // r_cut^2
   double g;        // G / r_u^2, taken into the sums with the masses' power of two
   float eps2;
-  float kappa;     // r_u / (sqrt(2) r_s): x = kappa r
-  float e2;        // kappa^2 log2(e): exp(-x^2) = exp2(-e2 r^2)
-  float tscale;    // table entries per unit of r^2
+  float tscale;    // table entries per unit of r^2, or of r
   int nc;
   unsigned items;  // capacity of the work list
 };
 
-constexpr int kTable = 1024;  // entries 0 .. kTable, entry i around r^2 = i / tscale
-constexpr double kTableU = 16.0;
+// Entries 0 .. kTable, entry i around r^2 = i / tscale up to u = kTableU, else
+// around r = i / tscale, and the last one, 0, for all r from kWideX on.
+template <bool WIDE>
+constexpr int kTable = WIDE ? 2048 : 1024;
+constexpr double kTableU = 16.0, kWideX = 9.3;
 // where the law passes from the subtraction to F: the subtraction loses 1 / S of
 // a rounding (4 at u = 2 for the exact split; erfc falls faster: 9 at 1.25, 22
 // at 2), the quadratics of F get worse as u^-3 (6e-8 at 1.25 with u to 12.5)
@@ -253,16 +257,23 @@ __device__ double smooth_part(double v, double kappa2, bool near) {
   return S / (v * sqrt(v));
 }
 
-// Entry i: c0 + d (c1 + d c2) with d = r^2 tscale - i in [-1/2, 1/2], through
-// the Chebyshev nodes of that interval, and 1 where the entry is near, else 0.
-template <int KERNEL>
+// Entry i: c0 + d (c1 + d c2) with d = r^2 tscale - i (WIDE: r tscale - i) in
+// [-1/2, 1/2], through the Chebyshev nodes of that interval, and 1 where the
+// entry is near, else 0.
+template <int KERNEL, bool WIDE>
 __global__ __launch_bounds__(256) void k_table(double kappa2, double tscale, float4* __restrict__ table) {
   const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i > kTable) return;
+  if (i > kTable<WIDE>) return;
   const double c = (double)i / tscale, d0 = 0.43301270189221932;  // sqrt(3) / 4
-  const bool near = kappa2 * c < kNearU<KERNEL>;
-  const double f0 = smooth_part<KERNEL>(c, kappa2, near), fp = smooth_part<KERNEL>(c + d0 / tscale, kappa2, near),
-               fm = smooth_part<KERNEL>(c - d0 / tscale, kappa2, near);
+  const auto square = [](double t) { return WIDE ? t * t : t; };
+  const bool near = kappa2 * square(c) < kNearU<KERNEL>;
+  const double f0 = smooth_part<KERNEL>(square(c), kappa2, near),
+               fp = smooth_part<KERNEL>(square(c + d0 / tscale), kappa2, near),
+               fm = smooth_part<KERNEL>(square(c - d0 / tscale), kappa2, near);
+  if (WIDE && i == kTable<WIDE>) {
+    table[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    return;
+  }
   table[i] = make_float4((float)f0, (float)((fp - fm) / (2.0 * d0)), (float)((fp + fm - 2.0 * f0) / (2.0 * d0 * d0)),
                          near ? 1.0f : 0.0f);
 }
@@ -271,22 +282,20 @@ __global__ __launch_bounds__(256) void k_table(double kappa2, double tscale, flo
 // below 1e18, so that its zero displacement alone makes it vanish, unless a
 // mass is not finite.  The comparison this saves is 4 % of the kernel (96^3
 // clustered particles: 6.78 against 6.46 ms).
-template <int KERNEL, bool TABLE, bool SOFT>
+template <int KERNEL, bool WIDE, bool SOFT>
 __global__ __launch_bounds__(256) void k_force(const float4* __restrict__ sorted, const unsigned* __restrict__ sidx,
                                                const unsigned* __restrict__ off, const uint2* __restrict__ items,
                                                const float4* __restrict__ table, const Params pr,
                                                float* __restrict__ ax, float* __restrict__ ay, float* __restrict__ az,
                                                Counters* __restrict__ cnt) {
   constexpr int kSums = 3 * 3 * kChunk;  // doubles: three wavefronts' sums of a heavy chunk
-  __shared__ float4 tab[TABLE ? kTable + 1 : kSums / 2];
-  static_assert(kSums / 2 <= kTable, "the sums reuse the table's LDS");
+  __shared__ float4 tab[kTable<WIDE> + 1];
+  static_assert(kSums / 2 <= kTable<WIDE>, "the sums reuse the table's LDS");
   const unsigned heavy = cnt->heavy, light = cnt->light, group = blockIdx.y * gridDim.x + blockIdx.x;
   const bool whole = group < heavy;  // uniform: the workgroup is one heavy chunk
   if (!whole && (group - heavy) * 4u >= light) return;
-  if constexpr (TABLE) {
-    for (int e = threadIdx.x; e <= kTable; e += 256) tab[e] = table[e];
-    __syncthreads();
-  }
+  for (int e = threadIdx.x; e <= kTable<WIDE>; e += 256) tab[e] = table[e];
+  __syncthreads();
   const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const unsigned w = whole ? group : (group - heavy) * 4u + wave;
   if (!whole && w >= light) return;
@@ -331,23 +340,22 @@ __global__ __launch_bounds__(256) void k_force(const float4* __restrict__ sorted
         if (r2b <= pr.rc2 && (decltype(keep)::value || r2b > 0.0f)) {
           const float r2 = r2b + pr.eps2;
           const float rinv = __builtin_amdgcn_rsqf(r2);
-          float f;
-          if constexpr (TABLE) {
-            // adding 1.5 * 2^23 leaves rint(t) in the low mantissa bits
-            const float tb = fmaf(r2, pr.tscale, 12582912.0f);
-            const float d = fmaf(r2, pr.tscale, -(tb - 12582912.0f));
-            const float4 q = tab[__float_as_uint(tb) - 0x4B400000u];
-            const float smooth = fmaf(d, fmaf(d, q.z, q.y), q.x);
-            if constexpr (KERNEL == GNG_SR_EXACT)
-              f = fmaf(q.w, rinv * rinv * rinv, smooth);
-            else
-              f = q.w != 0.0f ? rinv * rinv * (rinv - smooth) : smooth;
-          } else {
-            const float x = r2 * rinv * pr.kappa;
-            const float S = erfcf(x) + (KERNEL == GNG_SR_EXACT
-                                            ? 1.1283791670955126f * x * __builtin_amdgcn_exp2f(-r2 * pr.e2) : 0.0f);
-            f = S * (rinv * rinv * rinv);
+          float at = r2;
+          if constexpr (WIDE) {
+            at = r2 * rinv;
+            at = fmaf(fmaf(-at, at, r2), 0.5f * rinv, at);  // rsq's last bits count 2 u times in F
           }
+          // adding 1.5 * 2^23 leaves rint(t) in the low mantissa bits
+          float tb = fmaf(at, pr.tscale, 12582912.0f);
+          if constexpr (WIDE) tb = fminf(tb, 12582912.0f + (float)kTable<WIDE>);
+          const float d = fmaf(at, pr.tscale, -(tb - 12582912.0f));
+          const float4 q = tab[__float_as_uint(tb) - 0x4B400000u];
+          const float smooth = fmaf(d, fmaf(d, q.z, q.y), q.x);
+          float f;
+          if constexpr (KERNEL == GNG_SR_EXACT)
+            f = fmaf(q.w, rinv * rinv * rinv, smooth);
+          else
+            f = q.w != 0.0f ? rinv * rinv * (rinv - smooth) : smooth;
           f *= pj.w;
           fx += f * dx;
           fy += f * dy;
@@ -551,7 +559,7 @@ int gng_sr_create(int32_t device, gng_sr** out) {
   s->device = device;
   if (hipEventCreateWithFlags(&s->done_ev, hipEventDisableTiming | hipEventDisableSystemFence) != hipSuccess ||
       hipMalloc(&s->d_count, sizeof(Counters)) != hipSuccess ||
-      hipMalloc(&s->d_table, sizeof(float4) * (kTable + 1)) != hipSuccess) {
+      hipMalloc(&s->d_table, sizeof(float4) * (kTable<true> + 1)) != hipSuccess) {
     free_sr(s);
     delete s;
     return fail(GNG_ERR_OOM, "short-range counters");
@@ -625,32 +633,32 @@ int gng_sr_accelerations(gng_sr* sr, const float* d_x, const float* d_y, const f
   const double rc = r_cut * inv_ru, rs = r_split * inv_ru, kappa2 = 0.5 / (rs * rs), e2 = eps2 * inv_ru * inv_ru;
   // the table covers r^2 <= r_cut^2 + eps^2, with room for rounding at its end
   const double r2max = rc * rc + e2;
-  const bool table = kappa2 * r2max <= kTableU;
+  const bool wide = kappa2 * r2max > kTableU;
+  const double tend = wide ? std::min(std::sqrt(r2max), kWideX / std::sqrt(kappa2)) : r2max;
   Params pr;
   pr.csize = (float)(cside * inv_ru);
   pr.rc2 = (float)(rc * rc);
   pr.g = g * inv_ru * inv_ru;
   pr.eps2 = (float)e2;
-  pr.kappa = (float)std::sqrt(kappa2);
-  pr.e2 = (float)(kappa2 * 1.4426950408889634);
-  pr.tscale = (float)((kTable - 0.6) / r2max);
+  pr.tscale = (float)std::min(((wide ? kTable<true> : kTable<false>) - 0.6) / tend, 1e30);  // finite however small r_s is
   pr.nc = nc;
   pr.items = (unsigned)cap;
-  const bool exact = kernel == GNG_SR_EXACT;
-  if (table)
-    hipLaunchKernelGGL(exact ? k_table<GNG_SR_EXACT> : k_table<GNG_SR_REFERENCE>, dim3((kTable + 256) / 256), dim3(256),
-                       0, s, kappa2, (double)pr.tscale, sr->d_table);
   // 1 / r^3 stays below 1e18
   const bool soft = e2 >= 1e-12;
-  const auto pick = [&](auto k) {
+  const auto launch = [&](auto k, auto w) {
     constexpr int K = decltype(k)::value;
-    return table ? (soft ? k_force<K, true, true> : k_force<K, true, false>) : k_force<K, false, false>;
+    constexpr bool W = decltype(w)::value;
+    hipLaunchKernelGGL((k_table<K, W>), dim3((kTable<W> + 256) / 256), dim3(256), 0, s, kappa2, (double)pr.tscale,
+                       sr->d_table);
+    const long long groups = max_heavy(n) + (max_light(n, ncell) + 3) / 4;
+    const dim3 grid((unsigned)std::min(groups, kRow), (unsigned)((groups + kRow - 1) / kRow));
+    const auto force = soft ? k_force<K, W, true> : k_force<K, W, false>;
+    hipLaunchKernelGGL(force, grid, dim3(256), 0, s, sr->d_sorted, sr->d_sidx, sr->d_off, sr->d_items, sr->d_table, pr,
+                       d_ax, d_ay, d_az, sr->d_count);
   };
-  const auto force = exact ? pick(std::integral_constant<int, GNG_SR_EXACT>())
-                           : pick(std::integral_constant<int, GNG_SR_REFERENCE>());
-  const long long groups = max_heavy(n) + (max_light(n, ncell) + 3) / 4;
-  hipLaunchKernelGGL(force, dim3((unsigned)std::min(groups, kRow), (unsigned)((groups + kRow - 1) / kRow)), dim3(256), 0,
-                     s, sr->d_sorted, sr->d_sidx, sr->d_off, sr->d_items, sr->d_table, pr, d_ax, d_ay, d_az, sr->d_count);
+  const auto with_width = [&](auto k) { wide ? launch(k, std::true_type()) : launch(k, std::false_type()); };
+  if (kernel == GNG_SR_EXACT) with_width(std::integral_constant<int, GNG_SR_EXACT>());
+  else with_width(std::integral_constant<int, GNG_SR_REFERENCE>());
   GNG_HIP(hipGetLastError());
   sr->pairs_pending = true;
   return GNG_OK;

@@ -74,3 +74,33 @@ def test_smallest_sets(sr, n):
     got = sr.accelerations(pos, np.ones(n), 9.0, 0.6, 3.0, eps2=0.01)
     ref = lo.short_range_direct(pos, np.ones(n), 9.0, 0.6, 3.0, eps2=0.01)
     assert np.abs(got - ref).max() <= 1e-5 * max(np.abs(ref).max(), 1e-30)
+
+
+@pytest.mark.parametrize("kernel", ["exact", "reference"])
+@pytest.mark.parametrize("ratio", [5.66, 8.0, 13.0, 13.3, 30.0, 1e12])
+@pytest.mark.parametrize("eps", [0.0, 0.05])
+def test_pair_law_far_beyond_the_split(sr, kernel, ratio, eps):
+    """r_cut of many r_s, to past the end of the table (x = 9.3, r_cut = 13.2
+    r_s): a set with separations down to 0.1 r_s, and one whose pairs all lie
+    in the tail.  There a relative error e of r counts 2 x^2 times: below
+    2 * 30 * 2^-23, half of it for r^2 itself, at x^2 < 30."""
+    print(f"case far pair law kernel={kernel} ratio={ratio} eps={eps}", flush=True)
+    g = np.random.default_rng(int(min(ratio, 1e3) * 10))
+    box, rc = 12.0, 3.0
+    rs = rc / ratio
+    pos = g.uniform(0.0, box, (500, 3))
+    pos[:200] = 6.0 + 0.5 * min(rs, 0.5) * g.normal(size=(200, 3))
+    pos = pos.astype(np.float32).astype(np.float64)
+    m = g.uniform(0.5, 1.5, 500).astype(np.float32).astype(np.float64)
+    got = sr.accelerations(pos, m, box, rs, rc, eps2=(eps * rs) ** 2, kernel=kernel)
+    assert np.isfinite(got).all()
+    if ratio < 100.0:  # (beyond, FP32 positions do not resolve r_s)
+        ref = lo.short_range_direct(pos, m, box, rs, rc, eps2=(eps * rs) ** 2, kernel=kernel)
+        assert rms_rel(got, ref) < 1e-5
+    d = 2.0 ** 0.5 * 5.4 * rs  # x = 5.4
+    pairs = np.array([[1.0, 1.0, 1.0], [7.0, 7.0, 7.0]])
+    pairs = np.concatenate([pairs, pairs + [d, 0.0, 0.0]]).astype(np.float32).astype(np.float64)
+    if 5.66 < ratio < 100.0:
+        got = sr.accelerations(pairs, np.ones(4), box, rs, rc, eps2=(eps * rs) ** 2, kernel=kernel)
+        ref = lo.short_range_direct(pairs, np.ones(4), box, rs, rc, eps2=(eps * rs) ** 2, kernel=kernel)
+        assert rms_rel(got / np.abs(ref).max(), ref / np.abs(ref).max()) < 2.0 * 30.0 * 2.0 ** -23 * 1.5
