@@ -2172,6 +2172,9 @@ int autotune_impl(gng_pm_plan* p, const PartIn& in, long long n, const AccOut& o
     if (k == 7 && !p->ops->has_narrow_y_inv) continue;  // one tile width compiled
     // the plane kernels have one form of every pass
     if (p->ops->plane_fwd && (k == 0 || (k >= 2 && k <= 5))) continue;
+    // and the sort-free deposit none of the sorted one's (their timings would
+    // differ by noise alone, and the choice holds for larger solves too)
+    if (small_deposit(p, n) && (k == 1 || k == 6 || k == 8)) continue;
     Tuning trial = best;
     if (k == 4 || k == 5) {
       // chunked or whole-mesh pass pairs
