@@ -153,9 +153,12 @@ int& knob(Tuning& t, int k) {
 }
 
 // Process-wide cache of measured choices, keyed by (device architecture, nm).
-// When GNG_PM_TUNE_FILE names a file, it is read once (per line: arch, nm and
-// the kKnobs knobs in knob() order) and rewritten after every new measurement,
-// so later processes reuse the decisions.
+// When GNG_PM_TUNE_FILE names a file, it is read once (a first line of
+// kTuneFormat, then per line: arch, nm and the kKnobs knobs in knob() order) and
+// rewritten after every new measurement, so later processes reuse the decisions.
+// A file with another first line holds measurements of other kernels and is
+// not read; the number goes up when what a knob selects changes.
+constexpr const char* kTuneFormat = "gng_pm_tuning_2";
 std::mutex g_tune_mu;
 std::map<std::pair<std::string, int>, Tuning> g_tune;
 bool g_tune_loaded = false;
@@ -176,6 +179,10 @@ void load_tune_file_locked() {
   if (!fp) return;
   char arch[64];
   int nm, v[kKnobs];
+  if (std::fscanf(fp, "%63s", arch) != 1 || std::strcmp(arch, kTuneFormat) != 0) {
+    std::fclose(fp);
+    return;
+  }
   while (std::fscanf(fp, "%63s %d %d %d %d %d %d %d %d %d %d", arch, &nm, &v[0], &v[1], &v[2], &v[3], &v[4], &v[5],
                      &v[6], &v[7], &v[8]) == 2 + kKnobs) {
     Tuning t;
@@ -206,6 +213,7 @@ void store_tuning(int dev, int nm, const Tuning& t) {
   if (!f || !*f) return;
   FILE* fp = std::fopen(f, "w");
   if (!fp) return;
+  std::fprintf(fp, "%s\n", kTuneFormat);
   for (const auto& kv : g_tune)
     std::fprintf(fp, "%s %d %d %d %d %d %d %d %d %d %d\n", kv.first.first.c_str(), kv.first.second,
                  kv.second.z_persistent, kv.second.deposit_wide, kv.second.y_fwd_persistent,

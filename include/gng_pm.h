@@ -213,7 +213,8 @@ int gng_pm_force_meshes(gng_pm_plan *p, float *out);
  * a time from the defaults and keeps each flip that is faster.  The result
  * applies to this plan and to plans created later in the process with the
  * same device architecture and mesh side; with GNG_PM_TUNE_FILE set it is also
- * read from and written to that file.  Untuned plans use the persistent z pass
+ * read from and written to that file.  (A file written by a library whose choices
+ * select other kernels is not read.)  Untuned plans use the persistent z pass
  * at nm = 512 only, the 512-thread deposit only below 256 tiles, and two
  * tiles per deposit workgroup from nm = 1024 on.  Up to nm = 128 the force
  * solve transforms whole z planes in one kernel each way; the choices of its x,

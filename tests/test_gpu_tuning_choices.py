@@ -1,10 +1,16 @@
 """The autotuner keeps its defaults where the variants run the same work (the
 deposit of a small problem does not sort, so the sorted deposit's choices do
-nothing there)."""
+nothing there), and a tuning file is read only if it was written for the
+kernels that its choices select."""
+import os
+import subprocess
+import sys
+
 import pytest
 
 pytestmark = pytest.mark.gpu
 
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 DEPOSIT = ("deposit_threads", "deposit_split", "deposit_pair")
 
 
@@ -16,3 +22,42 @@ def test_deposit_choices_of_small_meshes_stay(pm, nm):
     for _ in range(12):
         got = plan.autotune(reps=1)
         assert got["tuned"] and {k: got[k] for k in DEPOSIT} == default
+
+
+SCRIPT = """
+import sys
+sys.path.insert(0, {pkg!r})
+import gadget_ng_pm_hip as pm
+t = pm.Plan(64, 1.0).tuning()
+if {measure!r}:
+    t = pm.Plan(64, 1.0).autotune(reps=1)
+print("TUNING", t["tuned"], t["deposit_threads"], t["deposit_pair"], flush=True)
+"""
+
+
+def in_a_process(path, measure=False):
+    """The tuning of a plan in a process with that tuning file."""
+    env = dict(os.environ, GNG_PM_TUNE_FILE=str(path))
+    code = SCRIPT.format(pkg=os.path.join(ROOT, "gadget-ng_amd"), measure=measure)
+    r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr
+    return next(line for line in r.stdout.splitlines() if line.startswith("TUNING")).split()[1:]
+
+
+def test_tuning_files_of_other_kernels_are_not_read(pm, tmp_path):
+    print("case tuning file", flush=True)
+    line = "gfx950 64 0 0 0 0 0 0 1 1 1\n"  # 256 threads and two tiles, unlike the default
+    default = ["False", "512", "False"]
+    old = tmp_path / "old"
+    old.write_text(line)
+    assert in_a_process(old) == default
+    (tmp_path / "other").write_text("gng_pm_tuning_1\n" + line)
+    assert in_a_process(tmp_path / "other") == default
+    (tmp_path / "empty").write_text("")
+    assert in_a_process(tmp_path / "empty") == default
+    (tmp_path / "new").write_text("gng_pm_tuning_2\n" + line)
+    assert in_a_process(tmp_path / "new") == ["True", "256", "True"]
+    # what one process measures, the next one reads
+    assert in_a_process(old, measure=True)[0] == "True"
+    assert old.read_text().startswith("gng_pm_tuning_2\n")
+    assert in_a_process(old)[0] == "True"
