@@ -642,7 +642,7 @@ struct gng_pm_plan {
   double* d_ic_sigma = nullptr;
   long long ic_sigma_cap = 0;
   float* d_ic_mask = nullptr;  // 1 per axis index, 0 at the Nyquist index (second order)
-  float2* d_ic_mesh[3] = {};   // meshes of the second order beside P, A, B (allocated on its first use)
+  float2* d_ic_mesh[3] = {};   // meshes of the second order beside P, A, B (IcMeshes)
   // Stage timing: every solve records kStages+1 events into the next slot of
   // a ring; nothing synchronises until gng_pm_stage_times() reads them.
   bool timing = false;
@@ -1572,6 +1572,31 @@ int run_ic(gng_pm_plan* p, const IcParams& ip, double vel_factor, double scale, 
   return GNG_OK;
 }
 
+// The second order's three further meshes (each half the complex mesh): all of
+// them or, with e set, none.  Up to kIcKeepBytes in all, 512^3, the plan
+// keeps them, since taking and freeing them costs a call of 1.43 ms at 256^3
+// 0.55 ms and one of 12.8 ms at 512^3 1.1 ms.  Larger ones, 12.9 GB at 1024^3,
+// go back when the call ends (2 of 118 ms): a plan that goes on to force solves
+// does not hold them.  Destroyed after the stream was waited for.
+constexpr size_t kIcKeepBytes = 2ull << 30;
+struct IcMeshes {
+  gng_pm_plan* p;
+  size_t each;
+  hipError_t e = hipSuccess;
+  explicit IcMeshes(gng_pm_plan* p_)
+      : p(p_), each(sizeof(float2) * (size_t)p_->cfg.grid_size * (size_t)mesh_plane(p_->cfg.grid_size)) {
+    for (float2*& m : p->d_ic_mesh)
+      if (!m && e == hipSuccess) e = hipMalloc(&m, each);
+  }
+  ~IcMeshes() {
+    if (e == hipSuccess && 3 * each <= kIcKeepBytes) return;
+    for (float2*& m : p->d_ic_mesh) {
+      (void)hipFree(m);
+      m = nullptr;
+    }
+  }
+};
+
 // Second-order (2LPT) particles (ic_2lpt.rs:348-553): the six second
 // derivatives of phi in two rounds of three fields through the z, y and x
 // passes with mode multipliers (round 0: xx yy zz, round 1: xz yz xy),
@@ -1601,8 +1626,11 @@ int run_ic_2lpt(gng_pm_plan* p, const IcParams& ip, double vel1, double vel2, do
       return fail(GNG_ERR_HIP, std::string("2LPT mask upload: ") + hipGetErrorString(e));
     }
   }
-  for (float2*& m : p->d_ic_mesh)
-    if (!m) GNG_HIP(hipMalloc(&m, sizeof(float2) * (size_t)nm * (size_t)mesh_plane(nm)));
+  IcMeshes meshes(p);
+  if (meshes.e != hipSuccess) {
+    (void)hipGetLastError();
+    return fail(GNG_ERR_OOM, std::string("2LPT meshes: ") + hipGetErrorString(meshes.e));
+  }
   float2 *modes = p->d_ic_mesh[0], *a1 = p->d_ic_mesh[1], *b1 = p->d_ic_mesh[2];
   float* S = reinterpret_cast<float*>(a1);  // the source, an unpadded real mesh
   p->density_valid = false;

@@ -64,13 +64,15 @@ int gng_ic_zeldovich_device(gng_pm_plan *p, uint64_t seed, const double *sigma, 
  *   vel = Psi1 vel1 + Psi2 vel2,
  * as (hi - lo) x 3 interleaved f64 in host memory.  vel1 = a^2 f1 H,
  * vel2 = a^2 f2 H d2_over_d1sq, d2_over_d1sq = -3/7 Omega_m(a)^(-1/143)
- * (:414-443), s the optional rescaling D(a_init) / D(1).  Needs one extra
- * n^3 f32 buffer while it runs. */
+ * (:414-443), s the optional rescaling D(a_init) / D(1).  Needs
+ * three further meshes of the plan's size (12 bytes a cell, 1.6 GB at 512^3)
+ * while it runs; up to 2 GiB of them stay with the plan for its next such call,
+ * more are freed before it returns. */
 int gng_ic_2lpt(gng_pm_plan *p, uint64_t seed, const double *sigma, int64_t sigma_len, double vel1, double vel2,
                 double d2_over_d1sq, double scale, int64_t lo, int64_t hi, double *pos, double *vel);
 
 /* Same into device memory, enqueued on `stream`; returns after the work
- * completes (the source buffer is freed). */
+ * completes. */
 int gng_ic_2lpt_device(gng_pm_plan *p, uint64_t seed, const double *sigma, int64_t sigma_len, double vel1,
                        double vel2, double d2_over_d1sq, double scale, int64_t lo, int64_t hi, double *d_pos,
                        double *d_vel, void *stream);

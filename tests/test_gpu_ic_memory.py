@@ -1,0 +1,66 @@
+"""What the second-order initial conditions leave allocated: nothing of the
+large meshes' workspace once the call has returned, nothing at all when the
+workspace does not fit, and then the plan still works."""
+import ctypes
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def free_bytes(pm):
+    pm.device_synchronize()
+    with open("/proc/self/maps") as f:
+        hip = ctypes.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
+
+    def get():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    return get
+
+
+def spectrum(n):
+    return lambda k: 0.05 * n ** 3 / max(k, 1.0)
+
+
+def test_large_meshes_are_given_back(pm, free_bytes):
+    from gadget_ng_pm_hip import ic
+    n = 1024
+    print(f"case 2lpt memory n={n}", flush=True)
+    plan = pm.Plan(n, 100.0)
+    ic.zeldovich_ics(plan, 3, spectrum(n), lo=0, hi=1000)  # the amplitude table
+    before = free_bytes()
+    pos = ic.zeldovich_2lpt_ics(plan, 3, spectrum(n), lo=0, hi=1000)[0]
+    assert np.isfinite(pos).all()
+    assert before - free_bytes() < 256 << 20  # (a mesh is 4.3 GB)
+
+
+def test_a_workspace_that_does_not_fit_leaves_nothing_behind(pm, free_bytes):
+    from gadget_ng_pm_hip import ic
+    n = 512
+    print(f"case 2lpt without memory n={n}", flush=True)
+    plan = pm.Plan(n, 100.0)
+    ic.zeldovich_ics(plan, 3, spectrum(n), lo=0, hi=1000)
+    mesh = 4 * n ** 3
+    hogs = [pm.DeviceArray((free_bytes() - 4 * mesh,), np.uint8)]
+    try:
+        for _ in range(32):
+            hogs.append(pm.DeviceArray((mesh,), np.uint8))
+    except pm.HipExecutionError:
+        pass
+    assert 3 < len(hogs) < 33
+    for h in hogs[-2:]:  # room for two of the three meshes
+        h.free()
+    before = free_bytes()
+    with pytest.raises(Exception):
+        ic.zeldovich_2lpt_ics(plan, 3, spectrum(n), lo=0, hi=1000)
+    assert before - free_bytes() < 64 << 20
+    for h in hogs:
+        h.free()
+    got = ic.zeldovich_2lpt_ics(plan, 3, spectrum(n), lo=0, hi=1000)
+    ref = ic.zeldovich_2lpt_ics(pm.Plan(n, 100.0), 3, spectrum(n), lo=0, hi=1000)
+    assert np.array_equal(got[0], ref[0]) and np.array_equal(got[1], ref[1])
