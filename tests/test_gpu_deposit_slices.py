@@ -37,6 +37,30 @@ def test_slices_at_their_limits(pm, oracle_mod, nm, count, corner, threads, pair
     assert np.abs(d0 - ref).max() <= 2.0 ** -24 * ref.max() * 1.01
 
 
+@pytest.mark.parametrize("threads,pair", [(256, False), (512, False), (256, True), (512, True)])
+def test_more_slices_wanted_than_there_are(pm, oracle_mod, threads, pair):
+    """Every particle in the cells just below a tile corner feeds eight tiles:
+    they want 8 * 6 = 48 slices of 8192 particles and there are
+    (2 * 40963 // 8192 + 16) & ~7 = 24, so some run whole beside the sliced
+    ones, in whatever order they ask."""
+    nm, count = 48, 5 * ITEMS + 3
+    print(f"case slices spent threads={threads} pair={pair}", flush=True)
+    rng = np.random.default_rng(7)
+    pos = rng.uniform(15.0, 16.0, (count, 3))
+    mass = rng.uniform(0.5, 1.5, count).astype(np.float32).astype(np.float64)
+    plan = pm.Plan(nm, float(nm), keep_density=True)
+    plan.set_tuning(deposit_threads=threads, deposit_pair=pair, deposit_split=False)
+    a0 = plan.accelerations_f64(pos, mass, 1.0)
+    d0 = plan.density()
+    plan.set_tuning(deposit_threads=threads, deposit_pair=pair, deposit_split=True)
+    for _ in range(3):
+        a1 = plan.accelerations_f64(pos, mass, 1.0)
+        assert np.array_equal(plan.density(), d0)
+        assert np.array_equal(a1, a0)
+    ref = oracle_mod.cic_assign(pos, mass, float(nm), nm).reshape(nm, nm, nm)
+    assert np.abs(d0 - ref).max() <= 2.0 ** -24 * ref.max() * 1.01
+
+
 @pytest.mark.parametrize("nm,count", [(16, 32768), (16, 32769), (48, 3 * 32768 + 5)])
 def test_moments_of_heavy_tiles(pm, nm, count):
     """Cell moments at and past the slice length, twice (the cleared words and
