@@ -861,7 +861,7 @@ int ensure_work(gng_pm_plan* p, long long n) {
   GNG_HIP(hipMalloc(&p->d_bucket, sizeof(unsigned) * m));
   GNG_HIP(hipMalloc(&p->d_rank, sizeof(unsigned) * m));
   // split deposit: slice workgroups, and half as many scratch tiles
-  const long long slots = deposit_slots(n, slice_items(n));
+  const long long slots = 2LL * deposit_slots(n, slice_items(n));
   const size_t t3 = (size_t)p->tm.T * p->tm.T * p->tm.T, tiles = (size_t)slots / 2;
   GNG_HIP(hipMalloc(&p->d_extra, sizeof(unsigned) * (size_t)slots));
   GNG_HIP(hipMalloc(&p->d_split_scratch, sizeof(unsigned long long) * t3 * tiles));
@@ -898,12 +898,13 @@ void run_sort(gng_pm_plan* p, const PartIn& in, long long n, unsigned* perm, boo
 }
 
 // The slices of a pass over the sorted records of n particles (none without
-// the work buffers for them), each `longer` times the deposit's length.
-DepositSplit deposit_split(const gng_pm_plan* p, long long n, unsigned longer = 1) {
+// the work buffers for them): the deposit's, or the moments' (four times as
+// long, and each particle in one tile only).
+DepositSplit slices_for(const gng_pm_plan* p, long long n, bool moments) {
   DepositSplit sp{};
   if (p->split_slots > 0) {
-    sp.items = slice_items(n) * longer;
-    sp.slots = std::min<unsigned>((unsigned)p->split_slots, deposit_slots(n, sp.items));
+    sp.items = slice_items(n) * (moments ? 4u : 1u);
+    sp.slots = deposit_slots(n, sp.items) * (moments ? 1u : 2u);
     sp.extra = p->d_extra;
     sp.scratch = p->d_split_scratch;
     sp.done = p->d_split_done;
@@ -963,7 +964,7 @@ int run_front(gng_pm_plan* p, const PartIn& in, long long n, hipStream_t s) {
     run_sort(p, in, n, p->tune.interp_sorted ? p->d_perm : nullptr, true, s);
     mark(p, 2, s);
     const unsigned ntiles = (unsigned)p->tm.nt * p->tm.nt * p->tm.nt;
-    const DepositSplit sp = p->tune.deposit_split ? deposit_split(p, n) : DepositSplit{};
+    const DepositSplit sp = p->tune.deposit_split ? slices_for(p, n, false) : DepositSplit{};
     hipLaunchKernelGGL(k_tile_ranges, dim3((ntiles + 255) / 256), dim3(256), 0, s, p->d_offset, p->tm, p->d_sc, n, sp);
     const int pair = p->tune.deposit_pair != 0;
     o.deposit[p->tune.deposit_wide][pair](dim3(sp.slots + xcd_grid(pair ? (ntiles + 1u) / 2u : ntiles)),
@@ -2371,7 +2372,7 @@ int gng_pm_cell_moments(gng_pm_plan* p, double* d_mom, void* stream) {
   // slices four times the deposit's: each ends with up to 20480 global atomics
   // (256^3 clustered: 708 / 556 / 536 / 534 us at 1, 2, 3 and 5 times)
   p->ops->cell_moments(ntiles, s, p->d_sorted, p->d_offset, cell_map(p), p->tm, p->d_sc, p->sorted_n,
-                       deposit_split(p, p->sorted_n, 4), d_mom);
+                       slices_for(p, p->sorted_n, true), d_mom);
   GNG_HIP(hipGetLastError());
   return GNG_OK;
 }

@@ -169,12 +169,13 @@ constexpr int kQSlots = 64;
 constexpr int kQStride = 16;  // 64-bit words between slots
 struct SolveScalars {
   unsigned int mmax_bits;  // max |m| as float bits (non-negative floats order as integers)
-  unsigned int split_budget;  // scratch tiles reserved by split deposit tiles
+  unsigned int split_budget;  // slices asked for by the deposit's heavy tiles (k_tile_ranges)
   long long qmean;            // integer part of the mean fixed-point mass per cell (k_tile_ranges)
   int shift;                  // fixed_shift, once the scatter is done (k_tile_ranges)
   unsigned int moment_budget; // slices reserved by the moments' heavy tiles (k_moments_plan)
   unsigned int plain;         // records in the caller's order (k_deposit_small: their number); 0: sorted
-  unsigned int pad[57];
+  unsigned int split_rest;    // slices taken from the second half of the table (k_tile_ranges)
+  unsigned int pad[56];
   unsigned long long qsum[kQSlots * kQStride];
 };
 
@@ -225,6 +226,7 @@ __device__ __forceinline__ void reset_scalars_body(SolveScalars* sc) {
   if (threadIdx.x == 0) {
     sc->mmax_bits = 0u;
     sc->split_budget = 0u;
+    sc->split_rest = 0u;
     sc->plain = 0u;
   }
   if (threadIdx.x < kQSlots) sc->qsum[threadIdx.x * kQStride] = 0ull;

@@ -38,15 +38,18 @@ def test_slices_at_their_limits(pm, oracle_mod, nm, count, corner, threads, pair
 
 
 @pytest.mark.parametrize("threads,pair", [(256, False), (512, False), (256, True), (512, True)])
-def test_more_slices_wanted_than_there_are(pm, oracle_mod, threads, pair):
-    """Every particle in the cells just below a tile corner feeds eight tiles:
-    they want 8 * 6 = 48 slices of 8192 particles and there are
-    (2 * 40963 // 8192 + 16) & ~7 = 24, so some run whole beside the sliced
-    ones, in whatever order they ask."""
-    nm, count = 48, 5 * ITEMS + 3
-    print(f"case slices spent threads={threads} pair={pair}", flush=True)
+@pytest.mark.parametrize("count,spread", [(5 * ITEMS + 3, 0.0), (8 * ITEMS, 0.0), (8 * ITEMS + 1, 0.0),
+                                          (100 * ITEMS, 0.0), (100 * ITEMS, 1.0)])
+def test_more_slices_wanted_than_there_are(pm, oracle_mod, count, spread, threads, pair):
+    """Every particle in the cell just below a tile corner feeds eight tiles.
+    5 * 8192 + 3 of them want 8 * 6 = 48 slices of 8192 particles, and the
+    table's first half has (2 * 40963 // 8192 + 16) & ~7 = 24: some tiles run
+    whole beside the sliced ones, in whatever order they ask.  From 8 * 8192 + 1
+    on they take slices of the second half."""
+    nm = 48
+    print(f"case slices spent count={count} spread={spread} threads={threads} pair={pair}", flush=True)
     rng = np.random.default_rng(7)
-    pos = rng.uniform(15.0, 16.0, (count, 3))
+    pos = rng.uniform(15.0 - spread, 16.0 + spread, (count, 3))
     mass = rng.uniform(0.5, 1.5, count).astype(np.float32).astype(np.float64)
     plan = pm.Plan(nm, float(nm), keep_density=True)
     plan.set_tuning(deposit_threads=threads, deposit_pair=pair, deposit_split=False)
