@@ -361,7 +361,7 @@ struct MeshOps {
   void (*x_inv_mul)(dim3, dim3, hipStream_t, float2*, float2*, float2*, const float2*, int3);
   // ensembles: every stage for all boxes of this mesh side in one launch
   // (box b of the BoxArgs table on blockIdx.z); grids are per box, z = boxes
-  void (*deposit_box[2])(dim3, dim3, hipStream_t, const BoxArgs*, TileMap);
+  void (*deposit_box[2])(dim3, dim3, hipStream_t, const BoxArgs*, TileMap, unsigned lead);
   void (*x_fwd_box)(dim3, dim3, hipStream_t, const BoxArgs*, const float2*);
   void (*y_fwd_box)(dim3, dim3, hipStream_t, const BoxArgs*, const float2*);
   void (*z_green_box)(dim3, dim3, hipStream_t, const BoxArgs*, const float2*);
@@ -506,11 +506,11 @@ MeshOps make_ops() {
   o.x_inv_mul = [](dim3 g, dim3 b, hipStream_t s, float2* A, float2* P, float2* B, const float2* tw, int3 codes) {
     hipLaunchKernelGGL((k_fft_x_inv<N, R, true>), g, b, 0, s, A, P, B, nullptr, tw, 0, 1.0f, codes);
   };
-  o.deposit_box[0] = [](dim3 g, dim3 b, hipStream_t s, const BoxArgs* bx, TileMap tm) {
-    hipLaunchKernelGGL((k_deposit_box<TD, 256>), g, b, 0, s, bx, tm);
+  o.deposit_box[0] = [](dim3 g, dim3 b, hipStream_t s, const BoxArgs* bx, TileMap tm, unsigned lead) {
+    hipLaunchKernelGGL((k_deposit_box<TD, 256>), g, b, 0, s, bx, tm, lead);
   };
-  o.deposit_box[1] = [](dim3 g, dim3 b, hipStream_t s, const BoxArgs* bx, TileMap tm) {
-    hipLaunchKernelGGL((k_deposit_box<TD, 512>), g, b, 0, s, bx, tm);
+  o.deposit_box[1] = [](dim3 g, dim3 b, hipStream_t s, const BoxArgs* bx, TileMap tm, unsigned lead) {
+    hipLaunchKernelGGL((k_deposit_box<TD, 512>), g, b, 0, s, bx, tm, lead);
   };
   if constexpr (N > kPlaneMax) {
     o.x_fwd_box = [](dim3 g, dim3 b, hipStream_t s, const BoxArgs* bx, const float2* tw) {
@@ -2494,6 +2494,7 @@ int upload_box_tables(gng_pm_batch* b, const std::vector<BoxGroup>& gs, const in
       a.ranges = p->d_tile_ranges;
       a.p0 = offsets[i];
       a.n = offsets[i + 1] - offsets[i];
+      if (p->tune.deposit_split) a.split = slices_for(p, a.n, false);
       h.push_back(a);
     }
   if ((long long)h.size() > b->box_cap) {
@@ -2533,8 +2534,12 @@ void launch_box_group(gng_pm_batch* b, const BoxGroup& gr, const BoxArgs* bx, lo
                        dim3(256), 0, s, bx, src, m);
   const unsigned ntiles = (unsigned)p0->tm.nt * p0->tm.nt * p0->tm.nt;
   hipLaunchKernelGGL(k_tile_ranges_box, dim3((ntiles + 255) / 256, 1, nbx), dim3(256), 0, s, bx, p0->tm);
-  o.deposit_box[p0->tune.deposit_wide](dim3(xcd_grid(ntiles), 1, nbx), dim3(p0->tune.deposit_wide ? 512 : 256), s, bx,
-                                       p0->tm);
+  // the most slice workgroups a box of the group has
+  unsigned lead = 0;
+  for (int i : gr.boxes)
+    if (b->plans[i]->tune.deposit_split) lead = 2u * deposit_slots(maxn, slice_items(maxn));
+  o.deposit_box[p0->tune.deposit_wide](dim3(lead + xcd_grid(ntiles), 1, nbx), dim3(p0->tune.deposit_wide ? 512 : 256), s,
+                                       bx, p0->tm, lead);
   if (o.plane_fwd) {
     o.plane_fwd_box(nbx, s, bx, p0->d_tw);
     o.z_small_box(nbx, s, bx, p0->d_tw);

@@ -200,6 +200,15 @@ struct GreenParams {
   const float* deconv;  // 1/sinc^4(pi n / N) per axis index, or null
 };
 
+// The slices of heavy deposit tiles (deposit.hpp).
+struct DepositSplit {
+  unsigned* extra;   // slice workgroup e -> rank | slice << 20, or kNoSlice
+  unsigned slots;    // slice workgroups launched, both halves of the deposit's table (0: no splitting)
+  unsigned items;    // particles per slice
+  unsigned long long* scratch;   // slots / 2 x T^3 partial tiles, zero between solves
+  unsigned* done;                // slots / 2 finished-slice counters, zero between solves
+};
+
 // One box of an ensemble: the `_box` form of each stage kernel takes a device
 // array of these and works on box blockIdx.z, so one launch runs a stage for
 // every box of one mesh side.  Meshes, sort buffers and scalars are the box's
@@ -218,6 +227,7 @@ struct BoxArgs {
   unsigned* bucket;
   unsigned* rank;
   unsigned* ranges;
+  DepositSplit split;
   long long n;
   long long p0;
 };

@@ -85,3 +85,40 @@ def test_moments_of_heavy_tiles(pm, nm, count):
     for _ in range(2):
         got = plan.cell_moments().reshape(-1, 5)
         assert np.abs(got - ref).max() <= count * 2.0 ** -38
+
+
+def test_boxes_of_an_ensemble(pm, oracle_mod):
+    """Clumped boxes beside plain, small and empty ones of the same side in one
+    launch per stage: the forces of one pipeline per box bit for bit, replayed,
+    and the oracle's."""
+    print("case slices of boxes", flush=True)
+    rng = np.random.default_rng(3)
+    boxes, parts = [], []
+    for nm, count, centre in ((32, 30001, 8.0), (32, 0, 8.0), (32, 700, 8.0), (32, 90000, 15.5), (48, 40000, 24.0)):
+        pos = (centre + rng.normal(0.0, 0.4, (count, 3))) % nm
+        pos[count // 2:] = rng.uniform(0.0, nm, (count - count // 2, 3))
+        pos = pos.astype(np.float32)
+        pos[pos >= nm] = 0.0
+        boxes.append({"grid_size": nm, "box_size": float(nm)})
+        parts.append(pos)
+    off = np.concatenate([[0], np.cumsum([len(p) for p in parts])])
+    pos = np.concatenate(parts)
+    mass = rng.uniform(0.5, 1.5, len(pos)).astype(np.float32)
+    d = [pm.DeviceArray.from_host(np.ascontiguousarray(a)) for a in (pos[:, 0], pos[:, 1], pos[:, 2], mass)]
+    out = [pm.DeviceArray((len(pos),), np.float32) for _ in range(3)]
+    batch = pm.Batch(boxes)
+    got = []
+    for tables in (True, True, False, True):
+        batch.set_box_tables(tables)
+        for _ in range(2):
+            batch.solve_device(*(a.ptr for a in d), off, 1.0, *(o.ptr for o in out))
+            pm.device_synchronize()
+            got.append(np.stack([o.numpy() for o in out], axis=1))
+    for g in got[1:]:
+        assert np.array_equal(g, got[0])
+    for b, bx in enumerate(boxes):
+        if off[b + 1] > off[b]:
+            sel = slice(off[b], off[b + 1])
+            ref = oracle_mod.pm_accelerations(pos[sel].astype(np.float64), mass[sel].astype(np.float64), bx["box_size"],
+                                              bx["grid_size"], 1.0)
+            assert np.sqrt(((got[0][sel] - ref) ** 2).sum() / (ref ** 2).sum()) < 1e-5
