@@ -119,6 +119,19 @@ constexpr long long kChunkFwdMiB = 256, kChunkInvMiB = 64;
 // 32768 before: 338, 343 and 673 us.
 unsigned slice_items(long long n) { return (unsigned)std::min<long long>(std::max<long long>(n / 1024, 8192), 32768); }
 
+// Where particles spread evenly give a tile more than that, slices are longer:
+// twice the even load, so that only clumps are split, or 1.5 / 256 of all loads,
+// which keeps the chip busy where there are fewer tiles than CUs.  Splitting
+// evenly loaded tiles costs their flush, 4096 atomics a slice at 20 G/s, for
+// nothing: deposit of 4.2e6 particles on 128^3 79 us so, 272 in slices of 8192
+// (116 in the version with 32768); 1.8e6 on 96^3, 216 tiles, 47, 161 (82);
+// 8.4e6 on 64^3, 64 tiles, 348, 555 (621).  From 65536 on splitting pays again:
+// 33.6e6 on 128^3 990 us, 1313 unsplit.
+unsigned dense_items(int T, int nt, long long n) {
+  const double edge = 1.0 + 1.0 / T, all = (double)n * edge * edge * edge;  // particles read by all tiles
+  return (unsigned)std::min({2.0 * all / ((double)nt * nt * nt), 1.5 * all / 256.0, 65536.0});
+}
+
 Tuning default_tuning(int nm) {
   Tuning t;
   t.z_persistent = nm == 512;
@@ -903,7 +916,7 @@ void run_sort(gng_pm_plan* p, const PartIn& in, long long n, unsigned* perm, boo
 DepositSplit slices_for(const gng_pm_plan* p, long long n, bool moments) {
   DepositSplit sp{};
   if (p->split_slots > 0) {
-    sp.items = slice_items(n) * (moments ? 4u : 1u);
+    sp.items = std::max(slice_items(n), dense_items(p->tm.T, p->tm.nt, n)) * (moments ? 4u : 1u);
     sp.slots = deposit_slots(n, sp.items) * (moments ? 1u : 2u);
     sp.extra = p->d_extra;
     sp.scratch = p->d_split_scratch;
@@ -2537,7 +2550,7 @@ void launch_box_group(gng_pm_batch* b, const BoxGroup& gr, const BoxArgs* bx, lo
   // the most slice workgroups a box of the group has
   unsigned lead = 0;
   for (int i : gr.boxes)
-    if (b->plans[i]->tune.deposit_split) lead = 2u * deposit_slots(maxn, slice_items(maxn));
+    if (b->plans[i]->tune.deposit_split) lead = std::max(lead, slices_for(b->plans[i], maxn, false).slots);
   o.deposit_box[p0->tune.deposit_wide](dim3(lead + xcd_grid(ntiles), 1, nbx), dim3(p0->tune.deposit_wide ? 512 : 256), s,
                                        bx, p0->tm, lead);
   if (o.plane_fwd) {

@@ -64,6 +64,26 @@ def test_more_slices_wanted_than_there_are(pm, oracle_mod, count, spread, thread
     assert np.abs(d0 - ref).max() <= 2.0 ** -24 * ref.max() * 1.01
 
 
+@pytest.mark.parametrize("nm,count", [(32, 1500000), (96, 1900000), (64, 1400001)])
+def test_dense_sets(pm, oracle_mod, nm, count):
+    """So many particles that an evenly loaded tile holds more than 8192 and the
+    slices get longer with the load (only the clump's tile is split at 96^3)."""
+    print(f"case dense nm={nm} count={count}", flush=True)
+    rng = np.random.default_rng(nm)
+    pos = rng.uniform(0.0, nm, (count, 3))
+    pos[: count // 10] = (8.0 + rng.normal(0.0, 0.7, (count // 10, 3))) % nm
+    mass = rng.uniform(0.5, 1.5, count).astype(np.float32).astype(np.float64)
+    plan = pm.Plan(nm, float(nm), keep_density=True)
+    got = []
+    for split in (False, True, True):
+        plan.set_tuning(deposit_split=split)
+        got.append((plan.accelerations_f64(pos, mass, 1.0), plan.density(), plan.cell_moments()))
+    for g in got[1:]:
+        assert all(np.array_equal(x, y) for x, y in zip(g, got[0]))
+    ref = oracle_mod.cic_assign(pos, mass, float(nm), nm).reshape(nm, nm, nm)
+    assert np.abs(got[0][1] - ref).max() <= 2.0 ** -24 * ref.max() * 1.01
+
+
 @pytest.mark.parametrize("nm,count", [(16, 32768), (16, 32769), (48, 3 * 32768 + 5)])
 def test_moments_of_heavy_tiles(pm, nm, count):
     """Cell moments at and past the slice length, twice (the cleared words and
