@@ -120,16 +120,18 @@ constexpr long long kChunkFwdMiB = 256, kChunkInvMiB = 64;
 unsigned slice_items(long long n) { return (unsigned)std::min<long long>(std::max<long long>(n / 1024, 8192), 32768); }
 
 // Where particles spread evenly give a tile more than that, slices are longer:
-// twice the even load, so that only clumps are split, or 1.5 / 256 of all loads,
-// which keeps the chip busy where there are fewer tiles than CUs.  Splitting
-// evenly loaded tiles costs their flush, 4096 atomics a slice at 20 G/s, for
-// nothing: deposit of 4.2e6 particles on 128^3 79 us so, 272 in slices of 8192
-// (116 in the version with 32768); 1.8e6 on 96^3, 216 tiles, 47, 161 (82);
-// 8.4e6 on 64^3, 64 tiles, 348, 555 (621).  From 65536 on splitting pays again:
-// 33.6e6 on 128^3 990 us, 1313 unsplit.
+// twice the even load, so that only clumps are split, or a length that pays for
+// its flush.  That is 4096 atomics a slice at 20 G/s, 0.2 us, times the tiles,
+// against 3 ns a particle for the longest workgroup: from 256 particles a tile
+// on (16384 from 64 tiles on), and 1.5 / 256 of all loads, a slice or two a CU.
+// Deposit of 4.2e6 particles on 128^3 78 us so, 261 in slices of 8192 (116 in the
+// version with 32768); 1.8e6 on 96^3, 216 tiles, 30, 159 (82); 0.5e6 on 64^3, 64
+// tiles, 27, 63 (75), and 8.4e6 348, 560 (621).  From 65536 on splitting pays
+// again: 33.6e6 on 128^3 995 us, 1313 unsplit.
 unsigned dense_items(int T, int nt, long long n) {
   const double edge = 1.0 + 1.0 / T, all = (double)n * edge * edge * edge;  // particles read by all tiles
-  return (unsigned)std::min({2.0 * all / ((double)nt * nt * nt), 1.5 * all / 256.0, 65536.0});
+  const double tiles = (double)nt * nt * nt, flush = std::min(256.0 * tiles, 16384.0);
+  return (unsigned)std::min(2.0 * all / tiles, std::clamp(1.5 * all / 256.0, flush, 65536.0));
 }
 
 Tuning default_tuning(int nm) {
