@@ -817,9 +817,16 @@ __global__ __launch_bounds__(256) void k_loss(const float4* __restrict__ pos, co
   // neighbouring lanes add neighbouring components and nodes, so a wavefront's
   // adds fall into few cache lines
   const float* flat = reinterpret_cast<const float*>(sum);
-  for (int i = threadIdx.x; i < 4 * kLossSlots; i += 256) {
-    const unsigned node = key[i >> 2];
-    if (node != kEmpty && (i & 3) != 3) atomicAdd(gy + (size_t)node * 4 + (i & 3), flat[i]);
+  for (int i0 = threadIdx.x; i0 < 4 * kLossSlots; i0 += 8 * 256) {
+    // eight keys in flight: most slots of few records are empty
+    unsigned node[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) node[k] = key[(i0 + 256 * k) >> 2];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int i = i0 + 256 * k;
+      if (node[k] != kEmpty && (i & 3) != 3) atomicAdd(gy + (size_t)node[k] * 4 + (i & 3), flat[i]);
+    }
   }
   if (threadIdx.x == 0) atomicAdd(loss, red[0] + red[1] + red[2] + red[3]);
 }
