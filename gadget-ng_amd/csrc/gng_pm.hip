@@ -140,11 +140,11 @@ Tuning default_tuning(int nm) {
   // 512 threads per deposit tile only where there are fewer tiles than CUs
   // (64^3: 12 against 13 us); elsewhere four 256-thread workgroups share a
   // CU's LDS and overlap each other's latencies (512^3, 256^3 particles: 253
-  // against 288 us).  Two tiles per workgroup pay on the largest mesh only
-  // (1024^3: 2.78 against 2.88 ms; 512^3: 260 against 253 us).
+  // against 288 us).  Two tiles per workgroup are left to the tuner: on 1024^3
+  // 2.74 against 2.78 ms for 512^3 clustered particles, but 2.13 against 1.89
+  // for a displaced lattice (512^3: 260 against 253 us).
   const int nt = nm / deposit_tile(nm);
   t.deposit_wide = nt * nt * nt < 256;
-  t.deposit_pair = nm >= 1024;
   t.chunk_fwd = chunk_rule(nm, kChunkFwdMiB);
   // at nm >= 1024 the inverse y pass runs as two launches on full lines, and
   // whole-mesh passes measured faster (10.5 against 11.0 ms at 1024^3)

@@ -213,15 +213,14 @@ int gng_pm_force_meshes(gng_pm_plan *p, float *out);
  * a time from the defaults and keeps each flip that is faster.  The result
  * applies to this plan and to plans created later in the process with the
  * same device architecture and mesh side; with GNG_PM_TUNE_FILE set it is also
- * read from and written to that file.  (A file written by a library whose choices
- * select other kernels is not read.)  Untuned plans use the persistent z pass
- * at nm = 512 only, the 512-thread deposit only below 256 tiles, and two
- * tiles per deposit workgroup from nm = 1024 on.  Up to nm = 128 the force
- * solve transforms whole z planes in one kernel each way; the choices of its x,
- * y and z passes are kept but have no effect there.  Solves of at most 16384
- * particles on at most 512 deposit tiles do not sort, and the deposit's choices
- * have no effect on them (interp_sorted, which needs the sort, turns it back
- * on).  No reference counterpart.
+ * read from and written to that file.  (A file written by a library whose
+ * choices select other kernels is not read.)  Untuned plans use the persistent
+ * z pass at nm = 512 only and the 512-thread deposit only below 256 tiles.  Up
+ * to nm = 128 the force solve transforms whole z planes in one kernel each way;
+ * the choices of its x, y and z passes are kept but have no effect there.
+ * Solves of at most 16384 particles on at most 512 deposit tiles do not sort,
+ * and the deposit's choices have no effect on them (interp_sorted, which needs
+ * the sort, turns it back on).  No reference counterpart.
  * Synchronous; the density and potential of earlier solves are invalidated. */
 typedef struct gng_pm_tuning_t {
   int32_t z_persistent;      /* z + Green pass: persistent workgroups          */
@@ -259,9 +258,9 @@ typedef struct gng_pm_tuning_t {
                                 the three live fields leave a 1024-thread
                                 workgroup alone on its CU.  Same values either
                                 way */
-  int32_t deposit_pair;      /* deposit: two tiles per workgroup (1, default from
-                                nm = 1024), whose records load while the other
-                                tile is written, or one (0).
+  int32_t deposit_pair;      /* deposit: two tiles per workgroup (1), whose
+                                records load while the other tile is written,
+                                or one (0, default).
                                 Same density bit for bit either way */
 } gng_pm_tuning_t;
 

@@ -24,6 +24,16 @@ def test_deposit_choices_of_small_meshes_stay(pm, nm):
         assert got["tuned"] and {k: got[k] for k in DEPOSIT} == default
 
 
+@pytest.mark.parametrize("nm,threads", [(64, 512), (128, 256), (512, 256), (1024, 256)])
+def test_default_deposit(pm, nm, threads):
+    """One tile a workgroup on every mesh: two are slower for even sets, also at
+    1024^3."""
+    print(f"case default deposit nm={nm}", flush=True)
+    got = pm.Plan(nm, 1.0, r_split=0.1).tuning()
+    if not got["tuned"]:  # (an earlier autotune of this process holds otherwise)
+        assert {k: got[k] for k in DEPOSIT} == {"deposit_threads": threads, "deposit_split": True, "deposit_pair": False}
+
+
 SCRIPT = """
 import sys
 sys.path.insert(0, {pkg!r})
