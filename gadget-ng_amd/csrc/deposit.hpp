@@ -350,8 +350,9 @@ constexpr unsigned kNoSlice = 0xffffffffu;
 // out: when most particles sit at tile edges.  A tile that finds it so counts a
 // particle that m tiles read as 1 / m, which adds up to n over the tiles, and
 // takes ceil(that / items) slices of the second half, which cannot run out; its
-// slices are up to eight times as long.  A solve of 10^6 particles about a tile
-// corner (sigma 0.7 cells) on 48^3: 389 us, 2256 where such tiles ran unsplit.
+// slices are up to eight times as long.  Workgroup e of the table runs entry e
+// of both halves, so the second costs no empty workgroups.  A solve of 10^6 particles about a tile
+// corner (sigma 0.7 cells) on 48^3: 414 us, 2256 where such tiles ran unsplit.
 inline unsigned deposit_slots(long long n, unsigned items) { return (unsigned)((2 * n / items + 16) & ~7LL); }
 
 // The flattened range layout of every tile rank r, written after the scatter
@@ -522,21 +523,16 @@ __device__ __forceinline__ unsigned xcd_item(unsigned b, unsigned n) {
 }
 constexpr unsigned xcd_grid(unsigned n) { return (n + 7u) / 8u * 8u; }
 
-// One slice of a heavy tile (sp): its share of the flattened ranges into the
+// Table entry v, one slice of a heavy tile (sp): its share of the flattened ranges into the
 // LDS tile, the LDS tile into the scratch tile, and the last slice of the
 // tile converts.
 template <int T, int NT>
 __device__ __forceinline__ void deposit_slice(unsigned long long* acc, const PartRec* __restrict__ sorted,
                                               const CellMap& cm, const TileMap& tm, const SolveScalars* sc,
                                               float* __restrict__ rho, long long rho_plane, float* __restrict__ keep,
-                                              const DepositSplit& sp) {
+                                              const DepositSplit& sp, unsigned v) {
   constexpr int T3 = T * T * T;
   const int tid = threadIdx.x, nt = tm.nt;
-  const unsigned e = blockIdx.x, half = sp.slots / 2u;
-  // uniform: no slice for this workgroup
-  if (e < half ? e >= sc->split_budget : e - half >= sc->split_rest) return;
-  const unsigned v = sp.extra[e];
-  if (v == kNoSlice) return;
   const unsigned rank = v & 0xfffffu;
   const unsigned* __restrict__ w = tm.ranges + (size_t)rank * kRangeWords;
   const unsigned all = w[13], S = w[28], slot = w[29];
@@ -601,8 +597,8 @@ __device__ __forceinline__ void deposit_slice(unsigned long long* acc, const Par
 // Hilbert curve); T is the tile side (T^3 int64 accumulators in LDS).  Cell
 // (x, y, z) of the shifted mass mesh is rho[z*rho_plane + y*nm + x]; keep
 // (when not null) receives the unshifted mass per cell, unpadded.  The first
-// `lead` workgroups of the grid (at least sp.slots) are the slices of the heavy
-// tiles, which the others skip.
+// `lead` workgroups of the grid (at least sp.slots / 2) are the slices of the
+// heavy tiles, which the others skip.
 // With two tiles, their rounds of records form one sequence, so the prefetch
 // ring runs across the tile boundary: the second tile's records load while
 // the first tile is converted and written.
@@ -615,7 +611,16 @@ __device__ __forceinline__ void deposit_body(const PartRec* __restrict__ sorted,
   const int tid = threadIdx.x;
   const int nt = tm.nt;
   if (blockIdx.x < lead) {
-    deposit_slice<T, NT>(acc, sorted, cm, tm, sc, rho, rho_plane, keep, sp);
+    // (uniform) the entries of this workgroup in either half of the table
+    const unsigned e = blockIdx.x, half = sp.slots / 2u;
+    if (e < min(sc->split_budget, half)) {
+      const unsigned v = sp.extra[e];
+      if (v != kNoSlice) deposit_slice<T, NT>(acc, sorted, cm, tm, sc, rho, rho_plane, keep, sp, v);
+    }
+    if (e < sc->split_rest) {
+      __syncthreads();
+      deposit_slice<T, NT>(acc, sorted, cm, tm, sc, rho, rho_plane, keep, sp, sp.extra[half + e]);
+    }
     return;
   }
   const unsigned ntiles = (unsigned)(nt * nt * nt), groups = (ntiles + TILES - 1u) / TILES;
@@ -705,7 +710,7 @@ template <int T, int NT, int TILES>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void k_deposit(
     const PartRec* __restrict__ sorted, const CellMap cm, const TileMap tm, const SolveScalars* sc,
     float* __restrict__ rho, long long rho_plane, float* __restrict__ keep, const DepositSplit sp) {
-  deposit_body<T, NT, TILES>(sorted, cm, tm, sc, rho, rho_plane, keep, sp, sp.slots);
+  deposit_body<T, NT, TILES>(sorted, cm, tm, sc, rho, rho_plane, keep, sp, sp.slots / 2u);
 }
 
 // Every box has its own slices; `lead` is the most of the group.  Four boxes of

@@ -982,7 +982,7 @@ int run_front(gng_pm_plan* p, const PartIn& in, long long n, hipStream_t s) {
     const DepositSplit sp = p->tune.deposit_split ? slices_for(p, n, false) : DepositSplit{};
     hipLaunchKernelGGL(k_tile_ranges, dim3((ntiles + 255) / 256), dim3(256), 0, s, p->d_offset, p->tm, p->d_sc, n, sp);
     const int pair = p->tune.deposit_pair != 0;
-    o.deposit[p->tune.deposit_wide][pair](dim3(sp.slots + xcd_grid(pair ? (ntiles + 1u) / 2u : ntiles)),
+    o.deposit[p->tune.deposit_wide][pair](dim3(sp.slots / 2u + xcd_grid(pair ? (ntiles + 1u) / 2u : ntiles)),
                                           dim3(p->tune.deposit_wide ? 512 : 256), s, p->d_sorted, cm, p->tm, p->d_sc,
                                           rho, rho_plane, p->keep_density ? p->d_rho : nullptr, sp);
   }
@@ -2552,7 +2552,7 @@ void launch_box_group(gng_pm_batch* b, const BoxGroup& gr, const BoxArgs* bx, lo
   // the most slice workgroups a box of the group has
   unsigned lead = 0;
   for (int i : gr.boxes)
-    if (b->plans[i]->tune.deposit_split) lead = std::max(lead, slices_for(b->plans[i], maxn, false).slots);
+    if (b->plans[i]->tune.deposit_split) lead = std::max(lead, slices_for(b->plans[i], maxn, false).slots / 2u);
   o.deposit_box[p0->tune.deposit_wide](dim3(lead + xcd_grid(ntiles), 1, nbx), dim3(p0->tune.deposit_wide ? 512 : 256), s,
                                        bx, p0->tm, lead);
   if (o.plane_fwd) {

@@ -202,8 +202,8 @@ struct GreenParams {
 
 // The slices of heavy deposit tiles (deposit.hpp).
 struct DepositSplit {
-  unsigned* extra;   // slice workgroup e -> rank | slice << 20, or kNoSlice
-  unsigned slots;    // slice workgroups launched, both halves of the deposit's table (0: no splitting)
+  unsigned* extra;   // table entry -> rank | slice << 20, or kNoSlice
+  unsigned slots;    // entries of the table, for the deposit in two halves (0: no splitting)
   unsigned items;    // particles per slice
   unsigned long long* scratch;   // slots / 2 x T^3 partial tiles, zero between solves
   unsigned* done;                // slots / 2 finished-slice counters, zero between solves
