@@ -765,7 +765,9 @@ __device__ __forceinline__ void fft_y_inv_body(float2* __restrict__ A, float2* _
                                                  int3 codes) {
   // PART 1: only the two fields from A (A and P); PART 2: only B.  Two such
   // launches read each input once, like the combined kernel, with fewer
-  // live registers (for 16 values per thread at N = 1024).
+  // live registers (for 16 values per thread at N = 1024; PART 1 still spills
+  // 17 of them, 72 bytes a lane, because A stays live through its first
+  // transform).
   constexpr int H = N / 2, IS = C + 1;
   constexpr bool DO_A = PART != 2, DO_B = PART != 1;
   using F = RegFft<N, true, false, C, T, 1, IS, true, N>;
