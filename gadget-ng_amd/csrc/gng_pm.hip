@@ -1203,9 +1203,9 @@ struct Xfer {
 // the solve's own stream reads (or fills) over the bus.  Below about this size
 // the threads' start, their streams' events and a DMA per array cost more than
 // one thread's copies: 1024 particles on 32^3 took 157 us through them and take
-// 59 this way; 26000 with an index list on 64^3, just below it, take 136 us, and
-// 32768, just above, 193 through the threads.  The first call takes 0.2 ms, and 9
-// where it pins the threads' slots.
+// 58 to 69 this way (from run to run); 26000 with an index list on 64^3, just
+// below it, take 136 us, and 32768, just above, 193 through the threads.  The
+// first call takes 0.2 ms, and 9 where it pins the threads' slots.
 constexpr size_t kSmallStage = 1u << 20;
 constexpr int kSmallSegs = 5;
 struct StageSegs {
