@@ -2,6 +2,7 @@
 large meshes' workspace once the call has returned, nothing at all when the
 workspace does not fit, and then the plan still works."""
 import ctypes
+import time
 
 import numpy as np
 import pytest
@@ -23,6 +24,16 @@ def free_bytes(pm):
     return get
 
 
+def given_back(free_bytes, before, most):
+    """Whether no more than `most` bytes are gone, once the driver has done its
+    bookkeeping (freed pages have been seen to come back late)."""
+    for _ in range(50):
+        if before - free_bytes() < most:
+            return True
+        time.sleep(0.2)
+    return False
+
+
 def spectrum(n):
     return lambda k: 0.05 * n ** 3 / max(k, 1.0)
 
@@ -36,7 +47,7 @@ def test_large_meshes_are_given_back(pm, free_bytes):
     before = free_bytes()
     pos = ic.zeldovich_2lpt_ics(plan, 3, spectrum(n), lo=0, hi=1000)[0]
     assert np.isfinite(pos).all()
-    assert before - free_bytes() < 256 << 20  # (a mesh is 4.3 GB)
+    assert given_back(free_bytes, before, 256 << 20)  # (a mesh is 4.3 GB)
 
 
 def test_a_workspace_that_does_not_fit_leaves_nothing_behind(pm, free_bytes):
@@ -58,7 +69,7 @@ def test_a_workspace_that_does_not_fit_leaves_nothing_behind(pm, free_bytes):
     before = free_bytes()
     with pytest.raises(Exception):
         ic.zeldovich_2lpt_ics(plan, 3, spectrum(n), lo=0, hi=1000)
-    assert before - free_bytes() < 64 << 20
+    assert given_back(free_bytes, before, 64 << 20)
     for h in hogs:
         h.free()
     got = ic.zeldovich_2lpt_ics(plan, 3, spectrum(n), lo=0, hi=1000)
