@@ -611,15 +611,17 @@ __device__ __forceinline__ void deposit_body(const PartRec* __restrict__ sorted,
   const int tid = threadIdx.x;
   const int nt = tm.nt;
   if (blockIdx.x < lead) {
-    // (uniform) the entries of this workgroup in either half of the table
+    // (uniform) the entries of this workgroup in either half of the table, through
+    // one copy of the slice code (24307 particles on 64^3: 85.9 us, 86.4 with two)
     const unsigned e = blockIdx.x, half = sp.slots / 2u;
-    if (e < min(sc->split_budget, half)) {
-      const unsigned v = sp.extra[e];
-      if (v != kNoSlice) deposit_slice<T, NT>(acc, sorted, cm, tm, sc, rho, rho_plane, keep, sp, v);
-    }
-    if (e < sc->split_rest) {
-      __syncthreads();
-      deposit_slice<T, NT>(acc, sorted, cm, tm, sc, rho, rho_plane, keep, sp, sp.extra[half + e]);
+    const unsigned first = min(sc->split_budget, half), rest = sc->split_rest;
+#pragma unroll 1
+    for (unsigned h = 0; h < 2u; ++h) {
+      if (e >= (h ? rest : first)) continue;
+      const unsigned v = sp.extra[h ? half + e : e];
+      if (v == kNoSlice) continue;
+      __syncthreads();  // the first entry's tile is read
+      deposit_slice<T, NT>(acc, sorted, cm, tm, sc, rho, rho_plane, keep, sp, v);
     }
     return;
   }
